@@ -19,7 +19,9 @@ modularity   The modularity of a given partition of a graph that is on the
 
 Graphs are R-MAT (0.57, 0.19, 0.19, 0.05), Chung-Lu with Pareto(2.1) degrees,
 or planted partitions in blocks of 64, symmetric, without self arcs or
-duplicates, with unit or U(0, 1] weights.
+duplicates, with unit or U(0, 1] weights.  "stream": the program keeps a
+stream of its own and gives it to its handles, as one that makes large
+handles one after another does; otherwise a handle makes its own.
 """
 import numpy as np
 import torch
@@ -38,20 +40,22 @@ def listed():
         dict(name="run-rmat-s14", kind="run", graph="rmat", n=1 << 14, ef=16, weighted=False, nb=2),
         # an odd size, weighted: a mid-size graph of an analysis job
         dict(name="run-chunglu-300k", kind="run", graph="chunglu", n=300007, mean=32.0, dmax=5000.0, weighted=True, nb=8),
-        # the largest graph of the request stream
-        dict(name="run-rmat-s20", kind="run", graph="rmat", n=1 << 20, ef=32, weighted=False, nb=32),
+        # the largest graph of the benchmark's request stream
+        dict(name="run-rmat-s20", kind="run", graph="rmat", n=1 << 20, ef=32, weighted=False, nb=32, stream=True),
         # the benchmark's graph: iterations of its first phase
-        dict(name="phase-rmat-s22", kind="phase", graph="rmat", n=1 << 22, ef=16, weighted=True, nb=32),
+        dict(name="phase-rmat-s22", kind="phase", graph="rmat", n=1 << 22, ef=16, weighted=True, nb=32, stream=True),
         # a flatter degree distribution, ragged size, unit weights
-        dict(name="phase-chunglu-2m", kind="phase", graph="chunglu", n=2100001, mean=32.0, dmax=50000.0, weighted=False, nb=32),
+        dict(name="phase-chunglu-2m", kind="phase", graph="chunglu", n=2100001, mean=32.0, dmax=50000.0, weighted=False, nb=32,
+             stream=True),
         # a driver that makes the single calls itself
         dict(name="steps-rmat-s17", kind="steps", graph="rmat", n=1 << 17, ef=16, weighted=True, nb=8),
         # many graphs at once, an eighth of the benchmark's 4,096
-        dict(name="batch-512-sbm", kind="batch", graphs=512, nmin=256, nmax=65536, inner=12.0, outer=2.0, weighted=True, nb=32),
+        dict(name="batch-512-sbm", kind="batch", graphs=512, nmin=256, nmax=65536, inner=12.0, outer=2.0, weighted=True, nb=32,
+             stream=True),
         # a handful of small graphs at once
         dict(name="batch-40-small", kind="batch", graphs=40, nmin=200, nmax=5000, inner=12.0, outer=2.0, weighted=False, nb=2),
         # a burst of requests
-        dict(name="serve-30-mixed", kind="serve", requests=30, smin=10, smax=19, weighted=False, nb=32),
+        dict(name="serve-24-mixed", kind="serve", requests=24, smin=10, smax=17, weighted=False, nb=32),
         # a graph of five windows
         dict(name="window-rmat-s19", kind="window", graph="rmat", n=1 << 19, ef=16, weighted=True, nb=32, parts=5),
         # a given partition scored on the device
@@ -69,17 +73,18 @@ def draw(rng):
     nb = rng.choice([2, 8, 32])
     if kind == "batch":
         graphs = _log(rng, 8, 512)
-        return dict(kind=kind, graphs=graphs, nmin=256, nmax=_log(rng, 1024, 65536), inner=12.0, outer=2.0, weighted=weighted, nb=nb)
+        return dict(kind=kind, graphs=graphs, nmin=256, nmax=_log(rng, 1024, 65536), inner=12.0, outer=2.0, weighted=weighted,
+                    nb=nb, stream=graphs > 64 or rng.random() < 0.5)
     if kind == "serve":
         smin = rng.randint(10, 13)
-        return dict(kind=kind, requests=rng.randint(4, 30), smin=smin, smax=rng.randint(smin, 18), weighted=weighted, nb=nb)
+        return dict(kind=kind, requests=rng.randint(4, 24), smin=smin, smax=rng.randint(smin, 16), weighted=weighted, nb=nb)
     hi = {"run": 1 << 20, "phase": 1 << 21, "steps": 1 << 19, "window": 1 << 19, "modularity": 1 << 21}[kind]
     lo = {"run": 1 << 10, "phase": 1 << 16, "steps": 1 << 12, "window": 1 << 15, "modularity": 1 << 10}[kind]
     n = _log(rng, lo, hi)
     graph = rng.choice(["rmat", "chunglu", "sbm"]) if kind != "modularity" else "sbm"
     c = dict(kind=kind, graph=graph, n=n, weighted=weighted)
     if kind != "modularity":
-        c["nb"] = nb
+        c |= dict(nb=nb, stream=n > 1 << 18 or rng.random() < 0.5)
     if graph == "rmat":
         c["ef"] = rng.choice([8, 16])
     elif graph == "chunglu":
@@ -193,19 +198,28 @@ def prepare(case, seed):
         sizes = _sizes(case)
         u, v = _sbm(sizes, case["inner"], case["outer"], gen)
         csr = _host(_csr(sum(sizes), u, v, case["weighted"], gen))
-        return dict(case=case, csr=(np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64),) + csr)
+        return dict(case=case, csr=(np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64),) + csr, stream=_stream(case))
     if kind == "serve":
         graphs = [_host(_csr(1 << s, *_rmat(1 << s, ef, gen), case["weighted"], gen)) for s, ef in _requests(case)]
         return dict(case=case, graphs=graphs, server=na.Server(slots=8, nbatches=case["nb"], tol=TOL, group=64))
     csr = _host(_graph(case, gen))
+    s = dict(case=case, csr=csr, stream=_stream(case))
     if kind in ("phase", "steps"):
-        return dict(case=case, handle=na.GraphGPU(csr, case["nb"]))
-    return dict(case=case, csr=csr)
+        s["handle"] = na.GraphGPU(csr, case["nb"], stream=_handle(s["stream"]))
+    return s
+
+
+def _stream(case):
+    return torch.cuda.Stream() if case.get("stream") else None
+
+
+def _handle(stream):
+    return stream.cuda_stream if stream else None
 
 
 # ---- one pass ----------------------------------------------------------------
-def _run_whole(csr, nb, window=0):
-    g = na.GraphGPU(csr, nb, window=window)
+def _run_whole(csr, nb, stream, window=0):
+    g = na.GraphGPU(csr, nb, stream=_handle(stream), window=window)
     st = na.LouvainGPU(tol=TOL, nbatches=nb).run(g)
     out = dict(clustering=g.clustering(), q=st.q, phases=st.phases, loops=st.total_loops)
     g.close()
@@ -241,8 +255,8 @@ def _run_steps(g, nb):
     return dict(q0=q0, q=q, loops=loops, communities=g.communities(), totals=g.community_weights())
 
 
-def _run_batch(csr, nb):
-    b = na.BatchGPU(csr=csr, nbatches=nb)
+def _run_batch(csr, nb, stream):
+    b = na.BatchGPU(csr=csr, nbatches=nb, stream=_handle(stream))
     b.run(tol=TOL)
     q = np.array([b.graph_stats(i).q for i in range(b.ngraphs)])
     out = dict(clustering=np.concatenate([b.clustering(i) for i in range(b.ngraphs)]), q=q)
@@ -265,15 +279,15 @@ def run(state):
     case = state["case"]
     kind = case["kind"]
     if kind == "run":
-        return _run_whole(state["csr"], case["nb"])
+        return _run_whole(state["csr"], case["nb"], state["stream"])
     if kind == "window":
-        return _run_whole(state["csr"], case["nb"], window=_window(state["csr"][0], case["parts"]))
+        return _run_whole(state["csr"], case["nb"], state["stream"], window=_window(state["csr"][0], case["parts"]))
     if kind == "phase":
         return _run_phase(state["handle"])
     if kind == "steps":
         return _run_steps(state["handle"], case["nb"])
     if kind == "batch":
-        return _run_batch(state["csr"], case["nb"])
+        return _run_batch(state["csr"], case["nb"], state["stream"])
     if kind == "serve":
         return _run_serve(state["server"], state["graphs"])
     s = state
