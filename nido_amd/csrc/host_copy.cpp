@@ -94,7 +94,11 @@ class Staging {
     }
     // The caller's stream has finished every copy out of or into the
     // buffers before the pair goes back (each copy ends with a stream
-    // synchronisation), so the events may be recorded again at once.
+    // synchronisation), so the events may be recorded again at once.  They
+    // are waited for only after this copy has recorded them: an event
+    // still refers to the stream it was recorded on last, which may have been
+    // destroyed since (waiting for one failed now and then with
+    // hipErrorCapturedEvent, read from whatever took the stream's place).
     char* buf(int i) const { return p_.buf[i]; }
     hipEvent_t done(int i) const { return p_.done[i]; }
 
@@ -226,7 +230,7 @@ hipError_t staged_h2d(void* dst, const void* src, size_t bytes, hipStream_t s)
     char* out = static_cast<char*>(dst);
     for (size_t at = 0, i = 0; e == hipSuccess && at < bytes; at += kChunk, i ^= 1) {
         const size_t n = std::min(kChunk, bytes - at);
-        e = hipEventSynchronize(done[i]);      // the buffer's previous copy has landed
+        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
         if (e != hipSuccess) break;
         constexpr size_t kPiece = size_t(1) << 20;
         const int64_t pieces = (int64_t)((n + kPiece - 1) / kPiece);
@@ -303,7 +307,7 @@ hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s
     const hipEvent_t done[2] = {st.done(0), st.done(1)};
     for (int64_t at = 0, i = 0; e == hipSuccess && at < n; at += kChunk, i ^= 1) {
         const int64_t m = std::min(kChunk, n - at);
-        e = hipEventSynchronize(done[i]);      // the buffer's previous copy has landed
+        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
         if (e != hipSuccess) break;
         int* b = buf[i];
         const int64_t* in = src + at;
@@ -330,7 +334,7 @@ hipError_t staged_h2d_local_ids(uint16_t* dst, const int64_t* src, int64_t n, hi
     const hipEvent_t done[2] = {st.done(0), st.done(1)};
     for (int64_t at = 0, i = 0; e == hipSuccess && at < n; at += kChunk, i ^= 1) {
         const int64_t m = std::min(kChunk, n - at);
-        e = hipEventSynchronize(done[i]);      // the buffer's previous copy has landed
+        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
         if (e != hipSuccess) break;
         narrow_local_checked(buf[i], src, at, m, chk);
         e = hipMemcpyAsync(dst + at, buf[i], sizeof(uint16_t) * (size_t)m, hipMemcpyHostToDevice, s);
@@ -351,7 +355,7 @@ hipError_t staged_h2d_weights(double* dst, const double* src, int64_t n, hipStre
     const hipEvent_t done[2] = {st.done(0), st.done(1)};
     for (int64_t at = 0, i = 0; e == hipSuccess && at < n; at += kChunk, i ^= 1) {
         const int64_t m = std::min(kChunk, n - at);
-        e = hipEventSynchronize(done[i]);      // the buffer's previous copy has landed
+        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
         if (e != hipSuccess) break;
         weights_checked(buf[i], src, at, m, chk);
         e = hipMemcpyAsync(dst + at, buf[i], sizeof(double) * (size_t)m, hipMemcpyHostToDevice, s);
