@@ -1321,22 +1321,21 @@ int do_iteration(nido_graph* g, double* q, double* dq, double* qt_out = nullptr)
 int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, const unsigned char* keep)
 {
     hipStream_t s = g->stream;
-    const int64_t nv = g->nv;
-    int64_t *arcs = nullptr, *toff = nullptr, *cnt = nullptr, *noff = nullptr, *ncol = nullptr;
-    int64_t *cpos = nullptr, *mstart = nullptr;
-    unsigned long long* mfill = nullptr;
-    int *members = nullptr, *ckey = nullptr, *hlist = nullptr;
+    const int64_t nv = g->nv, K1 = K + 1;
+    // sizes: seven arrays of K + 1 entries, the last entry of mfill the
+    // length of the mid list
+    int64_t *sizes = nullptr, *noff = nullptr, *ncol = nullptr, *hd = nullptr, *wpre = nullptr;
+    int *cid = nullptr, *members = nullptr, *ckey = nullptr, *mid = nullptr, *tkey = nullptr;
     double *nw = nullptr, *cw = nullptr;
-    int* tkey = nullptr;
     fx_t* tval = nullptr;
-    void* tmp = nullptr;
+    void *tmp = nullptr, *tmp2 = nullptr;
     auto cleanup = [&]() {
-        dev_free(arcs); dev_free(toff); dev_free(cnt); dev_free(noff);
-        dev_free(ncol); dev_free(nw); dev_free(tkey); dev_free(tval);
-        dev_free(cpos); dev_free(mstart); dev_free(mfill); dev_free(members); dev_free(ckey); dev_free(cw);
-        dev_free(hlist);
+        dev_free(sizes); dev_free(noff); dev_free(ncol); dev_free(hd); dev_free(wpre);
+        dev_free(cid); dev_free(members); dev_free(ckey); dev_free(mid); dev_free(tkey);
+        dev_free(nw); dev_free(cw); dev_free(tval);
         raw_free(tmp);
-        tmp = nullptr;
+        raw_free(tmp2);
+        tmp = tmp2 = nullptr;
     };
     int rc = NIDO_OK;
     // a failed HIP call leaves the loop with the error, and cleanup runs
@@ -1346,40 +1345,42 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         break;                                                                                             \
     }
     do {
-        if ((rc = dev_alloc(&arcs, K + 1)) || (rc = dev_alloc(&toff, K + 1)) ||
-            (rc = dev_alloc(&cnt, K + 1)) || (rc = dev_alloc(&noff, K + 1)) ||
-            (rc = dev_alloc(&cpos, K + 1)) || (rc = dev_alloc(&mstart, K + 1)) ||
-            (rc = dev_alloc(&mfill, K + 1)) || (rc = dev_alloc(&members, std::max<int64_t>(nv, 1))) ||
-            (rc = dev_alloc(&hlist, std::max<int64_t>(nv, 1))))
+        if ((rc = dev_alloc(&sizes, 7 * K1)) || (rc = dev_alloc(&noff, K1)) || (rc = dev_alloc(&mid, K1)) ||
+            (rc = dev_alloc(&cid, nv)) || (rc = dev_alloc(&members, nv)) ||
+            (rc = raw_alloc(&tmp, 4 * scan_temp_bytes(K1))))
             break;
-        if ((rc = raw_alloc(&tmp, scan_temp_bytes(K + 1)))) break;
+        int64_t *const arcs = sizes, *const cnt = sizes + K1;
+        unsigned long long* const mfill = reinterpret_cast<unsigned long long*>(sizes + 2 * K1);
+        const CoarseRows R{sizes + 3 * K1, sizes + 4 * K1, sizes + 5 * K1, sizes + 6 * K1, mid, mfill + K};
         // per coarse row: its arcs and members; rows of few arcs are
         // aggregated in LDS (compact entries at cpos), the others in HBM
         // tables (toff)
-        launch_fill_i64(arcs, 0, K + 1, s);
-        launch_fill_i64(cnt, 0, K + 1, s);
-        launch_fill_i64(reinterpret_cast<int64_t*>(mfill), 0, K + 1, s);   // [K]: HBM-row vertices
-        launch_member_counts(g->d_C, newid, g->d_off, nv, cnt, arcs, s, gid, keep);
-        launch_exclusive_scan(cnt, mstart, K, mstart + K, tmp, s);
-        launch_coarse_sizes(arcs, K, toff, cpos, s);
-        launch_exclusive_scan(toff, toff, K, toff + K, tmp, s);
-        launch_exclusive_scan(cpos, cpos, K, cpos + K, tmp, s);
-        int64_t T = 0, Tc = 0;
-        COARSEN_HIP(hipMemcpyAsync(&T, toff + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipMemcpyAsync(&Tc, cpos + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        launch_fill_i64(sizes, 0, 3 * K1, s);
+        launch_member_counts(g->d_C, newid, g->d_off, nv, cid, cnt, arcs, s, gid, keep);
+        launch_coarse_sizes(arcs, cnt, K, R, s);
+        launch_exclusive_scans(R.ml, K, 4, K1, tmp, s);
+        int64_t ML = 0, MH = 0, T = 0, Tc = 0;
+        COARSEN_HIP(hipMemcpyAsync(&ML, R.ml + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        COARSEN_HIP(hipMemcpyAsync(&MH, R.mh + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        COARSEN_HIP(hipMemcpyAsync(&T, R.toff + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        COARSEN_HIP(hipMemcpyAsync(&Tc, R.cpos + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         COARSEN_HIP(hipStreamSynchronize(s));
-        if ((rc = dev_alloc(&tkey, std::max<int64_t>(T, 1))) || (rc = dev_alloc(&tval, std::max<int64_t>(T, 1))) ||
-            (rc = dev_alloc(&ckey, std::max<int64_t>(Tc, 1))) || (rc = dev_alloc(&cw, std::max<int64_t>(Tc, 1))))
+        const int64_t nwords = T / kSlotWord;
+        if ((rc = dev_alloc(&ckey, Tc)) || (rc = dev_alloc(&cw, Tc)) || (rc = dev_alloc(&hd, MH + 1))) break;
+        if (T > 0 && ((rc = dev_alloc(&tkey, T)) || (rc = dev_alloc(&tval, T)) || (rc = dev_alloc(&wpre, nwords + 1)) ||
+                      (rc = raw_alloc(&tmp2, scan_temp_bytes(std::max(MH, nwords))))))
             break;
+        launch_member_scatter(cid, g->d_off, nv, R, ML, mfill, members, hd, s);
+        launch_coarse_lds(arcs, R, members, g->d_off, g->d_col32, g->d_w, cid, K, ckey, cw, cnt, s);
         if (T > 0) {
             launch_fill_i32(tkey, -1, T, s);
             launch_fill_fx(tval, T, s);
-        }
-        launch_member_scatter(g->d_C, newid, nv, mstart, mfill, members, toff, hlist, mfill + K, s, gid, keep);
-        launch_coarse_lds(arcs, mstart, members, g->d_off, g->d_col, g->d_w, g->d_C, newid, K, cpos, ckey, cw, cnt, s);
-        if (T > 0) {
-            launch_coarse_insert(g->d_off, g->d_col, g->d_w, g->d_C, newid, hlist, mfill + K, nv, toff, tkey, tval, s);
-            launch_coarse_count(toff, tkey, K, cnt, s);
+            launch_exclusive_scan(hd, hd, MH, hd + MH, tmp2, s);
+            launch_coarse_insert(hd, MH, g->ne, members + ML, cid, g->d_off, g->d_col32, g->d_w, R.toff, tkey, tval,
+                                 s);
+            launch_slot_words(tkey, nwords, wpre, s);
+            launch_exclusive_scan(wpre, wpre, nwords, wpre + nwords, tmp2, s);
+            launch_coarse_count(R.toff, wpre, K, cnt, s);
         }
         launch_exclusive_scan(cnt, noff, K, noff + K, tmp, s);
         COARSEN_HIP(hipGetLastError());
@@ -1388,7 +1389,8 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         COARSEN_HIP(hipStreamSynchronize(s));
         const int64_t nne = hoff[(size_t)K];
         if ((rc = dev_alloc(&ncol, nne)) || (rc = dev_alloc(&nw, nne))) break;
-        launch_coarse_emit(toff, tkey, tval, K, noff, ncol, nw, cpos, ckey, cw, s);
+        launch_coarse_emit(R.toff, K, noff, ncol, nw, R.cpos, ckey, cw, s);
+        launch_coarse_emit_hbm(R.toff, tkey, tval, K, wpre, nwords, noff, ncol, nw, s);
         COARSEN_HIP(hipGetLastError());
         COARSEN_HIP(hipStreamSynchronize(s));
         free_graph_arrays(g);

@@ -309,6 +309,9 @@ void launch_graph_sums(const fx_t* k, const int64_t* vb, int G, fx_t* out, hipSt
 size_t scan_temp_bytes(int64_t n);
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* total,
                            void* temp, hipStream_t s);
+// In place over `rows` arrays of n values, stride apart, each total at the
+// array's [n] (temp: rows * scan_temp_bytes(n)).
+void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, void* temp, hipStream_t s);
 
 // ---- coarsening ------------------------------------------------------------
 // With gid (per current vertex) / gid0 (per original vertex) set, only the
@@ -328,33 +331,45 @@ void launch_widen_local(const ArcPiece* pieces, int64_t n, const uint16_t* local
 // out[i] = clus[i] - base[gid0[i]] for the n0 original vertices.
 void launch_local_ids(const int64_t* clus, int64_t n0, const int* gid0, const int64_t* base, int64_t* out,
                       hipStream_t s);
-void launch_member_counts(const int64_t* C, const int64_t* newid, const int64_t* off, int64_t nv,
+// Coarse rows of at most kWaveRowArcs arcs are aggregated in LDS by one
+// wavefront, of at most kLdsRowArcs by one workgroup, longer ones in HBM
+// hash tables of whole kSlotWord-slot words.
+constexpr int64_t kWaveRowArcs = 64;
+constexpr int64_t kLdsRowArcs = 1024;
+constexpr int64_t kSlotWord = 64;
+// Per coarse row i, scanned over the rows (K + 1 entries each): the members
+// of LDS rows (ml) and of HBM rows (mh), table slots (toff, none for an LDS
+// row) and compact entries (cpos, none for an HBM row).  mid[0, *nmid): the
+// LDS rows a workgroup aggregates.
+struct CoarseRows {
+    int64_t *ml, *mh, *toff, *cpos;
+    int* mid;
+    unsigned long long* nmid;
+};
+// cid[v] = coarse row of v (-1: not kept); cnt / arcs: members and arcs per row.
+void launch_member_counts(const int64_t* C, const int64_t* newid, const int64_t* off, int64_t nv, int* cid,
                           int64_t* cnt, int64_t* arcs, hipStream_t s, const int* gid = nullptr,
                           const unsigned char* keep = nullptr);
-// Coarse rows of at most kLdsRowArcs arcs are aggregated in LDS, one
-// workgroup each, longer ones in HBM hash tables: tsz[i] table slots (0 for
-// an LDS row), csz[i] compact entries (0 for a table row).
-constexpr int64_t kLdsRowArcs = 1024;
-void launch_coarse_sizes(const int64_t* arcs, int64_t K, int64_t* tsz, int64_t* csz, hipStream_t s);
-// members[mstart[i] ...]: the vertices of coarse row i (mfill zeroed, K);
-// hlist[0, *nh): the vertices of rows with an HBM table (*nh zeroed).
-void launch_member_scatter(const int64_t* C, const int64_t* newid, int64_t nv, const int64_t* mstart,
-                           unsigned long long* mfill, int* members, const int64_t* toff, int* hlist,
-                           unsigned long long* nh, hipStream_t s, const int* gid = nullptr,
-                           const unsigned char* keep = nullptr);
+// The unscanned sizes into R, and R.mid (*R.nmid zeroed).
+void launch_coarse_sizes(const int64_t* arcs, const int64_t* cnt, int64_t K, const CoarseRows& R, hipStream_t s);
+// members[R.ml[i] ...): the vertices of LDS row i; members[ML + R.mh[i] ...):
+// those of HBM row i, their degrees at hd[R.mh[i] ...) (mfill zeroed, K).
+void launch_member_scatter(const int* cid, const int64_t* off, int64_t nv, const CoarseRows& R, int64_t ML,
+                           unsigned long long* mfill, int* members, int64_t* hd, hipStream_t s);
 // The LDS rows: distinct targets at ckey/cw[cpos[i] ...), their count in cnt[i].
-void launch_coarse_lds(const int64_t* arcs, const int64_t* mstart, const int* members, const int64_t* off,
-                       const int64_t* col, const double* w, const int64_t* C, const int64_t* newid, int64_t K,
-                       const int64_t* cpos, int* ckey, double* cw, int64_t* cnt, hipStream_t s);
-// The HBM-table rows: every listed vertex's arcs (hlist[0, *nh), nmax >= *nh
-// sizes the grid).
-void launch_coarse_insert(const int64_t* off, const int64_t* col, const double* w, const int64_t* C,
-                          const int64_t* newid, const int* hlist, const unsigned long long* nh, int64_t nmax,
-                          const int64_t* toff, int* tkey, fx_t* tval, hipStream_t s);
-void launch_coarse_count(const int64_t* toff, const int* tkey, int64_t K, int64_t* cnt,
-                         hipStream_t s);
-void launch_coarse_emit(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K,
-                        const int64_t* noff, int64_t* ncol, double* nw, const int64_t* cpos, const int* ckey,
-                        const double* cw, hipStream_t s);
+void launch_coarse_lds(const int64_t* arcs, const CoarseRows& R, const int* members, const int64_t* off,
+                       const int* col, const double* w, const int* cid, int64_t K, int* ckey, double* cw,
+                       int64_t* cnt, hipStream_t s);
+// The HBM rows: the arcs of members[0, n), whose degrees scan to hpre[0, n]
+// (max_arcs >= hpre[n] sizes the grid).
+void launch_coarse_insert(const int64_t* hpre, int64_t n, int64_t max_arcs, const int* members, const int* cid,
+                          const int64_t* off, const int* col, const double* w, const int64_t* toff, int* tkey,
+                          fx_t* tval, hipStream_t s);
+void launch_slot_words(const int* tkey, int64_t nwords, int64_t* wcnt, hipStream_t s);
+void launch_coarse_count(const int64_t* toff, const int64_t* wpre, int64_t K, int64_t* cnt, hipStream_t s);
+void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, double* nw,
+                        const int64_t* cpos, const int* ckey, const double* cw, hipStream_t s);
+void launch_coarse_emit_hbm(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K, const int64_t* wpre,
+                            int64_t nwords, const int64_t* noff, int64_t* ncol, double* nw, hipStream_t s);
 
 }  // namespace nido

@@ -405,7 +405,8 @@ mod_finish_graphs_kernel(ModDelta D, int nb, int G, double* __restrict__ q, cons
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive scan (int64), tiles of 2048 values per 256-thread workgroup.
+// Exclusive scan (int64), tiles of 2048 values per 256-thread workgroup;
+// blockIdx.y picks one of several arrays, stride apart.
 // ---------------------------------------------------------------------------
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;
@@ -432,9 +433,11 @@ __device__ __forceinline__ int64_t block_excl_scan(int64_t x, int64_t* warp_tot,
 }
 
 __global__ void __launch_bounds__(kBlock)
-scan_tile_sums_kernel(const int64_t* __restrict__ in, int64_t n, int64_t* __restrict__ sums)
+scan_tile_sums_kernel(const int64_t* __restrict__ in, int64_t n, int64_t* __restrict__ sums, int64_t stride)
 {
     __shared__ int64_t wt[kBlock / 64];
+    in += blockIdx.y * stride;
+    sums += (int64_t)blockIdx.y * gridDim.x;
     const int64_t t0 = (int64_t)blockIdx.x * kScanTile;
     int64_t s = 0;
 #pragma unroll
@@ -449,9 +452,13 @@ scan_tile_sums_kernel(const int64_t* __restrict__ in, int64_t n, int64_t* __rest
 
 __global__ void __launch_bounds__(kBlock)
 scan_tile_apply_kernel(const int64_t* in, int64_t* out, int64_t n,
-                       const int64_t* __restrict__ tile_off, int64_t* total)
+                       const int64_t* __restrict__ tile_off, int64_t* total, int64_t stride)
 {
     __shared__ int64_t wt[kBlock / 64];
+    in += blockIdx.y * stride;
+    out += blockIdx.y * stride;
+    if (tile_off) tile_off += (int64_t)blockIdx.y * gridDim.x;
+    if (total) total += blockIdx.y * stride;
     const int64_t t0 = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     int64_t v[kScanItems];
     int64_t s = 0;
@@ -534,9 +541,11 @@ __device__ __forceinline__ int group_slot(int* key, int i)
     }
 }
 
+// cid[v] = the coarse row of vertex v (-1: its graph does not take part),
+// and per coarse row its members and arcs.
 __global__ void __launch_bounds__(kBlock)
 member_counts_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ newid,
-                     const int64_t* __restrict__ off, int64_t nv, int64_t* __restrict__ cnt,
+                     const int64_t* __restrict__ off, int64_t nv, int* __restrict__ cid, int64_t* __restrict__ cnt,
                      int64_t* __restrict__ arcs, const int* __restrict__ gid,
                      const unsigned char* __restrict__ keep)
 {
@@ -550,16 +559,20 @@ member_counts_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ 
         }
         __syncthreads();
         const int64_t v = base + threadIdx.x;
-        if (v < nv && (!gid || keep[gid[v]])) {
-            const int h = group_slot(key, (int)newid[C[v]]);
-            atomicAdd(&nm[h], 1ull);
-            atomicAdd(&na[h], (unsigned long long)(off[v + 1] - off[v]));
+        if (v < nv) {
+            const int i = !gid || keep[gid[v]] ? (int)newid[C[v]] : -1;
+            cid[v] = i;
+            if (i >= 0) {
+                const int h = group_slot(key, i);
+                atomicAdd(&nm[h], 1ull);
+                atomicAdd(&na[h], (unsigned long long)(off[v + 1] - off[v]));
+            }
         }
         __syncthreads();
         for (int s = threadIdx.x; s < kGroupSlots; s += kBlock) {
             const int i = key[s];
             if (i < 0) continue;
-            if (cnt) atomicAdd(reinterpret_cast<unsigned long long*>(cnt + i), nm[s]);
+            atomicAdd(reinterpret_cast<unsigned long long*>(cnt + i), nm[s]);
             if (na[s]) atomicAdd(reinterpret_cast<unsigned long long*>(arcs + i), na[s]);
         }
         __syncthreads();   // the table is cleared for the next chunk
@@ -568,84 +581,196 @@ member_counts_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ 
 
 // Coarse row i with arcs[i] <= kLdsRowArcs is aggregated in LDS and needs
 // csz[i] = min(arcs, K) compact entries; a longer one gets an HBM hash table
-// of tsz[i] slots (a power of two >= twice its possible keys).
+// of tsz[i] slots (a power of two >= twice its possible keys, whole words of
+// kSlotWord slots).  ml / mh: the members of LDS and of HBM rows.  The rows
+// longer than a wavefront aggregates are listed in mid[0, *nmid).
 __global__ void __launch_bounds__(kBlock)
-coarse_sizes_kernel(const int64_t* __restrict__ arcs, int64_t K, int64_t* __restrict__ tsz,
-                    int64_t* __restrict__ csz)
+coarse_sizes_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ cnt, int64_t K,
+                    int64_t* __restrict__ ml, int64_t* __restrict__ mh, int64_t* __restrict__ tsz,
+                    int64_t* __restrict__ csz, int* __restrict__ mid, unsigned long long* __restrict__ nmid)
 {
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < K;
-         i += (int64_t)gridDim.x * kBlock) {
-        const int64_t need = arcs[i] < K ? arcs[i] : K;
-        int64_t s = 0;
-        if (arcs[i] > kLdsRowArcs) {
-            s = 2;
-            while (s < 2 * need) s <<= 1;
+    for (int64_t b = blockIdx.x * (int64_t)kBlock; b < K; b += (int64_t)gridDim.x * kBlock) {
+        const int64_t i = b + threadIdx.x;
+        bool listed = false;
+        if (i < K) {
+            const int64_t a = arcs[i], m = cnt[i];
+            const int64_t need = a < K ? a : K;
+            const bool hbm = a > kLdsRowArcs;
+            int64_t s = 0;
+            if (hbm) {
+                s = kSlotWord;
+                while (s < 2 * need) s <<= 1;
+            }
+            tsz[i] = s;
+            csz[i] = hbm ? 0 : need;
+            ml[i] = hbm ? 0 : m;
+            mh[i] = hbm ? m : 0;
+            listed = !hbm && a > kWaveRowArcs;
         }
-        tsz[i] = s;
-        csz[i] = arcs[i] > kLdsRowArcs ? 0 : need;
+        const unsigned long long w = __ballot(listed);
+        if (w) {   // uniform in the wavefront
+            unsigned long long at = 0;
+            if ((threadIdx.x & 63) == 0) at = atomicAdd(nmid, (unsigned long long)__popcll(w));
+            at = __shfl(at, 0, 64);
+            if (listed) mid[at + __popcll(w & ((1ull << (threadIdx.x & 63)) - 1))] = (int)i;
+        }
     }
 }
 
-// members[mstart[i] + r] = the vertices of coarse row i, in no set order,
-// and hlist[0, *nh) the vertices whose row has an HBM table (toff[i + 1] >
-// toff[i]).  Each workgroup reserves a block of its rows' member slots with
-// one atomic per distinct row (grouped in LDS as in member_counts_kernel).
+// members[ml[i] ...) = the vertices of LDS row i and members[ML + mh[i] ...)
+// those of HBM row i (ML = ml[K]), in no set order inside a row; hd gets the
+// degree of every HBM row's member.  Each workgroup reserves a block of its
+// rows' member slots with one atomic per distinct row (grouped in LDS as in
+// member_counts_kernel).
 __global__ void __launch_bounds__(kBlock)
-member_scatter_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ newid, int64_t nv,
-                      const int64_t* __restrict__ mstart, unsigned long long* __restrict__ mfill,
-                      int* __restrict__ members, const int64_t* __restrict__ toff, int* __restrict__ hlist,
-                      unsigned long long* __restrict__ nh, const int* __restrict__ gid,
-                      const unsigned char* __restrict__ keep)
+member_scatter_kernel(const int* __restrict__ cid, const int64_t* __restrict__ off, int64_t nv,
+                      const int64_t* __restrict__ ml, const int64_t* __restrict__ mh, int64_t ML,
+                      const int64_t* __restrict__ toff, unsigned long long* __restrict__ mfill,
+                      int* __restrict__ members, int64_t* __restrict__ hd)
 {
     __shared__ int key[kGroupSlots];
     __shared__ unsigned nm[kGroupSlots];
     __shared__ unsigned long long at[kGroupSlots];
-    __shared__ unsigned s_nh;
-    __shared__ unsigned long long s_hbase;
     for (int64_t base = blockIdx.x * (int64_t)kBlock; base < nv; base += (int64_t)gridDim.x * kBlock) {
         for (int s = threadIdx.x; s < kGroupSlots; s += kBlock) {
             key[s] = -1;
             nm[s] = 0;
         }
-        if (threadIdx.x == 0) s_nh = 0;
         __syncthreads();
         const int64_t v = base + threadIdx.x;
-        int64_t i = -1;
+        const int i = v < nv ? cid[v] : -1;
         int h = 0;
-        unsigned rank = 0, hrank = 0;
-        bool hbm = false;
-        if (v < nv && (!gid || keep[gid[v]])) {
-            i = newid[C[v]];
-            h = group_slot(key, (int)i);
+        unsigned rank = 0;
+        if (i >= 0) {
+            h = group_slot(key, i);
             rank = atomicAdd(&nm[h], 1u);
-            hbm = toff[i + 1] > toff[i];
-            if (hbm) hrank = atomicAdd(&s_nh, 1u);
         }
         __syncthreads();
         for (int s = threadIdx.x; s < kGroupSlots; s += kBlock)
             if (key[s] >= 0) at[s] = atomicAdd(mfill + key[s], (unsigned long long)nm[s]);
-        if (threadIdx.x == 0 && s_nh) s_hbase = atomicAdd(nh, (unsigned long long)s_nh);
         __syncthreads();
-        if (i >= 0) members[mstart[i] + (int64_t)(at[h] + rank)] = (int)v;
-        if (hbm) hlist[s_hbase + hrank] = (int)v;
+        if (i >= 0) {
+            const int64_t r = (int64_t)(at[h] + rank);
+            if (toff[i + 1] > toff[i]) {
+                members[ML + mh[i] + r] = (int)v;
+                hd[mh[i] + r] = off[v + 1] - off[v];
+            } else {
+                members[ml[i] + r] = (int)v;
+            }
+        }
         __syncthreads();   // the table is cleared for the next chunk
     }
 }
 
-// Coarse rows of at most kLdsRowArcs arcs, one workgroup each: the arcs of
-// its members (their concatenation, 256 at a time, each thread locating its
-// member by binary search over the scanned lengths) go into an LDS table
-// keyed by the coarse target, with exact Q64.64 sums; the arcs into the row
-// itself are summed per wavefront first and inserted once.  The row's
-// distinct targets land compactly at ckey/cw[cpos[i] ...) and their count
-// in cnt[i].  Keys whose weights sum to zero are kept, as in the HBM tables.
+// Coarse rows of at most kWaveRowArcs arcs, one wavefront each: a row has at
+// most as many members as arcs (or one member without arcs), so each lane
+// holds one member, the lengths are scanned with shuffles, and each lane
+// then takes one arc and inserts its coarse target into the wavefront's
+// 128-slot LDS table.  No workgroup barrier: most coarse rows of a sparse
+// graph are this short; bound by the round trips of a row (members, offsets,
+// arcs, ids), of which 8,192 wavefronts keep as many in flight.  R-MAT scale
+// 20's first coarse graph (316 K rows): 33 us, against 880 us with a
+// workgroup per row.
+constexpr int kWaveSlots = 2 * (int)kWaveRowArcs;
+__global__ void __launch_bounds__(kBlock)
+coarse_wave_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ ml,
+                   const int* __restrict__ members, const int64_t* __restrict__ off, const int* __restrict__ col,
+                   const double* __restrict__ w, const int* __restrict__ cid, int64_t K,
+                   const int64_t* __restrict__ cpos, int* __restrict__ ckey, double* __restrict__ cw,
+                   int64_t* __restrict__ cnt)
+{
+    __shared__ int s_key[kBlock / 64][kWaveSlots];
+    __shared__ unsigned long long s_lo[kBlock / 64][kWaveSlots], s_hi[kBlock / 64][kWaveSlots];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int* const key = s_key[wv];
+    unsigned long long *const lo = s_lo[wv], *const hi = s_hi[wv];
+    const int64_t nw = (int64_t)gridDim.x * (kBlock / 64);
+    for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + wv; i < K; i += nw) {   // uniform in the wavefront
+        const int64_t a = arcs[i];
+        if (a > kWaveRowArcs) continue;      // a longer LDS row or an HBM row
+        if (a == 0) {
+            if (lane == 0) cnt[i] = 0;
+            continue;
+        }
+#pragma unroll
+        for (int s = lane; s < kWaveSlots; s += 64) {
+            key[s] = -1;
+            lo[s] = 0;
+            hi[s] = 0;
+        }
+        const int64_t m0 = ml[i];
+        const int nm = (int)(ml[i + 1] - m0);   // <= a <= 64
+        int d = 0;
+        int64_t e0 = 0;
+        if (lane < nm) {
+            const int v = members[m0 + lane];
+            e0 = off[v];
+            d = (int)(off[v + 1] - e0);
+        }
+        int inc = d;
+#pragma unroll
+        for (int k = 1; k < 64; k <<= 1) {
+            const int y = __shfl_up(inc, k, 64);
+            if (lane >= k) inc += y;
+        }
+        int l = 0;   // the member of this lane's arc: members that end at or before it
+#pragma unroll
+        for (int sft = 32; sft > 0; sft >>= 1)
+            if (__shfl(inc, l + sft - 1, 64) <= lane) l += sft;
+        const int start = __shfl(inc, l, 64) - __shfl(d, l, 64);
+        const int64_t e = __shfl(e0, l, 64) + (lane - start);
+        wave_lds_sync();
+        if (lane < a) {
+            const int j = cid[col[e]];
+            const fx_t x = fx_from_double(w[e]);
+            unsigned h = ((unsigned)j * kHashMul) >> (32 - ilog2c(kWaveSlots));
+            for (;;) {   // ends: at most 64 of the 128 slots are taken
+                const int kk = key[h];
+                if (kk == j) break;
+                if (kk < 0) {
+                    const int prev = atomicCAS(&key[h], -1, j);
+                    if (prev < 0 || prev == j) break;
+                }
+                h = (h + 1) & (kWaveSlots - 1);
+            }
+            fx_atomic_add(&lo[h], &hi[h], x);
+        }
+        wave_lds_sync();
+        const int64_t base = cpos[i];
+        int n = 0;
+#pragma unroll
+        for (int s0 = 0; s0 < kWaveSlots; s0 += 64) {
+            const int s = s0 + lane;
+            const int j = key[s];
+            const unsigned long long m = __ballot(j >= 0);
+            if (j >= 0) {
+                const int r = n + __popcll(m & ((1ull << lane) - 1));
+                ckey[base + r] = j;
+                cw[base + r] = fx_to_double(fx_make(lo[s], (int64_t)hi[s]));
+            }
+            n += __popcll(m);
+        }
+        if (lane == 0) cnt[i] = n;
+        wave_lds_sync();                     // read before the next row clears the table
+    }
+}
+
+// The listed coarse rows (more than kWaveRowArcs, at most kLdsRowArcs arcs),
+// one workgroup each: the arcs of its members (their concatenation, 256 at a
+// time, each thread locating its member by binary search over the scanned
+// lengths) go into an LDS table keyed by the coarse target, with exact Q64.64
+// sums; the arcs into the row itself are summed per wavefront first and
+// inserted once.  The row's distinct targets land compactly at ckey/cw[cpos[i]
+// ...) and their count in cnt[i].  Keys whose weights sum to zero are kept,
+// as in the HBM tables.
 constexpr int kLdsSlots = 2 * kLdsRowArcs;
 __global__ void __launch_bounds__(kBlock)
-coarse_lds_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ mstart,
+coarse_lds_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ ml,
                   const int* __restrict__ members, const int64_t* __restrict__ off,
-                  const int64_t* __restrict__ col, const double* __restrict__ w, const int64_t* __restrict__ C,
-                  const int64_t* __restrict__ newid, int64_t K, const int64_t* __restrict__ cpos,
-                  int* __restrict__ ckey, double* __restrict__ cw, int64_t* __restrict__ cnt)
+                  const int* __restrict__ col, const double* __restrict__ w, const int* __restrict__ cid, int64_t K,
+                  const int* __restrict__ mid, const unsigned long long* __restrict__ nmid,
+                  const int64_t* __restrict__ cpos, int* __restrict__ ckey, double* __restrict__ cw,
+                  int64_t* __restrict__ cnt)
 {
     __shared__ int key[kLdsSlots];
     __shared__ unsigned long long lo[kLdsSlots], hi[kLdsSlots];
@@ -654,9 +779,10 @@ coarse_lds_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ 
     __shared__ int64_t s_e0[kBlock];
     __shared__ int s_nk;
     const int lane = threadIdx.x & 63;
-    for (int64_t i = blockIdx.x; i < K; i += gridDim.x) {
+    const int64_t n = (int64_t)*nmid;
+    for (int64_t t = blockIdx.x; t < n; t += gridDim.x) {
+        const int64_t i = mid[t];
         const int64_t a = arcs[i];
-        if (a > kLdsRowArcs) continue;   // uniform: an HBM-table row
         const int64_t need = a < K ? a : K;
         int lg = 6;
         while ((1ll << lg) < 2 * need) ++lg;
@@ -688,8 +814,8 @@ coarse_lds_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ 
         };
         fx_t self = 0;
         bool any_self = false;           // uniform in the wavefront
-        const int64_t m1 = mstart[i + 1];
-        for (int64_t m0 = mstart[i]; m0 < m1; m0 += kBlock) {   // uniform
+        const int64_t m1 = ml[i + 1];
+        for (int64_t m0 = ml[i]; m0 < m1; m0 += kBlock) {   // uniform
             const int64_t mi = m0 + threadIdx.x;
             int d = 0;
             int64_t e0 = 0;
@@ -715,7 +841,7 @@ coarse_lds_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ 
                     for (int st = top; st > 0; st >>= 1)
                         if (l + st < nm && s_pre[l + st] <= p) l += st;
                     const int64_t e = s_e0[l] + (p - s_pre[l]);
-                    j = (int)newid[C[col[e]]];
+                    j = cid[col[e]];
                     x = fx_from_double(w[e]);
                 }
                 const bool own = j == (int)i;
@@ -762,63 +888,205 @@ __device__ __forceinline__ void coarse_insert_one(int64_t i, int j, fx_t wf,
     fx_atomic_add(&val[2 * h], &val[2 * h + 1], wf);
 }
 
-// Every fine arc (u->x, w) goes into coarse row new(u) under key new(x);
-// internal arcs and old self-loops become the coarse self-loop
-// (graph_gpu.cpp:1233-1250).  Grid-stride over vertices, one wavefront per
-// vertex so that long rows stay coalesced.  The arcs of a row that land in
-// its own coarse vertex (most of them once communities have formed) are
-// summed across the wavefront first and inserted once: otherwise they all
-// take device atomics on the same self-loop slot.  The sums are exact
-// integers, so the grouping does not change them.
+// The rows with an HBM table: every fine arc (u->x, w) goes into coarse row
+// cid[u] under key cid[x]; internal arcs and old self-loops become the coarse
+// self-loop (graph_gpu.cpp:1233-1250).  The arcs of these rows' members, in
+// member order, are one flat range cut into tiles of kInsTile arcs, one
+// workgroup each, so a hub vertex or a giant community costs what its arcs
+// cost (R-MAT scale 20's first coarse graph, 60 M arcs: 0.65 ms, against 13.0
+// ms with a wavefront per vertex, set by its hubs; a Chung-Lu graph of 8.9 M
+// arcs 0.44 against 1.0 ms).  What bounds it now are the LDS atomics of the
+// sums and the gathers of cid.  A tile first sums its arcs per (row,
+// target) in an LDS table and then adds each sum to the row's HBM table with
+// one atomic; an arc that finds no slot within kInsProbe goes to the HBM
+// table directly.  The arcs that land in their own row (most of them once
+// communities have formed) are summed in registers first.  The sums are
+// exact integers, so the grouping does not change them.
+constexpr int kInsTile = 4096, kInsSlots = 1024, kInsProbe = 8, kInsUnroll = 4;
 __global__ void __launch_bounds__(kBlock)
-coarse_insert_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
-                     const double* __restrict__ w, const int64_t* __restrict__ C,
-                     const int64_t* __restrict__ newid, const int* __restrict__ hlist,
-                     const unsigned long long* __restrict__ nh, const int64_t* __restrict__ toff,
-                     int* __restrict__ tkey, fx_t* __restrict__ tval)
+coarse_insert_kernel(const int64_t* __restrict__ hpre, int64_t n, const int* __restrict__ members,
+                     const int* __restrict__ cid, const int64_t* __restrict__ off, const int* __restrict__ col,
+                     const double* __restrict__ w, const int64_t* __restrict__ toff, int* __restrict__ tkey,
+                     fx_t* __restrict__ tval)
+{
+    constexpr unsigned long long kEmpty = ~0ull;
+    __shared__ unsigned long long key[kInsSlots], lo[kInsSlots], hi[kInsSlots];
+    __shared__ int s_pre[kBlock], s_row[kBlock];
+    __shared__ int64_t s_e0[kBlock];
+    __shared__ int64_t s_m0;
+    __shared__ int s_end;
+    const int64_t A = hpre[n];
+    for (int64_t t0 = (int64_t)blockIdx.x * kInsTile; t0 < A; t0 += (int64_t)gridDim.x * kInsTile) {
+        const int64_t t1 = t0 + kInsTile < A ? t0 + kInsTile : A;
+        for (int s = threadIdx.x; s < kInsSlots; s += kBlock) {
+            key[s] = kEmpty;
+            lo[s] = 0;
+            hi[s] = 0;
+        }
+        // the last member whose arcs start at or before t0: a 64-way search
+        // by the first wavefront (hpre[l] <= t0 < hpre[r] throughout)
+        if (threadIdx.x < 64) {
+            int64_t l = 0, r = n;
+            while (r - l > 1) {
+                const int64_t step = (r - l + 63) / 64;
+                const int64_t at = l + (threadIdx.x + 1) * step;
+                const int c = __popcll(__ballot(at < r && hpre[at] <= t0));
+                r = l + (c + 1) * step < r ? l + (c + 1) * step : r;
+                l += c * step;
+            }
+            if (threadIdx.x == 0) s_m0 = l;
+        }
+        __syncthreads();
+        auto insert = [&](int i, int j, fx_t x) {
+            const unsigned long long k = ((unsigned long long)(unsigned)i << 32) | (unsigned)j;
+            unsigned h = (((unsigned)j ^ ((unsigned)i * kPartMul)) * kHashMul) >> (32 - ilog2c(kInsSlots));
+            for (int probe = 0; probe < kInsProbe; ++probe) {
+                unsigned long long kk = key[h];
+                if (kk == kEmpty) kk = atomicCAS(&key[h], kEmpty, k);
+                if (kk == kEmpty || kk == k) {
+                    fx_atomic_add(&lo[h], &hi[h], x);
+                    return;
+                }
+                h = (h + 1) & (kInsSlots - 1);
+            }
+            coarse_insert_one(i, j, x, toff, tkey, tval);
+        };
+        int own = -1;                      // the row whose self arcs `self` holds
+        fx_t self = 0;
+        for (int64_t m0 = s_m0;; m0 += kBlock) {   // uniform: chunks of kBlock members
+            const int64_t q = m0 + threadIdx.x;
+            const int64_t a = q < n ? hpre[q] : A, z = q < n ? hpre[q + 1] : A;
+            const int64_t a1 = a < t0 ? t0 : a < t1 ? a : t1;
+            s_pre[threadIdx.x] = (int)(a1 - t0);
+            if (z > t0 && a < t1 && z > a) {
+                const int v = members[q];
+                s_e0[threadIdx.x] = off[v] - a;
+                s_row[threadIdx.x] = cid[v];
+            }
+            if (threadIdx.x == kBlock - 1) s_end = (int)((z < t1 ? z : t1) - t0);
+            __syncthreads();
+            const int c0 = s_pre[0], c1 = s_end;
+            for (int x0 = c0; x0 < c1; x0 += kInsUnroll * kBlock) {
+                int row[kInsUnroll], tgt[kInsUnroll];
+                double wt[kInsUnroll];
+#pragma unroll
+                for (int r = 0; r < kInsUnroll; ++r) {
+                    const int x = x0 + r * kBlock + threadIdx.x;
+                    row[r] = -1;
+                    tgt[r] = 0;
+                    wt[r] = 0.0;
+                    if (x < c1) {
+                        int l = 0;         // the last member of the chunk whose arcs start at or before x
+#pragma unroll
+                        for (int st = kBlock / 2; st > 0; st >>= 1)
+                            if (s_pre[l + st] <= x) l += st;
+                        const int64_t e = s_e0[l] + t0 + x;
+                        row[r] = s_row[l];
+                        tgt[r] = col[e];
+                        wt[r] = w[e];
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < kInsUnroll; ++r)
+                    if (row[r] >= 0) tgt[r] = cid[tgt[r]];
+#pragma unroll
+                for (int r = 0; r < kInsUnroll; ++r) {
+                    if (row[r] < 0) continue;
+                    const fx_t x = fx_from_double(wt[r]);
+                    if (tgt[r] != row[r]) {
+                        insert(row[r], tgt[r], x);
+                    } else if (own == row[r]) {
+                        self += x;
+                    } else {
+                        if (own >= 0) insert(own, own, self);
+                        own = row[r];
+                        self = x;
+                    }
+                }
+            }
+            __syncthreads();               // the chunk's arrays are rewritten
+            if (c1 >= (int)(t1 - t0)) break;   // uniform
+        }
+        if (own >= 0) insert(own, own, self);
+        __syncthreads();
+        for (int s = threadIdx.x; s < kInsSlots; s += kBlock) {
+            const unsigned long long k = key[s];
+            if (k != kEmpty)
+                coarse_insert_one((int64_t)(k >> 32), (int)(unsigned)k, fx_make(lo[s], (int64_t)hi[s]), toff, tkey,
+                                  tval);
+        }
+        __syncthreads();                   // the table is cleared for the next tile
+    }
+}
+
+// HBM tables are whole words of kSlotWord = 64 slots: wcnt[x] = the taken
+// slots of word x, one lane per slot.
+__global__ void __launch_bounds__(kBlock)
+slot_words_kernel(const int* __restrict__ tkey, int64_t nwords, int64_t* __restrict__ wcnt)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t wid = (blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * kBlock) >> 6;
-    const int64_t n = (int64_t)*nh;
-    for (int64_t t = wid; t < n; t += nw) {
-        const int64_t v = hlist[t];              // a vertex whose coarse row has an HBM table
-        const int64_t i = newid[C[v]];
-        const int64_t e1 = off[v + 1];
-        for (int64_t e0 = off[v]; e0 < e1; e0 += 64) {   // uniform trip count in the wavefront
-            const int64_t e = e0 + lane;
-            const bool on = e < e1;
-            const int j = on ? (int)newid[C[col[e]]] : -1;
-            const fx_t x = on ? fx_from_double(w[e]) : fx_t(0);
-            const bool self = on && j == (int)i;
-            const fx_t sx = wave_sum_fx(self ? x : fx_t(0));   // every lane takes part
-            const bool any_self = __ballot(self) != 0;
-            if (on && !self) coarse_insert_one(i, j, x, toff, tkey, tval);
-            if (lane == 0 && any_self) coarse_insert_one(i, (int)i, sx, toff, tkey, tval);
+    const int64_t nw = (int64_t)gridDim.x * (kBlock / 64);
+    for (int64_t x = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); x < nwords; x += nw) {
+        const unsigned long long m = __ballot(tkey[x * kSlotWord + lane] >= 0);
+        if (lane == 0) wcnt[x] = __popcll(m);
+    }
+}
+
+// cnt[i] = the entries of HBM row i, from the scanned word counts.
+__global__ void __launch_bounds__(kBlock)
+coarse_count_kernel(const int64_t* __restrict__ toff, const int64_t* __restrict__ wpre, int64_t K,
+                    int64_t* __restrict__ cnt)
+{
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < K; i += (int64_t)gridDim.x * kBlock) {
+        const int64_t a = toff[i], z = toff[i + 1];
+        if (z > a) cnt[i] = wpre[z / kSlotWord] - wpre[a / kSlotWord];
+    }
+}
+
+// The entries of the HBM tables into the coarse CSR, a wavefront per kEmitRun
+// consecutive words (one lane per slot): the first word's row by binary
+// search, the next ones by walking on.  A table spreads over as many
+// wavefronts as it has slots (R-MAT scale 20's first coarse graph, one
+// community holding a quarter of it: 0.09 ms, against 7.7 ms with a wavefront
+// per row, and 6.4 ms more to count them that way).
+constexpr int kEmitRun = 32;
+__global__ void __launch_bounds__(kBlock)
+coarse_emit_hbm_kernel(const int64_t* __restrict__ toff, const int* __restrict__ tkey,
+                       const fx_t* __restrict__ tval, int64_t K, const int64_t* __restrict__ wpre, int64_t nwords,
+                       const int64_t* __restrict__ noff, int64_t* __restrict__ ncol, double* __restrict__ nw_out)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t nw = (int64_t)gridDim.x * (kBlock / 64);
+    for (int64_t t = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); t * kEmitRun < nwords; t += nw) {
+        const int64_t x0 = t * kEmitRun, x1 = x0 + kEmitRun < nwords ? x0 + kEmitRun : nwords;
+        int64_t i = 0, r = K;              // toff[i] <= x0 * kSlotWord < toff[r]
+        while (r - i > 1) {
+            const int64_t mid = (i + r) / 2;
+            if (toff[mid] <= x0 * kSlotWord) i = mid;
+            else r = mid;
+        }
+        int64_t z = toff[i + 1], delta = noff[i] - wpre[toff[i] / kSlotWord];
+        for (int64_t x = x0; x < x1; ++x) {
+            while (z <= x * kSlotWord) {   // x < nwords: ends at a row with slots
+                ++i;
+                z = toff[i + 1];
+                if (z > x * kSlotWord) delta = noff[i] - wpre[toff[i] / kSlotWord];
+            }
+            const int64_t s = x * kSlotWord + lane;
+            const int c = tkey[s];
+            const unsigned long long m = __ballot(c >= 0);
+            if (c >= 0) {
+                const int64_t p = delta + wpre[x] + __popcll(m & ((1ull << lane) - 1));
+                ncol[p] = c;
+                nw_out[p] = fx_to_double(tval[s]);
+            }
         }
     }
 }
 
+// The compact entries of the LDS-aggregated rows into the coarse CSR.
 __global__ void __launch_bounds__(kBlock)
-coarse_count_kernel(const int64_t* __restrict__ toff, const int* __restrict__ tkey, int64_t K,
-                    int64_t* __restrict__ cnt)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t wid = (blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * kBlock) >> 6;
-    for (int64_t i = wid; i < K; i += nw) {
-        if (toff[i + 1] == toff[i]) continue;   // uniform: counted by the LDS aggregation
-        int64_t c = 0;
-        for (int64_t s = toff[i] + lane; s < toff[i + 1]; s += 64) c += ld_i32_agent(&tkey[s]) >= 0;
-#pragma unroll
-        for (int msk = 32; msk > 0; msk >>= 1) c += __shfl_xor(c, msk, 64);
-        if (lane == 0) cnt[i] = c;
-    }
-}
-
-__global__ void __launch_bounds__(kBlock)
-coarse_emit_kernel(const int64_t* __restrict__ toff, const int* __restrict__ tkey,
-                   const fx_t* __restrict__ tval, int64_t K, const int64_t* __restrict__ noff,
+coarse_emit_kernel(const int64_t* __restrict__ toff, int64_t K, const int64_t* __restrict__ noff,
                    int64_t* __restrict__ ncol, double* __restrict__ nw_out, const int64_t* __restrict__ cpos,
                    const int* __restrict__ ckey, const double* __restrict__ cw)
 {
@@ -826,27 +1094,11 @@ coarse_emit_kernel(const int64_t* __restrict__ toff, const int* __restrict__ tke
     const int64_t wid = (blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 6;
     const int64_t nw = ((int64_t)gridDim.x * kBlock) >> 6;
     for (int64_t i = wid; i < K; i += nw) {
-        int64_t pos = noff[i];
-        if (toff[i + 1] == toff[i]) {   // uniform: compact entries of an LDS-aggregated row
-            const int64_t n = noff[i + 1] - pos, c0 = cpos[i];
-            for (int64_t r = lane; r < n; r += 64) {
-                ncol[pos + r] = ckey[c0 + r];
-                nw_out[pos + r] = cw[c0 + r];
-            }
-            continue;
-        }
-        for (int64_t s0 = toff[i]; s0 < toff[i + 1]; s0 += 64) {
-            const int64_t s = s0 + lane;
-            const int c = s < toff[i + 1] ? ld_i32_agent(&tkey[s]) : -1;
-            const unsigned long long m = __ballot(c >= 0);
-            if (c >= 0) {
-                const unsigned long long below = lane ? (m & ((1ull << lane) - 1)) : 0ull;
-                const int64_t p = pos + __popcll(below);
-                const unsigned long long* vv = reinterpret_cast<const unsigned long long*>(tval + s);
-                ncol[p] = c;
-                nw_out[p] = fx_to_double(fx_make(ld_u64_agent(vv), (int64_t)ld_u64_agent(vv + 1)));
-            }
-            pos += __popcll(m);
+        if (toff[i + 1] != toff[i]) continue;   // uniform: an HBM row
+        const int64_t pos = noff[i], n = noff[i + 1] - pos, c0 = cpos[i];
+        for (int64_t r = lane; r < n; r += 64) {
+            ncol[pos + r] = ckey[c0 + r];
+            nw_out[pos + r] = cw[c0 + r];
         }
     }
 }
@@ -1072,6 +1324,22 @@ size_t scan_temp_bytes(int64_t n)
     return bytes + 64;
 }
 
+static void scan_rows(const int64_t* in, int64_t* out, int64_t n, int rows, int64_t stride, int64_t* total,
+                      void* temp, hipStream_t s)
+{
+    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    const dim3 grid((unsigned)tiles, (unsigned)rows);
+    if (tiles == 1) {
+        scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, nullptr, total, stride);
+        return;
+    }
+    int64_t* sums = reinterpret_cast<int64_t*>(temp);
+    void* rest = sums + tiles * rows;
+    scan_tile_sums_kernel<<<grid, kBlock, 0, s>>>(in, n, sums, stride);
+    scan_rows(sums, sums, tiles, rows, tiles, nullptr, rest, s);
+    scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, sums, total, stride);
+}
+
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* total,
                            void* temp, hipStream_t s)
 {
@@ -1079,16 +1347,12 @@ void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* 
         if (total) launch_fill_i64(total, 0, 1, s);
         return;
     }
-    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-    if (tiles == 1) {
-        scan_tile_apply_kernel<<<1, kBlock, 0, s>>>(in, out, n, nullptr, total);
-        return;
-    }
-    int64_t* sums = reinterpret_cast<int64_t*>(temp);
-    void* rest = sums + tiles;
-    scan_tile_sums_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(in, n, sums);
-    launch_exclusive_scan(sums, sums, tiles, nullptr, rest, s);
-    scan_tile_apply_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(in, out, n, sums, total);
+    scan_rows(in, out, n, 1, 0, total, temp, s);
+}
+
+void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, void* temp, hipStream_t s)
+{
+    if (n > 0) scan_rows(x, x, n, rows, stride, x + n, temp, s);
 }
 
 void launch_mark_communities(const int64_t* C, int64_t nv, int64_t* flag, hipStream_t s,
@@ -1115,45 +1379,46 @@ void launch_local_ids(const int64_t* clus, int64_t n0, const int* gid0, const in
     if (n0 > 0) local_ids_kernel<<<grid_for(n0, kBlock), kBlock, 0, s>>>(clus, n0, gid0, base, out);
 }
 
-void launch_member_counts(const int64_t* C, const int64_t* newid, const int64_t* off, int64_t nv,
-                          int64_t* cnt, int64_t* arcs, hipStream_t s, const int* gid,
-                          const unsigned char* keep)
+void launch_member_counts(const int64_t* C, const int64_t* newid, const int64_t* off, int64_t nv, int* cid,
+                          int64_t* cnt, int64_t* arcs, hipStream_t s, const int* gid, const unsigned char* keep)
 {
     if (nv > 0)
-        member_counts_kernel<<<grid_for(nv, kBlock), kBlock, 0, s>>>(C, newid, off, nv, cnt, arcs, gid,
-                                                                      keep);
+        member_counts_kernel<<<grid_for(nv, kBlock), kBlock, 0, s>>>(C, newid, off, nv, cid, cnt, arcs, gid, keep);
 }
 
-void launch_coarse_sizes(const int64_t* arcs, int64_t K, int64_t* tsz, int64_t* csz, hipStream_t s)
-{
-    if (K > 0) coarse_sizes_kernel<<<grid_for(K, kBlock), kBlock, 0, s>>>(arcs, K, tsz, csz);
-}
-
-void launch_member_scatter(const int64_t* C, const int64_t* newid, int64_t nv, const int64_t* mstart,
-                           unsigned long long* mfill, int* members, const int64_t* toff, int* hlist,
-                           unsigned long long* nh, hipStream_t s, const int* gid, const unsigned char* keep)
-{
-    if (nv > 0)
-        member_scatter_kernel<<<grid_for(nv, kBlock), kBlock, 0, s>>>(C, newid, nv, mstart, mfill, members, toff,
-                                                                       hlist, nh, gid, keep);
-}
-
-void launch_coarse_lds(const int64_t* arcs, const int64_t* mstart, const int* members, const int64_t* off,
-                       const int64_t* col, const double* w, const int64_t* C, const int64_t* newid, int64_t K,
-                       const int64_t* cpos, int* ckey, double* cw, int64_t* cnt, hipStream_t s)
+void launch_coarse_sizes(const int64_t* arcs, const int64_t* cnt, int64_t K, const CoarseRows& R, hipStream_t s)
 {
     if (K > 0)
-        coarse_lds_kernel<<<grid_for(K, 1, 8192), kBlock, 0, s>>>(arcs, mstart, members, off, col, w, C, newid, K,
-                                                                  cpos, ckey, cw, cnt);
+        coarse_sizes_kernel<<<grid_for(K, kBlock), kBlock, 0, s>>>(arcs, cnt, K, R.ml, R.mh, R.toff, R.cpos, R.mid,
+                                                                   R.nmid);
 }
 
-void launch_coarse_insert(const int64_t* off, const int64_t* col, const double* w, const int64_t* C,
-                          const int64_t* newid, const int* hlist, const unsigned long long* nh, int64_t nmax,
-                          const int64_t* toff, int* tkey, fx_t* tval, hipStream_t s)
+void launch_member_scatter(const int* cid, const int64_t* off, int64_t nv, const CoarseRows& R, int64_t ML,
+                           unsigned long long* mfill, int* members, int64_t* hd, hipStream_t s)
 {
-    if (nmax > 0)
-        coarse_insert_kernel<<<grid_for(nmax, kBlock / 64), kBlock, 0, s>>>(off, col, w, C, newid, hlist, nh,
-                                                                            toff, tkey, tval);
+    if (nv > 0)
+        member_scatter_kernel<<<grid_for(nv, kBlock), kBlock, 0, s>>>(cid, off, nv, R.ml, R.mh, ML, R.toff, mfill,
+                                                                       members, hd);
+}
+
+void launch_coarse_lds(const int64_t* arcs, const CoarseRows& R, const int* members, const int64_t* off,
+                       const int* col, const double* w, const int* cid, int64_t K, int* ckey, double* cw,
+                       int64_t* cnt, hipStream_t s)
+{
+    if (K <= 0) return;
+    coarse_wave_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(arcs, R.ml, members, off, col, w, cid, K, R.cpos,
+                                                                   ckey, cw, cnt);
+    coarse_lds_kernel<<<grid_for(K, 1, 2048), kBlock, 0, s>>>(arcs, R.ml, members, off, col, w, cid, K, R.mid,
+                                                              R.nmid, R.cpos, ckey, cw, cnt);
+}
+
+void launch_coarse_insert(const int64_t* hpre, int64_t n, int64_t max_arcs, const int* members, const int* cid,
+                          const int64_t* off, const int* col, const double* w, const int64_t* toff, int* tkey,
+                          fx_t* tval, hipStream_t s)
+{
+    if (n > 0)
+        coarse_insert_kernel<<<grid_for(max_arcs, kInsTile, 16384), kBlock, 0, s>>>(hpre, n, members, cid, off, col, w,
+                                                                                   toff, tkey, tval);
 }
 
 void launch_modularity_seg(const SegItem* items, int64_t nitems, const int* src, const int* col,
@@ -1185,19 +1450,30 @@ void launch_fill_gid(const int64_t* vb, int G, int* gid, hipStream_t s)
     if (G > 0) fill_gid_kernel<<<grid_for(G, 1, 8192), kBlock, 0, s>>>(vb, G, gid);
 }
 
-void launch_coarse_count(const int64_t* toff, const int* tkey, int64_t K, int64_t* cnt,
-                         hipStream_t s)
+void launch_slot_words(const int* tkey, int64_t nwords, int64_t* wcnt, hipStream_t s)
 {
-    if (K > 0) coarse_count_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(toff, tkey, K, cnt);
+    if (nwords > 0)
+        slot_words_kernel<<<grid_for(nwords, kBlock / 64, 16384), kBlock, 0, s>>>(tkey, nwords, wcnt);
 }
 
-void launch_coarse_emit(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K,
-                        const int64_t* noff, int64_t* ncol, double* nw, const int64_t* cpos, const int* ckey,
-                        const double* cw, hipStream_t s)
+void launch_coarse_count(const int64_t* toff, const int64_t* wpre, int64_t K, int64_t* cnt, hipStream_t s)
+{
+    if (K > 0) coarse_count_kernel<<<grid_for(K, kBlock), kBlock, 0, s>>>(toff, wpre, K, cnt);
+}
+
+void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, double* nw,
+                        const int64_t* cpos, const int* ckey, const double* cw, hipStream_t s)
 {
     if (K > 0)
-        coarse_emit_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(toff, tkey, tval, K, noff,
-                                                                       ncol, nw, cpos, ckey, cw);
+        coarse_emit_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(toff, K, noff, ncol, nw, cpos, ckey, cw);
+}
+
+void launch_coarse_emit_hbm(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K, const int64_t* wpre,
+                            int64_t nwords, const int64_t* noff, int64_t* ncol, double* nw, hipStream_t s)
+{
+    if (nwords > 0)
+        coarse_emit_hbm_kernel<<<grid_for(nwords, kEmitRun * (kBlock / 64)), kBlock, 0, s>>>(
+            toff, tkey, tval, K, wpre, nwords, noff, ncol, nw);
 }
 
 }  // namespace nido
