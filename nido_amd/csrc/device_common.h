@@ -345,6 +345,39 @@ __device__ __forceinline__ int block_excl_scan_i32(int x, int* wtot, int* total)
     return pre + inc - x;
 }
 
+// The slot of key i (i >= 0) in an LDS table of S slots (S a power of two,
+// empty slots -1), creating it if absent.  The caller bounds the keys by S / 2,
+// so probing ends.
+template <int S>
+__device__ __forceinline__ int lds_slot(int* key, int i)
+{
+    unsigned h = ((unsigned)i * kHashMul) >> (32 - ilog2c(S));
+    for (;;) {
+        const int kk = key[h];
+        if (kk == i) return (int)h;
+        if (kk < 0) {
+            const int prev = atomicCAS(&key[h], -1, i);
+            if (prev < 0 || prev == i) return (int)h;
+        }
+        h = (h + 1) & (S - 1);
+    }
+}
+
+// The last l of [lo, hi) with off[l] <= x, given off[lo] <= x < off[hi] and off
+// nondecreasing: a 64-way search by one whole wavefront.
+__device__ __forceinline__ int64_t wave_row_of(const int64_t* __restrict__ off, int64_t lo, int64_t hi, int64_t x)
+{
+    const int lane = threadIdx.x & 63;
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + 63) / 64;
+        const int64_t at = lo + (lane + 1) * step;
+        const int c = __popcll(__ballot(at < hi && off[at] <= x));
+        hi = lo + (c + 1) * step < hi ? lo + (c + 1) * step : hi;
+        lo += c * step;
+    }
+    return lo;
+}
+
 // Workgroup-wide argmax + self-weight reduction; result valid in thread 0.
 struct BlockRed {
     double g[kBlock / 64];

@@ -521,25 +521,10 @@ local_ids_kernel(const int64_t* __restrict__ clus, int64_t n0, const int* __rest
         out[i] = clus[i] - base[gid0[i]];
 }
 
-// The coarse rows of a workgroup's kBlock consecutive vertices, grouped in
-// an LDS table of 2 * kBlock slots (at most kBlock keys: half full at most,
-// so probing ends): vertices of one community are often neighbours in id,
-// and each distinct row then takes one global atomic instead of one per
-// vertex.  Returns the slot of row i (i >= 0).
+// The coarse rows of a workgroup's kBlock consecutive vertices are grouped in
+// an LDS table: vertices of one community are often neighbours in id, and
+// each distinct row then takes one global atomic instead of one per vertex.
 constexpr int kGroupSlots = 2 * kBlock;
-__device__ __forceinline__ int group_slot(int* key, int i)
-{
-    unsigned h = ((unsigned)i * kHashMul) >> (32 - ilog2c(kGroupSlots));
-    for (;;) {
-        const int kk = key[h];
-        if (kk == i) return (int)h;
-        if (kk < 0) {
-            const int prev = atomicCAS(&key[h], -1, i);
-            if (prev < 0 || prev == i) return (int)h;
-        }
-        h = (h + 1) & (kGroupSlots - 1);
-    }
-}
 
 // cid[v] = the coarse row of vertex v (-1: its graph does not take part),
 // and per coarse row its members and arcs.
@@ -563,7 +548,7 @@ member_counts_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ 
             const int i = !gid || keep[gid[v]] ? (int)newid[C[v]] : -1;
             cid[v] = i;
             if (i >= 0) {
-                const int h = group_slot(key, i);
+                const int h = lds_slot<kGroupSlots>(key, i);
                 atomicAdd(&nm[h], 1ull);
                 atomicAdd(&na[h], (unsigned long long)(off[v + 1] - off[v]));
             }
@@ -642,7 +627,7 @@ member_scatter_kernel(const int* __restrict__ cid, const int64_t* __restrict__ o
         int h = 0;
         unsigned rank = 0;
         if (i >= 0) {
-            h = group_slot(key, i);
+            h = lds_slot<kGroupSlots>(key, i);
             rank = atomicAdd(&nm[h], 1u);
         }
         __syncthreads();
@@ -923,17 +908,8 @@ coarse_insert_kernel(const int64_t* __restrict__ hpre, int64_t n, const int* __r
             lo[s] = 0;
             hi[s] = 0;
         }
-        // the last member whose arcs start at or before t0: a 64-way search
-        // by the first wavefront (hpre[l] <= t0 < hpre[r] throughout)
-        if (threadIdx.x < 64) {
-            int64_t l = 0, r = n;
-            while (r - l > 1) {
-                const int64_t step = (r - l + 63) / 64;
-                const int64_t at = l + (threadIdx.x + 1) * step;
-                const int c = __popcll(__ballot(at < r && hpre[at] <= t0));
-                r = l + (c + 1) * step < r ? l + (c + 1) * step : r;
-                l += c * step;
-            }
+        if (threadIdx.x < 64) {   // the last member whose arcs start at or before t0
+            const int64_t l = wave_row_of(hpre, 0, n, t0);
             if (threadIdx.x == 0) s_m0 = l;
         }
         __syncthreads();
