@@ -206,6 +206,8 @@ void launch_vertex_weights(const int64_t* off, const double* w, const int* small
                            const RowItem* items, int64_t nitems, fx_t* k, double* kd,
                            int64_t nv, fx_t* acc, unsigned long long* maxabs, fx_t* part, int* src,
                            hipStream_t s);
+// out[i] = x[i] rounded to FP64.
+void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s);
 void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k, int64_t nv,
                       hipStream_t s);
 // *fneed = the fractional bits the finest weight needs (max over nonzero

@@ -103,6 +103,14 @@ round_kernel(const fx_t* __restrict__ k, double* __restrict__ kd, int64_t n,
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
+// out[i] = FP64(x[i]).
+__global__ void __launch_bounds__(kBlock)
+fx_round_kernel(const fx_t* __restrict__ x, double* __restrict__ out, int64_t n)
+{
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
+        out[i] = fx_to_double(x[i]);
+}
+
 // out[0] = sum of part[0..n) (one workgroup).
 __global__ void __launch_bounds__(kBlock)
 sum_partials_kernel(const fx_t* __restrict__ part, int n, fx_t* out)
@@ -1218,6 +1226,11 @@ void launch_vertex_weights(const int64_t* off, const double* w, const int* small
     const unsigned g = grid_for(nv, kBlock, kPartBlocks);
     round_kernel<<<g, kBlock, 0, s>>>(k, kd, nv, maxabs, part);
     sum_partials_kernel<<<1, kBlock, 0, s>>>(part, (int)g, acc);
+}
+
+void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s)
+{
+    if (n > 0) fx_round_kernel<<<grid_for(n, kBlock), kBlock, 0, s>>>(x, out, n);
 }
 
 void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k, int64_t nv,
