@@ -32,25 +32,39 @@ def _expected(off, col, w, comm):
     ([14] * 3000 + [9000], 1),
 ])
 def test_noalloc_at_tile_edges(degrees, base):
-    import torch
+    import ctypes
     import nido_amd as na
+    from test_zz_no_alloc import _setup
+    _, hip = _setup()    # the library's own HIP runtime: another one cannot start after it in this process
     rng = np.random.default_rng(len(degrees) + base)
     nv, ne = len(degrees), sum(degrees)
     off = (base + np.concatenate([[0], np.cumsum(degrees)])).astype(np.int64)
     col = rng.integers(nv, size=base + ne)
     w = rng.integers(1, 2048, base + ne) / 1024.0
     comm = rng.integers(max(1, nv // 3), size=nv)
+    bad = col.copy()
+    bad[base + ne - 1] = nv
     print(f"case: {nv} rows, {ne} arcs from {base}", flush=True)
-    d = [torch.from_numpy(x).cuda() for x in (off, col, w, comm)]
-    q = torch.zeros(1, dtype=torch.float64, device="cuda")
-    stream = torch.cuda.current_stream().cuda_stream
-    for _ in range(2):                                          # the second call finds the first one's sums
-        na.modularity_noalloc(nv, base + ne, *(x.data_ptr() for x in d), q.data_ptr(), stream)
-        assert q.item() == _expected(off, col, w, comm)
-    bad = d[1].clone()
-    bad[base + ne - 1] = nv                                     # an id out of range: NaN, and only for this call
-    na.modularity_noalloc(nv, base + ne, d[0].data_ptr(), bad.data_ptr(), *(x.data_ptr() for x in d[2:]), q.data_ptr(),
-                          stream)
-    assert np.isnan(q.item())
-    na.modularity_noalloc(nv, base + ne, *(x.data_ptr() for x in d), q.data_ptr(), stream)
-    assert q.item() == _expected(off, col, w, comm)
+    dev, got = [], np.zeros(1)
+    try:
+        for x in (off, col, w, comm, bad, got):
+            p = ctypes.c_void_p()
+            assert hip.hipMalloc(ctypes.byref(p), x.nbytes) == 0
+            dev.append(p.value)
+            assert hip.hipMemcpy(p.value, x.ctypes.data, x.nbytes, 1) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        d_off, d_col, d_w, d_comm, d_bad, d_q = dev
+
+        def q(cols):
+            na.modularity_noalloc(nv, base + ne, d_off, cols, d_w, d_comm, d_q, 0)
+            assert hip.hipDeviceSynchronize() == 0
+            assert hip.hipMemcpy(got.ctypes.data, d_q, 8, 2) == 0
+            return float(got[0])
+        expected = _expected(off, col, w, comm)
+        for _ in range(2):                                      # the second call finds the first one's sums
+            assert q(d_col) == expected
+        assert np.isnan(q(d_bad))                               # an id out of range: NaN, and only for this call
+        assert q(d_col) == expected
+    finally:
+        for p in dev:
+            hip.hipFree(p)
