@@ -129,7 +129,7 @@ struct SmallBins {
     int blk0[NUM_SMALL_BINS + 3];          // first block of each bin, of the key fill, of the delta; end
 };
 
-// One workgroup's share of a long row: partition p of P (P a power of 2);
+// One workgroup's share of a long row: partition p of P;
 // `slot` indexes the row within its batch's list of long rows.  For P > 1
 // the row's chunk j (of kKeyChunkArcs arcs) has its buckets at
 // bkey/bw[k0 + j * kKeyChunkArcs ...] and its segment starts at

@@ -13,7 +13,7 @@
 //   d <= 16/32/64/128   8/16/32/64 lanes per vertex, LDS table of 2d..4d slots
 //   d <= 512    one workgroup per vertex, 1024-slot LDS table
 //   d >  512    long rows, split by a hash of the community id into
-//               P = 2^ceil(log2(d / part_arcs)) partitions, so that every
+//               P partitions (partitions_of in host_bins.cpp), so that every
 //               e_{v,c} is complete and exact in one workgroup's LDS table;
 //               the last of the P workgroups to finish combines the P
 //               partial argmaxes.  For P > 2, launch 1 buckets the row's
@@ -178,6 +178,12 @@ __device__ __forceinline__ int lane_rank(unsigned long long mask)
 {
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
                                           __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+// Partition of community c in a row of P: its hash scaled to [0, P).
+__device__ __forceinline__ int part_of_key(int c, int P)
+{
+    return (int)__umulhi((unsigned)c * kPartMul, (unsigned)P);
 }
 
 // The slot of key c in an LDS open-addressing table of S slots (S a power
@@ -428,7 +434,6 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
         Mass m;
         if (!graph_mass<Multi>(A, ch.v, m)) continue;   // uniform over the workgroup
         const int P = ch.P;
-        const int psh = 32 - (31 - __builtin_clz((unsigned)P));   // top log2(P) bits of the hash
         for (int s = threadIdx.x; s <= P; s += kBlock) cnt[s] = 0;
         __syncthreads();
         // cc: community key (-1 self arc, -2 past the chunk); rk: rank in
@@ -442,7 +447,7 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
         }
 #pragma unroll
         for (int j = 0; j < kFillUnroll; ++j) cc[j] = cc[j] >= 0 ? (cc[j] != ch.v ? A.C[cc[j]] : -1) : -2;
-        auto part_of = [&](int c) { return c == -2 ? -1 : c < 0 ? P : (int)(((unsigned)c * kPartMul) >> psh); };
+        auto part_of = [&](int c) { return c == -2 ? -1 : c < 0 ? P : part_of_key(c, P); };
 #pragma unroll
         for (int j = 0; j < kFillUnroll; ++j) {
             const int pj = part_of(cc[j]);
@@ -678,7 +683,6 @@ lm_big_kernel(LmArgs A, BigArgs B)
         const double ki = A.kd[v];
         const bool whole = c0 < 0;       // the row is read from the CSR (P = 1 or few partitions)
         const int nch = whole ? 0 : (int)((d + kKeyChunkArcs - 1) / kKeyChunkArcs);
-        const int psh = 32 - (31 - __builtin_clz((unsigned)P));   // top log2(P) bits of the hash
 
         // Segments of chunks [g * kBlock, g * kBlock + kBlock) of partition p:
         // s_pre = exclusive scan of their lengths, s_lo = their starts.
@@ -783,7 +787,7 @@ lm_big_kernel(LmArgs A, BigArgs B)
                 if (P > 1) {
 #pragma unroll
                     for (int r = 0; r < kFill; ++r)
-                        if (cs[r] >= 0 && (int)(((unsigned)cs[r] * kPartMul) >> psh) != p) cs[r] = -1;
+                        if (cs[r] >= 0 && part_of_key(cs[r], P) != p) cs[r] = -1;
                 }
 #pragma unroll
                 for (int r = 0; r < kFill; ++r) insert(cs[r], ws[r]);
