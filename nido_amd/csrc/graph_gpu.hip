@@ -263,6 +263,10 @@ struct nido_graph {
     int64_t wq_cap = 0;
     bool fixed = false;            // this phase's short rows sum in 64-bit fixed point (d_wq)
     double wscale = 1.0;           // 2^-F
+    WeightGrid* d_grid = nullptr;
+    WeightGrid grid{};             // of the current weights, once grid_known
+    bool grid_known = false;
+    bool narrowed = false;         // d_col32 mirrors the current d_col
     fx_t* d_part = nullptr;        // 2 * kPartBlocks reduction partials
     void* d_scan_tmp = nullptr;
     // scalars
@@ -819,7 +823,8 @@ int setup_phase(nido_graph* g)
             NIDO_TRY(upload(&g->d_items, items, g->stream));
         }
 
-        launch_narrow_ids(g->d_col, g->d_col32, g->ne, g->stream);
+        if (!g->narrowed) launch_narrow_ids(g->d_col, g->d_col32, g->ne, g->stream);
+        g->narrowed = true;
         unsigned long long* d_maxk = reinterpret_cast<unsigned long long*>(g->d_tot + 1);
         launch_vertex_weights(g->d_off, g->d_w, g->d_small, g->nsmall, g->d_items, g->nitems, g->d_k,
                               g->d_kd, nv, g->d_acc + 2, d_maxk, g->d_part, g->d_src, g->stream);
@@ -844,17 +849,15 @@ int setup_phase(nido_graph* g)
     // (scaled by 2^(64 - F)), one word and no carry per LDS update.
     g->fixed = false;
     if (g->tuning.fixed_short && g->ne > 0 && g->twom != 0 && !g->windowed) {
-        int* d_fneed = reinterpret_cast<int*>(g->d_tot);
-        unsigned long long* d_wmax = reinterpret_cast<unsigned long long*>(g->d_tot + 1);
-        launch_weight_grid(g->d_w, g->ne, d_fneed, d_wmax, g->stream);
-        HIP_TRY(hipGetLastError());
-        int fneed = 0;
-        unsigned long long wbits = 0;
-        HIP_TRY(hipMemcpyAsync(&fneed, d_fneed, sizeof(fneed), hipMemcpyDeviceToHost, g->stream));
-        HIP_TRY(hipMemcpyAsync(&wbits, d_wmax, sizeof(wbits), hipMemcpyDeviceToHost, g->stream));
-        HIP_TRY(hipStreamSynchronize(g->stream));
-        const int F = std::max(fneed, 0);
-        const double wq_max = std::ldexp(nido_bitsd(wbits), F);   // exact: a power-of-two scaling
+        if (!g->grid_known) {
+            launch_weight_grid(g->d_w, g->ne, g->d_grid, g->stream);
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipMemcpyAsync(&g->grid, g->d_grid, sizeof(WeightGrid), hipMemcpyDeviceToHost, g->stream));
+            HIP_TRY(hipStreamSynchronize(g->stream));
+            g->grid_known = true;
+        }
+        const int fneed = g->grid.fneed, F = std::max(fneed, 0);
+        const double wq_max = std::ldexp(nido_bitsd(g->grid.wmax), F);   // exact: a power-of-two scaling
         const uint64_t dmax = (uint64_t)std::max<int64_t>(g->tuning.big_min_deg, kThreadMaxDeg);
         if (fneed <= 62 && wq_max < 0x1p62 &&
             (unsigned __int128)(uint64_t)wq_max * dmax < ((unsigned __int128)1 << 63)) {
@@ -1400,6 +1403,7 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         g->nv = K;
         g->ne = nne;
         g->h_off.swap(hoff);
+        g->grid_known = g->narrowed = false;
     } while (0);
 #undef COARSEN_HIP
     cleanup();
@@ -1436,6 +1440,7 @@ int coarsen_host(nido_graph* g, const int64_t* newid, int64_t K)
     g->nv = K;
     g->ne = nne;
     g->h_off.swap(noff);
+    g->grid_known = g->narrowed = false;
     return NIDO_OK;
 }
 
@@ -1883,17 +1888,21 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     bool nonneg = true;
     const int64_t whole[2] = {0, nv};
     const int64_t* gv = G > 1 ? vptr : whole;
-    // Inputs large enough for the pinned staging buffers are checked while
-    // they pass through them (ids and weights are read there anyway); the
-    // full host check runs first for smaller ones, and after the upload when
-    // the quick checks saw anything it has to decide exactly (a bad arc, a
-    // negative weight, a graph whose total of |w| nears the bound).
-    const bool fused = !(window > 0 && ne > window) && ne > 0 && staged_path(sizeof(double) * (size_t)ne);
-    if (fused) NIDO_TRY(check_offsets(nv, off, col, w));
-    else NIDO_TRY(check_csr(nv, off, col, w, G, gv, &nonneg, nullptr));
+    // Resident arcs are checked where they pass anyway: on their way through
+    // the pinned staging buffers when they are many, by the kernel that narrows
+    // the ids on the device otherwise.  The full host check runs first for a
+    // windowed graph, and afterwards when the quick ones saw anything it has to
+    // decide exactly (a bad arc, to name it; a negative weight; a total of |w|
+    // that may reach the bound).
+    const bool windowed0 = window > 0 && ne > window;
+    const bool fused = !windowed0 && ne > 0 && staged_path(sizeof(double) * (size_t)ne);
+    const bool on_device = !windowed0 && ne > 0 && !fused;
+    if (windowed0 || ne <= 0) NIDO_TRY(check_csr(nv, off, col, w, G, gv, &nonneg, nullptr));
+    else NIDO_TRY(check_offsets(nv, off, col, w));
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) {
         (void)hipGetLastError();
+        NIDO_TRY(check_csr(nv, off, col, w, G, gv, &nonneg, nullptr));
         return set_error(NIDO_ERR_HIP, "no HIP device available");
     }
     nido_graph* g = new nido_graph;
@@ -1929,7 +1938,6 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     // arcs than that) one window; the arcs of a windowed graph stay in
     // pinned host memory.
     g->window = window;
-    const bool windowed0 = window > 0 && ne > window;
     const int64_t cap = windowed0 ? window : ne;
     int rc;
     if (windowed0) {
@@ -1953,7 +1961,7 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
         (rc = dev_alloc(&g->d_col32, cap)) || (rc = dev_alloc(&g->d_C32, nv)) ||
         (rc = dev_alloc(&g->d_dcomms, nv)) || (rc = dev_alloc(&g->d_touched, nv)) ||
         (rc = dev_alloc(&g->d_term, nv)) || (rc = dev_alloc(&g->d_iacc, 2)) ||
-        (rc = dev_alloc(&g->d_part, 2 * (int64_t)kPartBlocks)))
+        (rc = dev_alloc(&g->d_part, 2 * (int64_t)kPartBlocks)) || (rc = dev_alloc(&g->d_grid, 1)))
         return fail(rc);
     if ((rc = raw_alloc(&g->d_scan_tmp, scan_temp_bytes(nv + 1)))) return fail(rc);
     if (hipHostMalloc(reinterpret_cast<void**>(&g->h_q), sizeof(double)) != hipSuccess)
@@ -1977,25 +1985,41 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     const bool local16 = fused && G > 1 && maxg <= 65536;
     if (staged_h2d(g->d_off, g->h_off.data(), sizeof(int64_t) * (size_t)(nv + 1), s) != hipSuccess ||
         (local16 && staged_h2d_local_ids(reinterpret_cast<uint16_t*>(g->d_col), col + base, ne, s, chk) != hipSuccess) ||
-        (ne > 0 && !windowed0 && !local16 &&
-         staged_h2d_ids(g->d_col32, col + base, ne, s, fused ? &chk : nullptr) != hipSuccess) ||
-        (ne > 0 && !windowed0 &&
-         (fused ? staged_h2d_weights(g->d_w, w + base, ne, s, chk)
-                : staged_h2d(g->d_w, w + base, sizeof(double) * (size_t)ne, s)) != hipSuccess))
+        (fused && !local16 && staged_h2d_ids(g->d_col32, col + base, ne, s, chk) != hipSuccess) ||
+        (fused && staged_h2d_weights(g->d_w, w + base, ne, s, chk) != hipSuccess) ||
+        (on_device && (staged_h2d(g->d_col, col + base, sizeof(int64_t) * (size_t)ne, s) != hipSuccess ||
+                       staged_h2d(g->d_w, w + base, sizeof(double) * (size_t)ne, s) != hipSuccess)))
         return fail(set_error(NIDO_ERR_HIP, "upload failed"));
     if (fused) {
         bool exact = chk.bad.load() != INT64_MAX || chk.neg.load();
         for (double x : chk.wabs) exact |= !(x <= 0x1p61);   // FP64 sums: far from 2^62 below this
         if (exact && (rc = check_csr(nv, off, col, w, G, gv, &nonneg, nullptr))) return fail(rc);
     }
+    // the arcs graph by graph in pieces, for many graphs in one handle
+    std::vector<ArcPiece> pieces;
+    if (local16 || (on_device && G > 1))
+        for (int i = 0; i < G; ++i)
+            for (int64_t e = gstart[(size_t)i]; e < gstart[(size_t)i + 1]; e += kPieceArcs)
+                pieces.push_back(ArcPiece{e, std::min(gstart[(size_t)i + 1], e + kPieceArcs), gv[i], gv[i + 1] - gv[i]});
+    if (on_device) {
+        ArcPiece* d_pieces = nullptr;
+        if (G > 1 && (rc = upload(&d_pieces, pieces, s))) return fail(rc);
+        launch_take_arcs(d_pieces, G > 1 ? (int64_t)pieces.size() : (ne + kPieceArcs - 1) / kPieceArcs, ne, nv, g->d_col,
+                         g->d_w, g->d_col32, g->d_grid, s);
+        const bool ok = hipGetLastError() == hipSuccess &&
+                        hipMemcpyAsync(&g->grid, g->d_grid, sizeof(WeightGrid), hipMemcpyDeviceToHost, s) == hipSuccess &&
+                        hipStreamSynchronize(s) == hipSuccess;
+        dev_free(d_pieces);
+        if (!ok) return fail(set_error(NIDO_ERR_HIP, "checking the uploaded arcs failed"));
+        // (the bits of a NaN order above those of infinity)
+        const bool exact = g->grid.flags != 0 || g->grid.wmax > nido_dbits(0x1p61) ||
+                           nido_bitsd(g->grid.wmax) * (double)ne > 0x1p61;
+        if (exact && (rc = check_csr(nv, off, col, w, G, gv, &nonneg, nullptr))) return fail(rc);
+        g->grid_known = g->narrowed = true;
+    }
     g->nonneg = nonneg;
     if (local16) {
-        // graph-local ids back to handle ids, graph by graph in pieces of at
-        // most 2^16 arcs
-        std::vector<ArcPiece> pieces;
-        for (int i = 0; i < G; ++i)
-            for (int64_t e = gstart[(size_t)i]; e < gstart[(size_t)i + 1]; e += 65536)
-                pieces.push_back(ArcPiece{e, std::min(gstart[(size_t)i + 1], e + 65536), gv[i]});
+        // graph-local ids back to handle ids
         ArcPiece* d_pieces = nullptr;
         if ((rc = dev_alloc(&d_pieces, std::max<int64_t>((int64_t)pieces.size(), 1)))) return fail(rc);
         const bool ok = pieces.empty() ||
@@ -2010,7 +2034,10 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     }
     // ids crossed the host link as int32 or 16-bit local ids (all below
     // nv < 2^31 - 1, checked); the int64 copy overwrites the local ids
-    if (!windowed0) launch_widen_ids(g->d_col32, g->d_col, ne, s);
+    if (fused) {
+        launch_widen_ids(g->d_col32, g->d_col, ne, s);
+        g->narrowed = true;
+    }
     if (G > 1) {
         g->G = G;
         g->vb.assign(vptr, vptr + G + 1);
@@ -2174,6 +2201,7 @@ int nido_graph_destroy(nido_graph* g)
     dev_free(g->d_C); dev_free(g->d_Cn); dev_free(g->d_k); dev_free(g->d_a); dev_free(g->d_kd);
     dev_free(g->d_clus); dev_free(g->d_work); dev_free(g->d_acc); dev_free(g->d_q); dev_free(g->d_tot);
     dev_free(g->d_src); dev_free(g->d_part); dev_free(g->d_col32); dev_free(g->d_C32); dev_free(g->d_wq);
+    dev_free(g->d_grid);
     dev_free(g->d_gid); dev_free(g->d_gid0); dev_free(g->d_vb); dev_free(g->d_vbn); dev_free(g->d_mg);
     dev_free(g->d_twomg); dev_free(g->d_act); dev_free(g->d_keep); dev_free(g->d_gacc); dev_free(g->d_gq);
     dev_free(g->d_moved);

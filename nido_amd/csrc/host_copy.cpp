@@ -208,6 +208,28 @@ void weights_checked(double* b, const double* src, int64_t at, int64_t m, ArcChe
         });
     }
 }
+
+// n ids through two pinned buffers of kChunk ids each, narrowed into them by
+// fill(buffer, src, first, count).
+template <typename Fill>
+hipError_t ids_in_chunks(int* dst, const int64_t* src, int64_t n, hipStream_t s, int64_t kChunk, Fill&& fill)
+{
+    Staging st(sizeof(int) * (size_t)kChunk);
+    hipError_t e = st.status();
+    int* const buf[2] = {reinterpret_cast<int*>(st.buf(0)), reinterpret_cast<int*>(st.buf(1))};
+    const hipEvent_t done[2] = {st.done(0), st.done(1)};
+    for (int64_t at = 0, i = 0; e == hipSuccess && at < n; at += kChunk, i ^= 1) {
+        const int64_t m = std::min(kChunk, n - at);
+        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
+        if (e != hipSuccess) break;
+        fill(buf[i], src, at, m);
+        e = hipMemcpyAsync(dst + at, buf[i], sizeof(int) * (size_t)m, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess) e = hipEventRecord(done[i], s);
+    }
+    const hipError_t w = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = w;
+    return st.finish(e);
+}
 }  // namespace
 
 bool staged_path(size_t bytes)
@@ -285,44 +307,28 @@ hipError_t staged_d2h(void* dst, const void* src, size_t bytes, hipStream_t s)
     return st.finish(e);
 }
 
-hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s, ArcCheck* chk)
+hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s)
 {
     const int64_t kChunk = g_chunk_bytes.load() / (int64_t)sizeof(int);   // ids per pinned buffer
     if (n * (int64_t)sizeof(int) < g_min_bytes.load()) {   // one pageable copy, no pinned allocation
         std::vector<int> t((size_t)n);
-        if (chk) {
-            narrow_checked(t.data(), src, 0, n, *chk);
-        } else {
-            // threads only for graphs larger than a serving request, whose
-            // requests already run side by side
 #pragma omp parallel for schedule(static) if (n >= (int64_t(1) << 26))
-            for (int64_t j = 0; j < n; ++j) t[(size_t)j] = (int)src[j];
-        }
+        for (int64_t j = 0; j < n; ++j) t[(size_t)j] = (int)src[j];
         hipError_t e = hipMemcpyAsync(dst, t.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }
-    Staging st(sizeof(int) * (size_t)kChunk);
-    hipError_t e = st.status();
-    int* const buf[2] = {reinterpret_cast<int*>(st.buf(0)), reinterpret_cast<int*>(st.buf(1))};
-    const hipEvent_t done[2] = {st.done(0), st.done(1)};
-    for (int64_t at = 0, i = 0; e == hipSuccess && at < n; at += kChunk, i ^= 1) {
-        const int64_t m = std::min(kChunk, n - at);
-        if (at >= 2 * kChunk) e = hipEventSynchronize(done[i]);   // this call's copy from the buffer has landed
-        if (e != hipSuccess) break;
-        int* b = buf[i];
-        const int64_t* in = src + at;
-        if (chk) {
-            narrow_checked(b, src, at, m, *chk);
-        } else {
+    return ids_in_chunks(dst, src, n, s, kChunk, [](int* b, const int64_t* in, int64_t at, int64_t m) {
 #pragma omp parallel for schedule(static) if (m >= (int64_t(1) << 20))
-            for (int64_t j = 0; j < m; ++j) b[j] = (int)in[j];
-        }
-        e = hipMemcpyAsync(dst + at, b, sizeof(int) * (size_t)m, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = hipEventRecord(done[i], s);
-    }
-    const hipError_t w = hipStreamSynchronize(s);
-    if (e == hipSuccess) e = w;
-    return st.finish(e);
+        for (int64_t j = 0; j < m; ++j) b[j] = (int)in[at + j];
+    });
+}
+
+hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s, ArcCheck& chk)
+{
+    const int64_t kChunk = g_chunk_bytes.load() / (int64_t)sizeof(int);
+    return ids_in_chunks(dst, src, n, s, kChunk, [&](int* b, const int64_t* in, int64_t at, int64_t m) {
+        narrow_checked(b, in, at, m, chk);
+    });
 }
 
 hipError_t staged_h2d_local_ids(uint16_t* dst, const int64_t* src, int64_t n, hipStream_t s, ArcCheck& chk)

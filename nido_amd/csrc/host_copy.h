@@ -46,7 +46,9 @@ hipError_t staged_d2h(void* dst, const void* src, size_t bytes, hipStream_t s);
 // The same for n ids below 2^31 stored as int64 on the host, sent as int32
 // (narrowed while staging): half the bytes over the host link.  Pinned
 // staging from the same byte threshold as staged_h2d (2^26 ids by default).
-hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s, ArcCheck* chk = nullptr);
+hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s);
+// Always through the staging buffers, checked by chk on the way.
+hipError_t staged_h2d_ids(int* dst, const int64_t* src, int64_t n, hipStream_t s, ArcCheck& chk);
 
 // The ids of a handle whose graphs all have at most 2^16 vertices, sent as
 // 16-bit ids local to their graph (a quarter of the int64 bytes; the device

@@ -210,10 +210,30 @@ void launch_vertex_weights(const int64_t* off, const double* w, const int* small
 void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s);
 void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k, int64_t nv,
                       hipStream_t s);
-// *fneed = the fractional bits the finest weight needs (max over nonzero
-// weights; 2000 for a subnormal or non-finite one, INT_MIN when every weight
-// is 0), *wmax = the bits of max |w|.
-void launch_weight_grid(const double* w, int64_t ne, int* fneed, unsigned long long* wmax, hipStream_t s);
+// What a pass over the weights finds: the bits of max |w| (|x| bit patterns
+// order like the values), the fractional bits the finest nonzero one needs
+// (2000 for a subnormal or non-finite weight, INT_MIN when every weight is 0),
+// and flags.
+struct WeightGrid {
+    unsigned long long wmax;
+    int fneed;
+    int flags;
+};
+constexpr unsigned kArcOutside = 1;        // a column outside its graph
+constexpr unsigned kArcNegative = 2;       // a weight below zero
+void launch_weight_grid(const double* w, int64_t ne, WeightGrid* G, hipStream_t s);
+// Arcs [e0, e1) belong to the graph of nv vertices whose first one is base.
+struct ArcPiece {
+    int64_t e0, e1;
+    int64_t base, nv;
+};
+// Arcs of a piece at most.  The workgroup of a piece passes over it 256 arcs at
+// a time: 4,096 give a graph of a million arcs a workgroup per CU.
+constexpr int64_t kPieceArcs = 4096;
+// The checks and the narrowing of ne uploaded arcs; n pieces, or with a null
+// list ceil(ne / kPieceArcs) of them, of one graph of nv vertices.
+void launch_take_arcs(const ArcPiece* pieces, int64_t n, int64_t ne, int64_t nv, const int64_t* col, const double* w,
+                      int* col32, WeightGrid* G, hipStream_t s);
 // wq[e] = w[e] * scale, exact for weights on the 1/scale grid.
 void launch_to_fixed(const double* w, int64_t* wq, int64_t ne, double scale, hipStream_t s);
 // col32[e] = (int)col[e]
@@ -322,11 +342,6 @@ void launch_mark_communities(const int64_t* C, int64_t nv, int64_t* flag, hipStr
                              const int* gid = nullptr, const unsigned char* keep = nullptr);
 void launch_update_clustering(int64_t* clus, int64_t n0, const int64_t* C, const int64_t* newid,
                               hipStream_t s, const int* gid0 = nullptr, const unsigned char* keep = nullptr);
-// Arcs [e0, e1) belong to a graph whose first vertex is base.
-struct ArcPiece {
-    int64_t e0, e1;
-    int64_t base;
-};
 // col32[e] = base + local[e] over the pieces: ids that crossed the host link
 // as 16-bit graph-local ids.
 void launch_widen_local(const ArcPiece* pieces, int64_t n, const uint16_t* local, int* col32, hipStream_t s);
