@@ -124,6 +124,60 @@ void dev_free(T*& p)
     p = nullptr;
 }
 
+// Device scratch handed out in pieces and taken back all at once, for work
+// that follows on one stream: what an earlier call put there has been read by
+// the time a later call's kernels write.  Up to kArenaKeep bytes stay with the
+// handle between calls (a phase of a small graph made 20 allocations and frees
+// of 4 to 12 us each); larger blocks go back to the pool, where other handles
+// find them.
+constexpr size_t kArenaKeep = size_t(64) << 20;
+struct Arena {
+    struct Block {
+        char* p;
+        size_t bytes, used;
+    };
+    std::vector<Block> blocks;
+    template <typename T>
+    int get(T** out, int64_t count)
+    {
+        const size_t need = (sizeof(T) * (size_t)(count > 0 ? count : 1) + 255) & ~size_t(255);
+        for (Block& b : blocks)
+            if (b.bytes - b.used >= need) {
+                *out = reinterpret_cast<T*>(b.p + b.used);
+                b.used += need;
+                return NIDO_OK;
+            }
+        void* p = nullptr;
+        const size_t bytes = std::max(need, size_t(1) << 20);
+        blocks.reserve(blocks.size() + 1);
+        const int rc = raw_alloc(&p, bytes);
+        if (rc != NIDO_OK) return rc;
+        blocks.push_back(Block{static_cast<char*>(p), bytes, need});
+        *out = static_cast<T*>(p);
+        return NIDO_OK;
+    }
+    void reset(size_t keep = kArenaKeep)
+    {
+        size_t kept = 0, n = 0;
+        for (Block& b : blocks) {
+            if (kept + b.bytes <= keep) {
+                kept += b.bytes;
+                b.used = 0;
+                blocks[n++] = b;
+            } else {
+                raw_free(b.p);
+            }
+        }
+        blocks.resize(n);
+    }
+};
+// Takes back what a scope got, also where it leaves with an error.
+struct ArenaScope {
+    Arena& a;
+    explicit ArenaScope(Arena& x) : a(x) { a.reset(); }
+    ~ArenaScope() { a.reset(); }
+};
+
 struct PhaseHist {
     nido_phase_stats st{};
     std::vector<double> iter_q;
@@ -263,20 +317,24 @@ struct nido_graph {
     int64_t wq_cap = 0;
     bool fixed = false;            // this phase's short rows sum in 64-bit fixed point (d_wq)
     double wscale = 1.0;           // 2^-F
-    WeightGrid* d_grid = nullptr;
-    WeightGrid grid{};             // of the current weights, once grid_known
-    bool grid_known = false;
-    bool narrowed = false;         // d_col32 mirrors the current d_col
+    PhaseOut* d_out = nullptr;
     fx_t* d_part = nullptr;        // 2 * kPartBlocks reduction partials
     void* d_scan_tmp = nullptr;
     // scalars
     fx_t* d_acc = nullptr;         // [0] internal weight, [1] sum of squares, [2] 2m
     double* d_q = nullptr;
     int64_t* d_tot = nullptr;      // [2] scan totals
-    double* h_q = nullptr;         // pinned
+    // Pinned memory for small copies in both directions (send, fetch): a
+    // pageable copy of 64 KiB to 1 MiB takes 35 to 430 us, one through here 10
+    // to 70.  pin_used bytes of it belong to copies the stream may not have
+    // made yet.
+    PinnedBlock pin;
+    size_t pin_used = 0;
+    Arena ws;                      // scratch of one call at a time, kept between calls
     // local-moving bins: per batch, the fused small-row launch and the
     // partitioned long-row launch
     BinRow* d_binv = nullptr;
+    int64_t binv_cap = 0, items_cap = 0, chunks_cap = 0, poff_cap = 0, toff_cap = 0, seg_cap = 0;
     std::vector<SmallBins> small_bins;   // nb
     std::vector<BigArgs> big_args;       // nb
     BigItem* d_big_items = nullptr;
@@ -297,12 +355,6 @@ struct nido_graph {
     int* d_tkey = nullptr;
     fx_t* d_tval = nullptr;
     int64_t tab_cap = 0;
-    // degree / modularity work lists
-    int* d_small = nullptr;
-    int64_t nsmall = 0;
-    RowItem* d_items = nullptr;
-    int64_t nitems = 0;
-
     fx_t twom = 0;
     double twom_d = 0, m = 0;
     bool nonneg = true;            // every weight >= 0 (coarse weights are sums of these)
@@ -427,13 +479,83 @@ void batch_bounds(const std::vector<int64_t>& off, int64_t nv, int nb, std::vect
 }
 
 
-template <typename T>
-int upload(T** d, const std::vector<T>& h, hipStream_t s)
+constexpr size_t kPinBytes = size_t(4) << 20;   // of a handle's pinned block
+constexpr size_t kPinScalars = 4096;             // its first bytes: single results
+
+// The second stream and its events, made by the first iteration that uses them
+// (a replayed one, or one that streams its arcs): with the stream's end they
+// took 0.1 to 0.3 ms of every handle.
+int need_side(nido_graph* g)
 {
-    dev_free(*d);
-    NIDO_TRY(dev_alloc(d, (int64_t)h.size()));
-    if (!h.empty()) HIP_TRY(staged_h2d(*d, h.data(), sizeof(T) * h.size(), s));
+    if (g->side) return NIDO_OK;
+    for (hipEvent_t* e : {&g->ev_fork, &g->ev_join, &g->ev_copied[0], &g->ev_copied[1], &g->ev_free[0], &g->ev_free[1]})
+        if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    HIP_TRY(hipStreamCreateWithFlags(&g->side, hipStreamNonBlocking));
     return NIDO_OK;
+}
+
+// Waits for the handle's stream.
+int wait_stream(nido_graph* g)
+{
+    HIP_TRY(hipStreamSynchronize(g->stream));
+    g->pin_used = 0;
+    return NIDO_OK;
+}
+
+// `bytes` of host memory to the device in stream order; src is free at once.
+int send(nido_graph* g, void* dst, const void* src, size_t bytes)
+{
+    if (bytes == 0) return NIDO_OK;
+    if (bytes > kPinBytes - kPinScalars) {
+        HIP_TRY(staged_h2d(dst, src, bytes, g->stream));
+        g->pin_used = 0;                            // it waits for the stream
+        return NIDO_OK;
+    }
+    if (g->pin_used + bytes > kPinBytes - kPinScalars) NIDO_TRY(wait_stream(g));
+    char* p = g->pin.p + kPinScalars + g->pin_used;
+    std::memcpy(p, src, bytes);
+    HIP_TRY(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, g->stream));
+    g->pin_used += (bytes + 63) & ~size_t(63);
+    return NIDO_OK;
+}
+
+// `bytes` of device memory to the host, once the stream gets there.
+int fetch(nido_graph* g, void* dst, const void* src, size_t bytes)
+{
+    if (bytes == 0) return wait_stream(g);
+    if (bytes > kPinBytes - kPinScalars) {
+        HIP_TRY(staged_d2h(dst, src, bytes, g->stream));
+        g->pin_used = 0;
+        return NIDO_OK;
+    }
+    char* p = g->pin.p;
+    if (bytes > kPinScalars) {
+        if (g->pin_used + bytes > kPinBytes - kPinScalars) NIDO_TRY(wait_stream(g));
+        p += kPinScalars + g->pin_used;
+    }
+    HIP_TRY(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, g->stream));
+    NIDO_TRY(wait_stream(g));
+    std::memcpy(dst, p, bytes);
+    return NIDO_OK;
+}
+
+// Device array *d of room for n values: the one there if it is large enough.
+template <typename T>
+int reserve(T** d, int64_t* cap, int64_t n)
+{
+    if (*d && n <= *cap) return NIDO_OK;
+    dev_free(*d);
+    *cap = 0;
+    NIDO_TRY(dev_alloc(d, n));
+    *cap = std::max<int64_t>(n, 1);
+    return NIDO_OK;
+}
+
+template <typename T>
+int upload(nido_graph* g, T** d, int64_t* cap, const std::vector<T>& h)
+{
+    NIDO_TRY(reserve(d, cap, (int64_t)h.size()));
+    return send(g, *d, h.data(), sizeof(T) * h.size());
 }
 
 void drop_iteration_graph(nido_graph* g);
@@ -464,56 +586,33 @@ int device_bins(nido_graph* g, PhaseBins& pb, const unsigned char* keep)
     std::vector<int64_t> tb0;
     bin_tiles(nb, G, g->parts, g->gparts, keep, tiles, tb0);
     const int64_t T = (int64_t)tiles.size(), nc = NUM_BINS * T;
+    ArenaScope scope(g->ws);
     BinTile* d_tiles = nullptr;
-    int64_t *d_tb0 = nullptr, *d_cnt = nullptr, *d_starts = nullptr, *d_total = nullptr;
-    void* tmp = nullptr;
-    auto cleanup = [&]() {
-        dev_free(d_tiles); dev_free(d_tb0); dev_free(d_cnt); dev_free(d_starts); dev_free(d_total);
-        raw_free(tmp);
-        tmp = nullptr;
-    };
-    std::vector<int64_t> starts((size_t)nb * NUM_BINS, -1);
+    int64_t *d_tb0 = nullptr, *d_cnt = nullptr, *d_starts = nullptr;
+    char* tmp = nullptr;
+    // the first position of every (batch, bin), then the rows in all
+    std::vector<int64_t> starts((size_t)nb * NUM_BINS + 1, -1);
     int64_t rows = 0;
-    int rc = NIDO_OK;
-    do {
-        if ((rc = dev_alloc(&d_tiles, std::max<int64_t>(T, 1))) || (rc = dev_alloc(&d_tb0, (int64_t)nb + 1)) ||
-            (rc = dev_alloc(&d_cnt, std::max<int64_t>(nc, 1))) ||
-            (rc = dev_alloc(&d_starts, std::max<int64_t>((int64_t)nb * NUM_BINS, 1))) ||
-            (rc = dev_alloc(&d_total, 1)) || (rc = raw_alloc(&tmp, scan_temp_bytes(std::max<int64_t>(nc, 1)))))
-            break;
-        if (T > 0 && (hipMemcpyAsync(d_tiles, tiles.data(), sizeof(BinTile) * (size_t)T, hipMemcpyHostToDevice,
-                                     s) != hipSuccess ||
-                      hipMemcpyAsync(d_tb0, tb0.data(), sizeof(int64_t) * tb0.size(), hipMemcpyHostToDevice,
-                                     s) != hipSuccess)) {
-            rc = set_error(NIDO_ERR_HIP, "bin tile upload failed");
-            break;
-        }
-        if (T > 0) {
-            launch_bin_count(d_tiles, T, g->d_off, g->tuning.thread_max_deg, g->tuning.big_min_deg, d_cnt, s);
-            launch_exclusive_scan(d_cnt, d_cnt, nc, d_total, tmp, s);
-            if (hipMemcpyAsync(&rows, d_total, sizeof(int64_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess) {
-                rc = set_error(NIDO_ERR_HIP, "bin count failed");
-                break;
-            }
-        }
-        dev_free(g->d_binv);
-        if ((rc = dev_alloc(&g->d_binv, std::max<int64_t>(rows, 1)))) break;
-        if (T > 0) {
-            launch_bin_scatter(d_tiles, T, g->d_off, g->tuning.thread_max_deg, g->tuning.big_min_deg, d_cnt,
-                               g->d_binv, s);
-            launch_bin_starts(d_cnt, d_tb0, nb, d_starts, s);
-            if (hipGetLastError() != hipSuccess ||
-                hipMemcpyAsync(starts.data(), d_starts, sizeof(int64_t) * starts.size(), hipMemcpyDeviceToHost,
-                               s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess) {
-                rc = set_error(NIDO_ERR_HIP, "bin scatter failed");
-                break;
-            }
-        }
-    } while (false);
-    cleanup();
-    if (rc != NIDO_OK) return rc;
+    NIDO_TRY(g->ws.get(&d_tiles, T));
+    NIDO_TRY(g->ws.get(&d_tb0, (int64_t)nb + 1));
+    NIDO_TRY(g->ws.get(&d_cnt, nc));
+    NIDO_TRY(g->ws.get(&d_starts, (int64_t)starts.size()));
+    NIDO_TRY(g->ws.get(&tmp, (int64_t)scan_temp_bytes(std::max<int64_t>(nc, 1))));
+    if (T > 0) {
+        NIDO_TRY(send(g, d_tiles, tiles.data(), sizeof(BinTile) * (size_t)T));
+        NIDO_TRY(send(g, d_tb0, tb0.data(), sizeof(int64_t) * tb0.size()));
+        launch_bin_count(d_tiles, T, g->d_off, g->tuning.thread_max_deg, g->tuning.big_min_deg, d_cnt, s);
+        launch_exclusive_scan(d_cnt, d_cnt, nc, d_starts + nb * NUM_BINS, tmp, s);
+        launch_bin_starts(d_cnt, d_tb0, nb, d_starts, s);
+        // every row lands in a bin, or has no arcs: nv bounds the rows
+        NIDO_TRY(reserve(&g->d_binv, &g->binv_cap, g->nv));
+        launch_bin_scatter(d_tiles, T, g->d_off, g->tuning.thread_max_deg, g->tuning.big_min_deg, d_cnt, g->d_binv, s);
+        HIP_TRY(hipGetLastError());
+        NIDO_TRY(fetch(g, starts.data(), d_starts, sizeof(int64_t) * starts.size()));
+        rows = starts.back();
+    } else {
+        NIDO_TRY(reserve(&g->d_binv, &g->binv_cap, 1));
+    }
     // a batch without tiles starts where the next one does
     int64_t next = rows;
     for (int b = nb - 1; b >= 0; --b) {
@@ -526,12 +625,11 @@ int device_bins(nido_graph* g, PhaseBins& pb, const unsigned char* keep)
     std::vector<int64_t> cnt((size_t)nb * NUM_BINS), bverts((size_t)nb, 0), barcs((size_t)nb, 0);
     for (size_t i = 0; i < cnt.size(); ++i) cnt[i] = (i + 1 < cnt.size() ? starts[i + 1] : rows) - starts[i];
     std::vector<std::vector<BinRow>> big((size_t)nb);
+    int64_t nbig = 0;
     for (int b = 0; b < nb; ++b) {
         const int64_t n = cnt[(size_t)b * NUM_BINS + BIN_BIG];
         big[(size_t)b].resize((size_t)n);
-        if (n > 0)
-            HIP_TRY(hipMemcpyAsync(big[(size_t)b].data(), g->d_binv + starts[(size_t)b * NUM_BINS + BIN_BIG],
-                                   sizeof(BinRow) * (size_t)n, hipMemcpyDeviceToHost, s));
+        nbig += n;
         auto range = [&](int64_t v0, int64_t v1) {
             bverts[(size_t)b] += v1 - v0;
             barcs[(size_t)b] += off[(size_t)v1] - off[(size_t)v0];
@@ -542,52 +640,31 @@ int device_bins(nido_graph* g, PhaseBins& pb, const unsigned char* keep)
                 if (!keep || keep[i])
                     range(g->gparts[(size_t)i * (nb + 1) + b], g->gparts[(size_t)i * (nb + 1) + b + 1]);
     }
-    HIP_TRY(hipStreamSynchronize(s));
+    // the long rows of every batch: into the pinned block and one wait, or
+    // batch by batch when they do not fit it
+    if (sizeof(BinRow) * (size_t)nbig <= kPinBytes - kPinScalars && nbig > 0) {
+        NIDO_TRY(wait_stream(g));
+        BinRow* p = reinterpret_cast<BinRow*>(g->pin.p + kPinScalars);
+        for (int b = 0; b < nb; ++b) {
+            const size_t n = big[(size_t)b].size();
+            if (n) HIP_TRY(hipMemcpyAsync(p, g->d_binv + starts[(size_t)b * NUM_BINS + BIN_BIG], sizeof(BinRow) * n,
+                                          hipMemcpyDeviceToHost, s));
+            p += n;
+        }
+        NIDO_TRY(wait_stream(g));
+        p = reinterpret_cast<BinRow*>(g->pin.p + kPinScalars);
+        for (int b = 0; b < nb; ++b) {
+            std::copy(p, p + big[(size_t)b].size(), big[(size_t)b].begin());
+            p += big[(size_t)b].size();
+        }
+    } else {
+        for (int b = 0; b < nb; ++b)
+            if (!big[(size_t)b].empty())
+                NIDO_TRY(fetch(g, big[(size_t)b].data(), g->d_binv + starts[(size_t)b * NUM_BINS + BIN_BIG],
+                               sizeof(BinRow) * big[(size_t)b].size()));
+    }
     build_phase_lists(off.data(), nb, cnt, big, bverts, barcs, g->tuning, pb);
     return NIDO_OK;
-}
-
-// The row lists of the degree and modularity sweeps built on the device.
-int device_row_lists(nido_graph* g)
-{
-    const int64_t nv = g->nv, nt = (nv + kBinTileVerts - 1) / kBinTileVerts;
-    hipStream_t s = g->stream;
-    int64_t *cs = nullptr, *ci = nullptr, *tot = nullptr;
-    void* tmp = nullptr;
-    auto cleanup = [&]() {
-        dev_free(cs); dev_free(ci); dev_free(tot);
-        raw_free(tmp);
-        tmp = nullptr;
-    };
-    int64_t h_tot[2] = {0, 0};
-    int rc = NIDO_OK;
-    do {
-        if ((rc = dev_alloc(&cs, std::max<int64_t>(nt, 1))) || (rc = dev_alloc(&ci, std::max<int64_t>(nt, 1))) ||
-            (rc = dev_alloc(&tot, 2)) || (rc = raw_alloc(&tmp, scan_temp_bytes(std::max<int64_t>(nt, 1)))))
-            break;
-        if (nt > 0) {
-            launch_rowlist_count(g->d_off, nv, cs, ci, s);
-            launch_exclusive_scan(cs, cs, nt, tot, tmp, s);
-            launch_exclusive_scan(ci, ci, nt, tot + 1, tmp, s);
-            if (hipMemcpyAsync(h_tot, tot, sizeof(h_tot), hipMemcpyDeviceToHost, s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess) {
-                rc = set_error(NIDO_ERR_HIP, "row list count failed");
-                break;
-            }
-        }
-        dev_free(g->d_small);
-        dev_free(g->d_items);
-        if ((rc = dev_alloc(&g->d_small, std::max<int64_t>(h_tot[0], 1))) ||
-            (rc = dev_alloc(&g->d_items, std::max<int64_t>(h_tot[1], 1))))
-            break;
-        if (nt > 0) launch_rowlist_scatter(g->d_off, nv, cs, ci, g->d_small, g->d_items, s);
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-            rc = set_error(NIDO_ERR_HIP, "row list scatter failed");
-    } while (false);
-    cleanup();
-    g->nsmall = h_tot[0];
-    g->nitems = h_tot[1];
-    return rc;
 }
 
 // The work lists of the phase's launches (degree bins, long-row items,
@@ -625,9 +702,9 @@ int build_lists(nido_graph* g, const unsigned char* keep)
     g->long_bytes = pb.long_bytes;
     g->blist0 = pb.blist0;
     g->blistn = pb.blistn;
-    if (!dev_lists) NIDO_TRY(upload(&g->d_binv, binv, g->stream));
-    NIDO_TRY(upload(&g->d_big_items, bitems, g->stream));
-    NIDO_TRY(upload(&g->d_key_chunks, chunks, g->stream));
+    if (!dev_lists) NIDO_TRY(upload(g, &g->d_binv, &g->binv_cap, binv));
+    NIDO_TRY(upload(g, &g->d_big_items, &g->items_cap, bitems));
+    NIDO_TRY(upload(g, &g->d_key_chunks, &g->chunks_cap, chunks));
     if (key_need > g->key_cap) {
         dev_free(g->d_bkey);
         dev_free(g->d_bw);
@@ -640,8 +717,8 @@ int build_lists(nido_graph* g, const unsigned char* keep)
         NIDO_TRY(dev_alloc(&g->d_cpo, cpo_need));
         g->cpo_cap = cpo_need;
     }
-    NIDO_TRY(upload(&g->d_big_poff, poff, g->stream));
-    NIDO_TRY(upload(&g->d_big_toff, toff, g->stream));
+    NIDO_TRY(upload(g, &g->d_big_poff, &g->poff_cap, poff));
+    NIDO_TRY(upload(g, &g->d_big_toff, &g->toff_cap, toff));
     if (tab_need > g->tab_cap) {
         dev_free(g->d_tkey);
         dev_free(g->d_tval);
@@ -749,7 +826,6 @@ int setup_phase(nido_graph* g)
     g->win_double = g->win_single;
     for (int b = 0; g->win_double && b < g->nb; ++b)
         g->win_double = 2 * (off[(size_t)g->parts[(size_t)b + 1]] - off[(size_t)g->parts[(size_t)b]]) <= g->window;
-    const bool dev_lists = !g->windowed && nv >= g_device_lists_min.load();
     if (!g->windowed || g->win_single) {
         // incremental modularity: room for every row chunk of the largest batch
         int64_t need = 0;
@@ -778,25 +854,28 @@ int setup_phase(nido_graph* g)
                 NIDO_TRY(dev_alloc(&g->d_gp, (int64_t)g->gparts.size()));
                 g->gp_cap = (int64_t)g->gparts.size();
             }
-            HIP_TRY(hipMemcpyAsync(g->d_gp, g->gparts.data(), sizeof(int64_t) * g->gparts.size(),
-                                   hipMemcpyHostToDevice, g->stream));
+            NIDO_TRY(send(g, g->d_gp, g->gparts.data(), sizeof(int64_t) * g->gparts.size()));
         }
         if (need > g->dchunk_cap) {
             dev_free(g->d_dchunks);
             NIDO_TRY(dev_alloc(&g->d_dchunks, need));
             g->dchunk_cap = need;
         }
-        dev_free(g->d_dcounts);
-        NIDO_TRY(dev_alloc(&g->d_dcounts, 2 * (int64_t)g->nb));
+        if (!g->d_dcounts) NIDO_TRY(dev_alloc(&g->d_dcounts, 2 * (int64_t)g->nb));
         launch_fill_i32(g->d_dcounts, 0, 2 * (int64_t)g->nb, g->stream);
-        launch_fill_i32(g->d_touched, 0, g->n0, g->stream);
-        HIP_TRY(hipStreamSynchronize(g->stream));
+        launch_fill_i32(g->d_touched, 0, g->nv, g->stream);
+    }
+    // the device sums the rows while the host builds the lists
+    if (!g->windowed) {
+        launch_vertex_weights(g->d_off, g->d_w, g->ne, g->d_k, g->d_kd, nv, g->d_out, g->d_part, g->d_src, g->stream);
+        HIP_TRY(hipGetLastError());
     }
     // after the delta buffers above: the short-row launches keep their
     // addresses (g->delta())
     NIDO_TRY(build_lists(g, nullptr));
     fx_t twom = 0;
     unsigned long long maxk_bits = 0;
+    PhaseOut out{};
     if (g->windowed) {
         // the arcs are on the host: k_v, 2m and max |k_v| from there
         std::vector<fx_t> hk((size_t)nv);
@@ -811,27 +890,9 @@ int setup_phase(nido_graph* g)
         }
         HIP_TRY(hipStreamSynchronize(g->stream));   // hk / hkd go out of scope
     } else {
-        if (dev_lists) {
-            NIDO_TRY(device_row_lists(g));
-        } else {
-            std::vector<int> small;
-            std::vector<RowItem> items;
-            build_row_lists(off.data(), nv, small, items);
-            g->nsmall = (int64_t)small.size();
-            g->nitems = (int64_t)items.size();
-            NIDO_TRY(upload(&g->d_small, small, g->stream));
-            NIDO_TRY(upload(&g->d_items, items, g->stream));
-        }
-
-        if (!g->narrowed) launch_narrow_ids(g->d_col, g->d_col32, g->ne, g->stream);
-        g->narrowed = true;
-        unsigned long long* d_maxk = reinterpret_cast<unsigned long long*>(g->d_tot + 1);
-        launch_vertex_weights(g->d_off, g->d_w, g->d_small, g->nsmall, g->d_items, g->nitems, g->d_k,
-                              g->d_kd, nv, g->d_acc + 2, d_maxk, g->d_part, g->d_src, g->stream);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(&twom, g->d_acc + 2, sizeof(fx_t), hipMemcpyDeviceToHost, g->stream));
-        HIP_TRY(hipMemcpyAsync(&maxk_bits, d_maxk, sizeof(maxk_bits), hipMemcpyDeviceToHost, g->stream));
-        HIP_TRY(hipStreamSynchronize(g->stream));
+        NIDO_TRY(fetch(g, &out, g->d_out, sizeof(out)));
+        twom = out.twom;
+        maxk_bits = out.maxk;
     }
     g->twom = twom;
     g->twom_d = fx_to_double(twom);
@@ -849,15 +910,8 @@ int setup_phase(nido_graph* g)
     // (scaled by 2^(64 - F)), one word and no carry per LDS update.
     g->fixed = false;
     if (g->tuning.fixed_short && g->ne > 0 && g->twom != 0 && !g->windowed) {
-        if (!g->grid_known) {
-            launch_weight_grid(g->d_w, g->ne, g->d_grid, g->stream);
-            HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(&g->grid, g->d_grid, sizeof(WeightGrid), hipMemcpyDeviceToHost, g->stream));
-            HIP_TRY(hipStreamSynchronize(g->stream));
-            g->grid_known = true;
-        }
-        const int fneed = g->grid.fneed, F = std::max(fneed, 0);
-        const double wq_max = std::ldexp(nido_bitsd(g->grid.wmax), F);   // exact: a power-of-two scaling
+        const int fneed = out.grid.fneed, F = std::max(fneed, 0);
+        const double wq_max = std::ldexp(nido_bitsd(out.grid.wmax), F);   // exact: a power-of-two scaling
         const uint64_t dmax = (uint64_t)std::max<int64_t>(g->tuning.big_min_deg, kThreadMaxDeg);
         if (fneed <= 62 && wq_max < 0x1p62 &&
             (unsigned __int128)(uint64_t)wq_max * dmax < ((unsigned __int128)1 << 63)) {
@@ -885,8 +939,7 @@ int setup_phase(nido_graph* g)
                                       std::min(v1, v0 + i * kSegVerts), std::min(v1, v0 + (i + 1) * kSegVerts)});
         }
         g->nseg = (int64_t)seg.size();
-        NIDO_TRY(upload(&g->d_seg, seg, g->stream));
-        HIP_TRY(hipStreamSynchronize(g->stream));
+        NIDO_TRY(upload(g, &g->d_seg, &g->seg_cap, seg));
     }
     return NIDO_OK;
 }
@@ -964,10 +1017,8 @@ int do_modularity(nido_graph* g, double* q)
     }
     g->inc_ok = g->G == 1 && (!g->windowed || g->win_single);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(g->h_q, g->d_q, sizeof(double), hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
+    NIDO_TRY(fetch(g, q, g->d_q, sizeof(double)));
     g->prof.harvest();
-    *q = *g->h_q;
     return NIDO_OK;
 }
 
@@ -1155,6 +1206,7 @@ int iteration_launches(nido_graph* g, bool inc)
     } live_guard{g};
     g->win_live = g->win_double && g->nb > 0;
     if (g->win_live) {
+        NIDO_TRY(need_side(g));
         // the halves are free once the main stream's earlier work (which may
         // read the window) is done; window_load must copy afresh afterwards
         HIP_TRY(hipEventRecord(g->ev_free[0], g->stream));
@@ -1282,6 +1334,7 @@ int launch_or_replay(nido_graph* g, bool inc)
     if (!replaying(g)) return iteration_launches(g, inc);
     hipGraphExec_t& exec = g->iter_exec[inc ? 1 : 0];
     if (!exec) {
+        NIDO_TRY(need_side(g));
         HIP_TRY(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
         const int rc = iteration_launches(g, inc);
         hipGraph_t graph = nullptr;
@@ -1306,10 +1359,8 @@ int do_iteration(nido_graph* g, double* q, double* dq, double* qt_out = nullptr)
     NIDO_TRY(run_iteration_launches(g));
     double qt = 0;
     if (g->twom != 0) {
-        HIP_TRY(hipMemcpyAsync(g->h_q, g->d_q, sizeof(double), hipMemcpyDeviceToHost, g->stream));
-        HIP_TRY(hipStreamSynchronize(g->stream));
+        NIDO_TRY(fetch(g, &qt, g->d_q, sizeof(double)));
         g->prof.harvest();
-        qt = *g->h_q;
     }
     if (qt_out) *qt_out = qt;
     *dq = qt - *q;
@@ -1325,20 +1376,16 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
 {
     hipStream_t s = g->stream;
     const int64_t nv = g->nv, K1 = K + 1;
+    ArenaScope scope(g->ws);
     // sizes: seven arrays of K + 1 entries, the last entry of mfill the
     // length of the mid list
-    int64_t *sizes = nullptr, *noff = nullptr, *ncol = nullptr, *hd = nullptr, *wpre = nullptr;
+    int64_t *sizes = nullptr, *totals = nullptr, *noff = nullptr, *ncol = nullptr, *hd = nullptr, *wpre = nullptr;
     int *cid = nullptr, *members = nullptr, *ckey = nullptr, *mid = nullptr, *tkey = nullptr;
     double *nw = nullptr, *cw = nullptr;
     fx_t* tval = nullptr;
-    void *tmp = nullptr, *tmp2 = nullptr;
+    char *tmp = nullptr, *tmp2 = nullptr;
     auto cleanup = [&]() {
-        dev_free(sizes); dev_free(noff); dev_free(ncol); dev_free(hd); dev_free(wpre);
-        dev_free(cid); dev_free(members); dev_free(ckey); dev_free(mid); dev_free(tkey);
-        dev_free(nw); dev_free(cw); dev_free(tval);
-        raw_free(tmp);
-        raw_free(tmp2);
-        tmp = tmp2 = nullptr;
+        dev_free(noff); dev_free(ncol); dev_free(nw);
     };
     int rc = NIDO_OK;
     // a failed HIP call leaves the loop with the error, and cleanup runs
@@ -1348,9 +1395,9 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         break;                                                                                             \
     }
     do {
-        if ((rc = dev_alloc(&sizes, 7 * K1)) || (rc = dev_alloc(&noff, K1)) || (rc = dev_alloc(&mid, K1)) ||
-            (rc = dev_alloc(&cid, nv)) || (rc = dev_alloc(&members, nv)) ||
-            (rc = raw_alloc(&tmp, 4 * scan_temp_bytes(K1))))
+        if ((rc = g->ws.get(&sizes, 7 * K1)) || (rc = g->ws.get(&totals, 4)) || (rc = dev_alloc(&noff, K1)) ||
+            (rc = g->ws.get(&mid, K1)) || (rc = g->ws.get(&cid, nv)) || (rc = g->ws.get(&members, nv)) ||
+            (rc = g->ws.get(&tmp, 4 * (int64_t)scan_temp_bytes(K1))))
             break;
         int64_t *const arcs = sizes, *const cnt = sizes + K1;
         unsigned long long* const mfill = reinterpret_cast<unsigned long long*>(sizes + 2 * K1);
@@ -1361,17 +1408,14 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         launch_fill_i64(sizes, 0, 3 * K1, s);
         launch_member_counts(g->d_C, newid, g->d_off, nv, cid, cnt, arcs, s, gid, keep);
         launch_coarse_sizes(arcs, cnt, K, R, s);
-        launch_exclusive_scans(R.ml, K, 4, K1, tmp, s);
-        int64_t ML = 0, MH = 0, T = 0, Tc = 0;
-        COARSEN_HIP(hipMemcpyAsync(&ML, R.ml + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipMemcpyAsync(&MH, R.mh + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipMemcpyAsync(&T, R.toff + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipMemcpyAsync(&Tc, R.cpos + K, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipStreamSynchronize(s));
+        launch_exclusive_scans(R.ml, K, 4, K1, totals, tmp, s);
+        int64_t tot[4] = {0, 0, 0, 0};
+        if ((rc = fetch(g, tot, totals, sizeof(tot)))) break;
+        const int64_t ML = tot[0], MH = tot[1], T = tot[2], Tc = tot[3];
         const int64_t nwords = T / kSlotWord;
-        if ((rc = dev_alloc(&ckey, Tc)) || (rc = dev_alloc(&cw, Tc)) || (rc = dev_alloc(&hd, MH + 1))) break;
-        if (T > 0 && ((rc = dev_alloc(&tkey, T)) || (rc = dev_alloc(&tval, T)) || (rc = dev_alloc(&wpre, nwords + 1)) ||
-                      (rc = raw_alloc(&tmp2, scan_temp_bytes(std::max(MH, nwords))))))
+        if ((rc = g->ws.get(&ckey, Tc)) || (rc = g->ws.get(&cw, Tc)) || (rc = g->ws.get(&hd, MH + 1))) break;
+        if (T > 0 && ((rc = g->ws.get(&tkey, T)) || (rc = g->ws.get(&tval, T)) || (rc = g->ws.get(&wpre, nwords + 1)) ||
+                      (rc = g->ws.get(&tmp2, (int64_t)scan_temp_bytes(std::max(MH, nwords))))))
             break;
         launch_member_scatter(cid, g->d_off, nv, R, ML, mfill, members, hd, s);
         launch_coarse_lds(arcs, R, members, g->d_off, g->d_col32, g->d_w, cid, K, ckey, cw, cnt, s);
@@ -1388,14 +1432,13 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         launch_exclusive_scan(cnt, noff, K, noff + K, tmp, s);
         COARSEN_HIP(hipGetLastError());
         std::vector<int64_t> hoff((size_t)K + 1);
-        COARSEN_HIP(hipMemcpyAsync(hoff.data(), noff, sizeof(int64_t) * (size_t)(K + 1), hipMemcpyDeviceToHost, s));
-        COARSEN_HIP(hipStreamSynchronize(s));
+        if ((rc = fetch(g, hoff.data(), noff, sizeof(int64_t) * (size_t)(K + 1)))) break;
         const int64_t nne = hoff[(size_t)K];
         if ((rc = dev_alloc(&ncol, nne)) || (rc = dev_alloc(&nw, nne))) break;
-        launch_coarse_emit(R.toff, K, noff, ncol, nw, R.cpos, ckey, cw, s);
-        launch_coarse_emit_hbm(R.toff, tkey, tval, K, wpre, nwords, noff, ncol, nw, s);
+        // the fine graph's 32-bit columns have been read: the coarse ones take their place
+        launch_coarse_emit(R.toff, K, noff, ncol, g->d_col32, nw, R.cpos, ckey, cw, s);
+        launch_coarse_emit_hbm(R.toff, tkey, tval, K, wpre, nwords, noff, ncol, g->d_col32, nw, s);
         COARSEN_HIP(hipGetLastError());
-        COARSEN_HIP(hipStreamSynchronize(s));
         free_graph_arrays(g);
         g->d_off = noff; noff = nullptr;
         g->d_col = ncol; ncol = nullptr;
@@ -1403,7 +1446,6 @@ int coarsen(nido_graph* g, const int64_t* newid, int64_t K, const int* gid, cons
         g->nv = K;
         g->ne = nne;
         g->h_off.swap(hoff);
-        g->grid_known = g->narrowed = false;
     } while (0);
 #undef COARSEN_HIP
     cleanup();
@@ -1440,7 +1482,6 @@ int coarsen_host(nido_graph* g, const int64_t* newid, int64_t K)
     g->nv = K;
     g->ne = nne;
     g->h_off.swap(noff);
-    g->grid_known = g->narrowed = false;
     return NIDO_OK;
 }
 
@@ -1455,10 +1496,9 @@ int do_aggregation(nido_graph* g, int* done)
     launch_exclusive_scan(newid, newid, nv, g->d_tot, g->d_scan_tmp, s);
     HIP_TRY(hipGetLastError());
     int64_t K = 0;
-    HIP_TRY(hipMemcpyAsync(&K, g->d_tot, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     launch_update_clustering(g->d_clus, g->n0, g->d_C, newid, s);   // graph_gpu.cpp:1389
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
+    NIDO_TRY(fetch(g, &K, g->d_tot, sizeof(int64_t)));
     if (K == nv || K == 1) {                                          // graph_gpu.cpp:1391-1392
         *done = 1;
         return NIDO_OK;
@@ -1567,17 +1607,14 @@ int batch_modularity(nido_graph* g, std::vector<double>& q)
     }
     HIP_TRY(hipGetLastError());
     q.resize((size_t)g->G);
-    HIP_TRY(hipMemcpyAsync(q.data(), g->d_gq, sizeof(double) * (size_t)g->G, hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
+    NIDO_TRY(fetch(g, q.data(), g->d_gq, sizeof(double) * (size_t)g->G));
     g->prof.harvest();
     return NIDO_OK;
 }
 
 int upload_flags(nido_graph* g, unsigned char* d, const std::vector<unsigned char>& h)
 {
-    HIP_TRY(hipMemcpyAsync(d, h.data(), h.size(), hipMemcpyHostToDevice, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));   // h may change right after
-    return NIDO_OK;
+    return send(g, d, h.data(), h.size());
 }
 
 // Renumbers the communities of the graphs with keep[g] set (ascending, per
@@ -1593,9 +1630,7 @@ int batch_renumber(nido_graph* g, const std::vector<unsigned char>& keep, std::v
     launch_gather_bases(newid, g->d_tot, g->d_vb, g->G, g->nv, g->d_vbn, s);
     HIP_TRY(hipGetLastError());
     nvb.resize((size_t)g->G + 1);
-    HIP_TRY(hipMemcpyAsync(nvb.data(), g->d_vbn, sizeof(int64_t) * nvb.size(), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return NIDO_OK;
+    return fetch(g, nvb.data(), g->d_vbn, sizeof(int64_t) * nvb.size());
 }
 
 int do_batch_run(nido_graph* g, int64_t max_loops, double tol, double tol_phase, nido_run_stats* st)
@@ -1639,9 +1674,7 @@ int do_batch_run(nido_graph* g, int64_t max_loops, double tol, double tol_phase,
             NIDO_TRY(upload_flags(g, g->d_act, act));
             NIDO_TRY(run_iteration_launches(g));
             qt.resize((size_t)G + 1);
-            HIP_TRY(hipMemcpyAsync(qt.data(), g->d_gq, sizeof(double) * ((size_t)G + 1), hipMemcpyDeviceToHost,
-                                   g->stream));
-            HIP_TRY(hipStreamSynchronize(g->stream));
+            NIDO_TRY(fetch(g, qt.data(), g->d_gq, sizeof(double) * ((size_t)G + 1)));
             g->prof.harvest();
             std::memcpy(&g->last_moved, &qt[(size_t)G], sizeof(int64_t));
             bool rollback = false;
@@ -1745,8 +1778,7 @@ int do_batch_run(nido_graph* g, int64_t max_loops, double tol, double tol_phase,
             HIP_TRY(hipGetLastError());
             NIDO_TRY(coarsen(g, g->d_work, nvb[(size_t)G], g->d_gid, g->d_keep));
             g->vb = nvb;
-            HIP_TRY(hipMemcpyAsync(g->d_vb, g->vb.data(), sizeof(int64_t) * g->vb.size(), hipMemcpyHostToDevice,
-                                   g->stream));
+            NIDO_TRY(send(g, g->d_vb, g->vb.data(), sizeof(int64_t) * g->vb.size()));
             launch_fill_gid(g->d_vb, G, g->d_gid, g->stream);
             HIP_TRY(hipGetLastError());
             NIDO_TRY(setup_phase(g));
@@ -1759,19 +1791,13 @@ int do_batch_run(nido_graph* g, int64_t max_loops, double tol, double tol_phase,
     }
     // clusterings: graph-local ids on the device, then one copy to the host
     if (g->n0) {
+        ArenaScope scope(g->ws);
         int64_t *d_loc = nullptr, *d_base = nullptr;
-        int rc = dev_alloc(&d_loc, g->n0);
-        if (rc == NIDO_OK) rc = dev_alloc(&d_base, G);
-        if (rc == NIDO_OK && hipMemcpyAsync(d_base, base.data(), sizeof(int64_t) * (size_t)G,
-                                            hipMemcpyHostToDevice, g->stream) != hipSuccess)
-            rc = set_error(NIDO_ERR_HIP, "clustering bases upload failed");
-        if (rc == NIDO_OK) {
-            launch_local_ids(g->d_clus, g->n0, g->d_gid0, d_base, d_loc, g->stream);
-            rc = host_clustering(g, d_loc);   // waits for the stream: base may go out of scope
-        }
-        dev_free(d_loc);
-        dev_free(d_base);
-        NIDO_TRY(rc);
+        NIDO_TRY(g->ws.get(&d_loc, g->n0));
+        NIDO_TRY(g->ws.get(&d_base, G));
+        NIDO_TRY(send(g, d_base, base.data(), sizeof(int64_t) * (size_t)G));
+        launch_local_ids(g->d_clus, g->n0, g->d_gid0, d_base, d_loc, g->stream);
+        NIDO_TRY(host_clustering(g, d_loc));
     }
     S.t_total = now_s() - t0;
     S.phases = nphase;
@@ -1920,14 +1946,6 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
             return fail(set_error(NIDO_ERR_HIP, "hipStreamCreate failed"));
         g->own_stream = true;
     }
-    if (hipStreamCreateWithFlags(&g->side, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_join, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_copied[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_copied[1], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_free[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_free[1], hipEventDisableTiming) != hipSuccess)
-        return fail(set_error(NIDO_ERR_HIP, "creating the side stream or its events failed"));
     AllocScope scope(g->stream);
     g->n0 = nv;
     g->nv = nv;
@@ -1961,11 +1979,11 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
         (rc = dev_alloc(&g->d_col32, cap)) || (rc = dev_alloc(&g->d_C32, nv)) ||
         (rc = dev_alloc(&g->d_dcomms, nv)) || (rc = dev_alloc(&g->d_touched, nv)) ||
         (rc = dev_alloc(&g->d_term, nv)) || (rc = dev_alloc(&g->d_iacc, 2)) ||
-        (rc = dev_alloc(&g->d_part, 2 * (int64_t)kPartBlocks)) || (rc = dev_alloc(&g->d_grid, 1)))
+        (rc = dev_alloc(&g->d_part, 2 * (int64_t)kPartBlocks)) || (rc = dev_alloc(&g->d_out, 1)))
         return fail(rc);
     if ((rc = raw_alloc(&g->d_scan_tmp, scan_temp_bytes(nv + 1)))) return fail(rc);
-    if (hipHostMalloc(reinterpret_cast<void**>(&g->h_q), sizeof(double)) != hipSuccess)
-        return fail(set_error(NIDO_ERR_NOMEM, "pinned allocation failed"));
+    g->pin = pinned_get(kPinBytes);
+    if (!g->pin.p) return fail(set_error(NIDO_ERR_NOMEM, "pinned allocation failed"));
     hipStream_t s = g->stream;
     launch_fill_fx(g->d_acc, 4, s);
     // Clustering::commIds_ starts as the identity (clustering.cpp:4-10)
@@ -1983,12 +2001,13 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     int64_t maxg = 0;
     for (int i = 0; i < G; ++i) maxg = std::max(maxg, gv[i + 1] - gv[i]);
     const bool local16 = fused && G > 1 && maxg <= 65536;
-    if (staged_h2d(g->d_off, g->h_off.data(), sizeof(int64_t) * (size_t)(nv + 1), s) != hipSuccess ||
-        (local16 && staged_h2d_local_ids(reinterpret_cast<uint16_t*>(g->d_col), col + base, ne, s, chk) != hipSuccess) ||
+    if ((rc = send(g, g->d_off, g->h_off.data(), sizeof(int64_t) * (size_t)(nv + 1)))) return fail(rc);
+    if (on_device && ((rc = send(g, g->d_col, col + base, sizeof(int64_t) * (size_t)ne)) ||
+                      (rc = send(g, g->d_w, w + base, sizeof(double) * (size_t)ne))))
+        return fail(rc);
+    if ((local16 && staged_h2d_local_ids(reinterpret_cast<uint16_t*>(g->d_col), col + base, ne, s, chk) != hipSuccess) ||
         (fused && !local16 && staged_h2d_ids(g->d_col32, col + base, ne, s, chk) != hipSuccess) ||
-        (fused && staged_h2d_weights(g->d_w, w + base, ne, s, chk) != hipSuccess) ||
-        (on_device && (staged_h2d(g->d_col, col + base, sizeof(int64_t) * (size_t)ne, s) != hipSuccess ||
-                       staged_h2d(g->d_w, w + base, sizeof(double) * (size_t)ne, s) != hipSuccess)))
+        (fused && staged_h2d_weights(g->d_w, w + base, ne, s, chk) != hipSuccess))
         return fail(set_error(NIDO_ERR_HIP, "upload failed"));
     if (fused) {
         bool exact = chk.bad.load() != INT64_MAX || chk.neg.load();
@@ -2002,42 +2021,35 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
             for (int64_t e = gstart[(size_t)i]; e < gstart[(size_t)i + 1]; e += kPieceArcs)
                 pieces.push_back(ArcPiece{e, std::min(gstart[(size_t)i + 1], e + kPieceArcs), gv[i], gv[i + 1] - gv[i]});
     if (on_device) {
+        ArenaScope tmp(g->ws);
         ArcPiece* d_pieces = nullptr;
-        if (G > 1 && (rc = upload(&d_pieces, pieces, s))) return fail(rc);
+        if (G > 1 && ((rc = g->ws.get(&d_pieces, (int64_t)pieces.size())) ||
+                      (rc = send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size()))))
+            return fail(rc);
         launch_take_arcs(d_pieces, G > 1 ? (int64_t)pieces.size() : (ne + kPieceArcs - 1) / kPieceArcs, ne, nv, g->d_col,
-                         g->d_w, g->d_col32, g->d_grid, s);
-        const bool ok = hipGetLastError() == hipSuccess &&
-                        hipMemcpyAsync(&g->grid, g->d_grid, sizeof(WeightGrid), hipMemcpyDeviceToHost, s) == hipSuccess &&
-                        hipStreamSynchronize(s) == hipSuccess;
-        dev_free(d_pieces);
-        if (!ok) return fail(set_error(NIDO_ERR_HIP, "checking the uploaded arcs failed"));
+                         g->d_w, g->d_col32, &g->d_out->grid, s);
+        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "checking the uploaded arcs failed"));
+        WeightGrid grid{};
+        if ((rc = fetch(g, &grid, &g->d_out->grid, sizeof(grid)))) return fail(rc);
         // (the bits of a NaN order above those of infinity)
-        const bool exact = g->grid.flags != 0 || g->grid.wmax > nido_dbits(0x1p61) ||
-                           nido_bitsd(g->grid.wmax) * (double)ne > 0x1p61;
+        const bool exact = grid.flags != 0 || grid.wmax > nido_dbits(0x1p61) ||
+                           nido_bitsd(grid.wmax) * (double)ne > 0x1p61;
         if (exact && (rc = check_csr(nv, off, col, w, G, gv, &nonneg, nullptr))) return fail(rc);
-        g->grid_known = g->narrowed = true;
     }
     g->nonneg = nonneg;
     if (local16) {
         // graph-local ids back to handle ids
+        ArenaScope tmp(g->ws);
         ArcPiece* d_pieces = nullptr;
-        if ((rc = dev_alloc(&d_pieces, std::max<int64_t>((int64_t)pieces.size(), 1)))) return fail(rc);
-        const bool ok = pieces.empty() ||
-                        (hipMemcpyAsync(d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size(),
-                                        hipMemcpyHostToDevice, s) == hipSuccess &&
-                         (launch_widen_local(d_pieces, (int64_t)pieces.size(),
-                                             reinterpret_cast<const uint16_t*>(g->d_col), g->d_col32, s),
-                          hipGetLastError() == hipSuccess) &&
-                         hipStreamSynchronize(s) == hipSuccess);   // pieces go out of scope
-        dev_free(d_pieces);
-        if (!ok) return fail(set_error(NIDO_ERR_HIP, "widening the graph-local ids failed"));
+        if ((rc = g->ws.get(&d_pieces, (int64_t)pieces.size())) ||
+            (rc = send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size())))
+            return fail(rc);
+        launch_widen_local(d_pieces, (int64_t)pieces.size(), reinterpret_cast<const uint16_t*>(g->d_col), g->d_col32, s);
+        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "widening the graph-local ids failed"));
     }
     // ids crossed the host link as int32 or 16-bit local ids (all below
     // nv < 2^31 - 1, checked); the int64 copy overwrites the local ids
-    if (fused) {
-        launch_widen_ids(g->d_col32, g->d_col, ne, s);
-        g->narrowed = true;
-    }
+    if (fused) launch_widen_ids(g->d_col32, g->d_col, ne, s);
     if (G > 1) {
         g->G = G;
         g->vb.assign(vptr, vptr + G + 1);
@@ -2049,24 +2061,18 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
             (rc = dev_alloc(&g->d_gq, (int64_t)G + 1)) ||
             (rc = dev_alloc(&g->d_moved, kMovedSlots)))
             return fail(rc);
-        if (hipMemcpyAsync(g->d_vb, g->vb.data(), sizeof(int64_t) * (size_t)(G + 1), hipMemcpyHostToDevice, s) !=
-            hipSuccess)
-            return fail(set_error(NIDO_ERR_HIP, "upload failed"));
+        if ((rc = send(g, g->d_vb, g->vb.data(), sizeof(int64_t) * (size_t)(G + 1)))) return fail(rc);
         launch_fill_gid(g->d_vb, G, g->d_gid, s);
         launch_fill_gid(g->d_vb, G, g->d_gid0, s);
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-            return fail(set_error(NIDO_ERR_HIP, "graph id set-up failed"));
+        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "graph id set-up failed"));
     }
     if ((rc = setup_phase(g))) return fail(rc);
     if (G > 1) {
         // 2m per graph, exactly (graph_cuda.cu:1855): the sum of its k_v
         g->twom_g.assign((size_t)G, 0);
         launch_graph_sums(g->d_k, g->d_vb, G, g->d_gacc, s);
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(g->twom_g.data(), g->d_gacc, sizeof(fx_t) * (size_t)G, hipMemcpyDeviceToHost, s) !=
-                hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            return fail(set_error(NIDO_ERR_HIP, "per-graph 2m failed"));
+        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "per-graph 2m failed"));
+        if ((rc = fetch(g, g->twom_g.data(), g->d_gacc, sizeof(fx_t) * (size_t)G))) return fail(rc);
         g->twom_dg.assign((size_t)G, 0.0);
         std::vector<double> mg(2 * (size_t)G), tw((size_t)G);
         for (int i = 0; i < G; ++i) {
@@ -2074,24 +2080,16 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
             mg[2 * (size_t)i] = tw[(size_t)i] * 0.5;
             mg[2 * (size_t)i + 1] = 1.0 / mg[2 * (size_t)i];   // unused while the graph has no weight
         }
-        if (hipMemcpyAsync(g->d_mg, mg.data(), sizeof(double) * 2 * (size_t)G, hipMemcpyHostToDevice, s) !=
-                hipSuccess ||
-            hipMemcpyAsync(g->d_twomg, tw.data(), sizeof(double) * (size_t)G, hipMemcpyHostToDevice, s) !=
-                hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            return fail(set_error(NIDO_ERR_HIP, "upload failed"));
+        if ((rc = send(g, g->d_mg, mg.data(), sizeof(double) * 2 * (size_t)G)) ||
+            (rc = send(g, g->d_twomg, tw.data(), sizeof(double) * (size_t)G)))
+            return fail(rc);
     }
     if (!g->windowed && ne > 0) {
-        fx_t* d_h = nullptr;   // four 64-bit sums
+        unsigned long long* const d_h = reinterpret_cast<unsigned long long*>(g->d_acc);   // four 64-bit sums
         unsigned long long h[4];
-        if ((rc = dev_alloc(&d_h, 2))) return fail(rc);
-        launch_fill_fx(d_h, 2, s);
-        launch_sym_hash(g->d_src, g->d_col32, g->d_w, ne, reinterpret_cast<unsigned long long*>(d_h), s);
-        const bool ok = hipGetLastError() == hipSuccess &&
-                        hipMemcpyAsync(h, d_h, sizeof(h), hipMemcpyDeviceToHost, s) == hipSuccess &&
-                        hipStreamSynchronize(s) == hipSuccess;
-        dev_free(d_h);
-        if (!ok) return fail(set_error(NIDO_ERR_HIP, "arc symmetry check failed"));
+        launch_sym_hash(g->d_src, g->d_col32, g->d_w, ne, reinterpret_cast<unsigned long long*>(g->d_part), d_h, s);
+        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "arc symmetry check failed"));
+        if ((rc = fetch(g, h, d_h, sizeof(h)))) return fail(rc);
         g->symmetric = h[0] == h[1] && h[2] == h[3];
     } else if (g->windowed && ne > 0) {   // the arcs are on the host
         g->symmetric = host_arcs_symmetric(nv, g->h_off.data(), g->h_col32, g->h_w);
@@ -2108,17 +2106,14 @@ int host_clustering(nido_graph* g, const int64_t* src)
         g->bclus.reset(new int64_t[(size_t)std::max<int64_t>(g->n0, 1)]);   // no zero fill: copied over
         g->bclus_n = g->n0;
     }
-    HIP_TRY(staged_d2h(g->bclus.get(), src, sizeof(int64_t) * (size_t)g->n0, g->stream));
-    return NIDO_OK;
+    return fetch(g, g->bclus.get(), src, sizeof(int64_t) * (size_t)g->n0);
 }
 
 template <typename T>
 int d2h(nido_graph* g, T* dst, const T* src, int64_t n)
 {
     if (!dst) return set_error(NIDO_ERR_INVALID, "null output array");
-    if (n > 0) HIP_TRY(hipMemcpyAsync(dst, src, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    return NIDO_OK;
+    return fetch(g, dst, src, sizeof(T) * (size_t)(n > 0 ? n : 0));
 }
 
 }  // namespace
@@ -2201,7 +2196,8 @@ int nido_graph_destroy(nido_graph* g)
     dev_free(g->d_C); dev_free(g->d_Cn); dev_free(g->d_k); dev_free(g->d_a); dev_free(g->d_kd);
     dev_free(g->d_clus); dev_free(g->d_work); dev_free(g->d_acc); dev_free(g->d_q); dev_free(g->d_tot);
     dev_free(g->d_src); dev_free(g->d_part); dev_free(g->d_col32); dev_free(g->d_C32); dev_free(g->d_wq);
-    dev_free(g->d_grid);
+    dev_free(g->d_out);
+    g->ws.reset(0);
     dev_free(g->d_gid); dev_free(g->d_gid0); dev_free(g->d_vb); dev_free(g->d_vbn); dev_free(g->d_mg);
     dev_free(g->d_twomg); dev_free(g->d_act); dev_free(g->d_keep); dev_free(g->d_gacc); dev_free(g->d_gq);
     dev_free(g->d_moved);
@@ -2212,9 +2208,8 @@ int nido_graph_destroy(nido_graph* g)
     dev_free(g->d_key_chunks); dev_free(g->d_bkey); dev_free(g->d_bw); dev_free(g->d_cpo);
     dev_free(g->d_pg); dev_free(g->d_pc); dev_free(g->d_pself); dev_free(g->d_cnt);
     dev_free(g->d_tkey); dev_free(g->d_tval);
-    dev_free(g->d_small); dev_free(g->d_items);
     raw_free(g->d_scan_tmp);
-    if (g->h_q) (void)hipHostFree(g->h_q);
+    pinned_put(g->pin);
     if (g->h_col32) (void)hipHostFree(g->h_col32);
     if (g->h_w) (void)hipHostFree(g->h_w);
     if (g->ev_fork) (void)hipEventDestroy(g->ev_fork);

@@ -316,40 +316,4 @@ void build_phase_lists(const int64_t* off, int nb, const std::vector<int64_t>& c
     merge_batches(W, nb, false, pb);
 }
 
-void build_row_lists(const int64_t* off, int64_t nv, std::vector<int>& small, std::vector<RowItem>& items)
-{
-    const int T = nv >= kParallelRows ? std::max(1, omp_get_max_threads()) : 1;
-    std::vector<std::vector<int>> ls((size_t)T);
-    std::vector<std::vector<RowItem>> li((size_t)T);
-#pragma omp parallel num_threads(T)
-    {
-        const int tid = omp_get_thread_num(), nt = omp_get_num_threads();
-        const int64_t v0 = nv * tid / nt, v1 = nv * (tid + 1) / nt;
-        auto& s = ls[(size_t)tid];
-        auto& it = li[(size_t)tid];
-        for (int64_t v = v0; v < v1; ++v) {
-            const int64_t d = off[v + 1] - off[v];
-            if (d <= kSmallRow) {
-                s.push_back((int)v);
-            } else {
-                for (int64_t e = off[v]; e < off[v + 1]; e += kItemArcs)
-                    it.push_back(RowItem{v, e, std::min(off[v + 1], e + kItemArcs)});
-            }
-        }
-    }
-    size_t ns = 0, ni = 0;
-    for (int i = 0; i < T; ++i) {
-        ns += ls[(size_t)i].size();
-        ni += li[(size_t)i].size();
-    }
-    small.clear();
-    items.clear();
-    small.reserve(ns);
-    items.reserve(ni);
-    for (int i = 0; i < T; ++i) {
-        small.insert(small.end(), ls[(size_t)i].begin(), ls[(size_t)i].end());
-        items.insert(items.end(), li[(size_t)i].begin(), li[(size_t)i].end());
-    }
-}
-
 }  // namespace nido

@@ -1,6 +1,5 @@
 // host_bins.h -- per-phase work lists of the local-moving launches, built on
-// the host (OpenMP): batch boundaries, degree bins, long-row items and the
-// row lists of the degree and modularity sweeps.
+// the host (OpenMP): batch boundaries, degree bins and long-row items.
 #pragma once
 #include <stdint.h>
 
@@ -11,8 +10,6 @@
 
 namespace nido {
 
-constexpr int64_t kSmallRow = kSmallRowArcs;
-constexpr int64_t kItemArcs = kItemRowArcs;
 // Host work lists are built with threads only from this many vertices up:
 // smaller graphs are the serving loop's, whose requests already run side by
 // side, one host thread each.
@@ -80,9 +77,5 @@ void host_vertex_weights(int64_t nv, const int64_t* off, const double* w, fx_t* 
 void host_coarsen(int64_t nv, const int64_t* off, const int* col, const double* w, const int64_t* C,
                   const int64_t* newid, int64_t K, std::vector<int64_t>& noff, std::vector<int>& ncol,
                   std::vector<double>& nw);
-
-// Rows of at most kSmallRow arcs (one lane each) and kItemArcs-arc slices
-// of the longer rows, both in ascending vertex order.
-void build_row_lists(const int64_t* off, int64_t nv, std::vector<int>& small, std::vector<RowItem>& items);
 
 }  // namespace nido

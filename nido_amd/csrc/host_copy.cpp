@@ -108,6 +108,11 @@ class Staging {
     bool reuse_ = false;
 };
 
+std::mutex g_pin_mu;
+std::vector<PinnedBlock>* g_pin = new std::vector<PinnedBlock>();   // never destroyed: no HIP calls at exit
+size_t g_pin_idle = 0;
+constexpr size_t kPinKeep = size_t(1) << 30;
+
 void atomic_min(std::atomic<int64_t>& a, int64_t x)
 {
     int64_t cur = a.load();
@@ -231,6 +236,53 @@ hipError_t ids_in_chunks(int* dst, const int64_t* src, int64_t n, hipStream_t s,
     return st.finish(e);
 }
 }  // namespace
+
+PinnedBlock pinned_get(size_t bytes)
+{
+    PinnedBlock b;
+    if (hipGetDevice(&b.device) != hipSuccess) return b;
+    const size_t want = std::max<size_t>(bytes, 1);
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        size_t best = g_pin->size();
+        for (size_t i = 0; i < g_pin->size(); ++i) {
+            const PinnedBlock& c = (*g_pin)[i];
+            if (c.device == b.device && c.bytes >= want && c.bytes / 4 <= want &&
+                (best == g_pin->size() || c.bytes < (*g_pin)[best].bytes))
+                best = i;
+        }
+        if (best < g_pin->size()) {
+            b = (*g_pin)[best];
+            g_pin->erase(g_pin->begin() + (ptrdiff_t)best);
+            g_pin_idle -= b.bytes;
+            return b;
+        }
+    }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return b;
+    }
+    b.p = static_cast<char*>(p);
+    b.bytes = want;
+    return b;
+}
+
+void pinned_put(PinnedBlock& b)
+{
+    if (!b.p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        if (g_pin_idle + b.bytes <= kPinKeep) {
+            g_pin->push_back(b);
+            g_pin_idle += b.bytes;
+            b = PinnedBlock{};
+            return;
+        }
+    }
+    (void)hipHostFree(b.p);
+    b = PinnedBlock{};
+}
 
 bool staged_path(size_t bytes)
 {

@@ -26,6 +26,19 @@ struct ArcCheck {
     std::mutex mu;
 };
 
+// Pinned host memory kept between uses: pinning 64 MiB takes 16 ms and its
+// first pages as long again.  get() hands out an idle block of at least
+// `bytes` and at most four times that, or pins a new one; put() keeps it unless
+// the idle blocks then held more than 1 GiB.  One process-wide pool for all
+// threads; the caller's streams are done with a block it puts back.
+struct PinnedBlock {
+    char* p = nullptr;
+    size_t bytes = 0;
+    int device = -1;
+};
+PinnedBlock pinned_get(size_t bytes);   // p is null when there is no memory
+void pinned_put(PinnedBlock& b);        // leaves b empty
+
 // Whether an upload of this many bytes goes through the pinned staging
 // buffers (where the ArcCheck variants check on the way).
 bool staged_path(size_t bytes);

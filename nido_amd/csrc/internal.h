@@ -89,8 +89,6 @@ struct BinRow {
 // NUM_BINS * tb0[b] + t - tb0[b], stride = the batch's tile count), so one
 // exclusive scan of cnt orders the rows by (batch, bin, id).
 constexpr int64_t kBinTileVerts = 2048;
-constexpr int64_t kSmallRowArcs = 32;      // rows handled by one lane in the degree/modularity sweeps
-constexpr int64_t kItemRowArcs = 1024;     // longer rows are cut into slices of this many arcs
 struct BinTile {
     int64_t v0, v1, at, stride;
 };
@@ -101,14 +99,6 @@ void launch_bin_scatter(const BinTile* tiles, int64_t ntiles, const int64_t* off
 // out[b * NUM_BINS + k]: the first position of group (b, k); -1 for a batch
 // without tiles.
 void launch_bin_starts(const int64_t* base, const int64_t* tb0, int nb, int64_t* out, hipStream_t s);
-// Row lists over tiles of kBinTileVerts vertices: cs / ci receive each
-// tile's rows of at most kSmallRowArcs arcs and slices of the longer rows;
-// after their exclusive scans, the scatter writes small[] and items[] in
-// ascending vertex order.
-void launch_rowlist_count(const int64_t* off, int64_t nv, int64_t* cs, int64_t* ci, hipStream_t s);
-void launch_rowlist_scatter(const int64_t* off, int64_t nv, const int64_t* cs, const int64_t* ci, int* small,
-                            RowItem* items, hipStream_t s);
-
 // The first launch of a batch: the small bins plus the key fill of the
 // batch's partitioned long rows.
 struct SmallBins {
@@ -196,20 +186,6 @@ void launch_fill_fx(fx_t* p, int64_t n, hipStream_t s);
 // Blocks of the reduction kernels, each leaving one partial sum.
 constexpr unsigned kPartBlocks = 1024;
 
-// k_v and 2m, and src[e] = the row of arc e, in one pass over the arcs.
-// `small` lists rows of at most kSmallRowArcs arcs (kRowLanes lanes each),
-// `items` slices of longer rows (one wavefront each).  *acc receives sum(k)
-// exactly, *maxabs the bits of max |FP64(k_v)|; part holds kPartBlocks
-// partials.
-constexpr int kRowLanes = 8;
-void launch_vertex_weights(const int64_t* off, const double* w, const int* small, int64_t nsmall,
-                           const RowItem* items, int64_t nitems, fx_t* k, double* kd,
-                           int64_t nv, fx_t* acc, unsigned long long* maxabs, fx_t* part, int* src,
-                           hipStream_t s);
-// out[i] = x[i] rounded to FP64.
-void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s);
-void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k, int64_t nv,
-                      hipStream_t s);
 // What a pass over the weights finds: the bits of max |w| (|x| bit patterns
 // order like the values), the fractional bits the finest nonzero one needs
 // (2000 for a subnormal or non-finite weight, INT_MIN when every weight is 0),
@@ -219,9 +195,23 @@ struct WeightGrid {
     int fneed;
     int flags;
 };
+// What the passes over a phase's arcs and vertices find: 2m exactly, the bits of
+// max |FP64(k_v)|, the grid of the weights.
+struct PhaseOut {
+    fx_t twom;
+    unsigned long long maxk;
+    WeightGrid grid;
+};
+// k_v, kd and *out, and src[e] = the row of arc e; part holds kPartBlocks
+// partials.
+void launch_vertex_weights(const int64_t* off, const double* w, int64_t ne, fx_t* k, double* kd, int64_t nv,
+                           PhaseOut* out, fx_t* part, int* src, hipStream_t s);
+// out[i] = x[i] rounded to FP64.
+void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s);
+void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k, int64_t nv,
+                      hipStream_t s);
 constexpr unsigned kArcOutside = 1;        // a column outside its graph
 constexpr unsigned kArcNegative = 2;       // a weight below zero
-void launch_weight_grid(const double* w, int64_t ne, WeightGrid* G, hipStream_t s);
 // Arcs [e0, e1) belong to the graph of nv vertices whose first one is base.
 struct ArcPiece {
     int64_t e0, e1;
@@ -236,8 +226,7 @@ void launch_take_arcs(const ArcPiece* pieces, int64_t n, int64_t ne, int64_t nv,
                       int* col32, WeightGrid* G, hipStream_t s);
 // wq[e] = w[e] * scale, exact for weights on the 1/scale grid.
 void launch_to_fixed(const double* w, int64_t* wq, int64_t ne, double scale, hipStream_t s);
-// col32[e] = (int)col[e]
-void launch_narrow_ids(const int64_t* col, int* col32, int64_t n, hipStream_t s);
+// col[e] = col32[e]
 void launch_widen_ids(const int* col32, int64_t* col, int64_t n, hipStream_t s);
 
 // Fills L.blk0 from L.n and L.nchunks; returns the number of blocks of the
@@ -287,11 +276,11 @@ void launch_commit_tracked(int64_t v0, int64_t v1, int b, int64_t* C, int64_t* C
 void launch_commit_tracked_list(const BinRow* list, int64_t n, int b, int64_t* C, int64_t* Cn, int* C32,
                                 const fx_t* k, fx_t* a, const int64_t* off, const ModDelta& D,
                                 const unsigned char* flag, hipStream_t s);
-// out[0..3] (zeroed by the caller) += hash sums of the arcs in both
-// directions: out[0] == out[1] and out[2] == out[3] when every arc (v, u, w)
-// has a reverse arc (u, v, w), the condition the incremental update needs.
-void launch_sym_hash(const int* src, const int* col, const double* w, int64_t ne, unsigned long long* out,
-                     hipStream_t s);
+// out[0..3] = hash sums of the arcs in both directions: out[0] == out[1] and
+// out[2] == out[3] when every arc (v, u, w) has a reverse arc (u, v, w), the
+// condition the incremental update needs; part holds 4 * kPartBlocks values.
+void launch_sym_hash(const int* src, const int* col, const double* w, int64_t ne, unsigned long long* part,
+                     unsigned long long* out, hipStream_t s);
 // Batch b's delta (v0, v1 are its bounds for one graph; unused with D.gid).
 void launch_mod_delta(int b, int64_t v0, int64_t v1, const int64_t* Cn, const int* C32, const int* col,
                       const double* w, const fx_t* a, double twom_d, const ModDelta& D, hipStream_t s);
@@ -332,8 +321,9 @@ size_t scan_temp_bytes(int64_t n);
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* total,
                            void* temp, hipStream_t s);
 // In place over `rows` arrays of n values, stride apart, each total at the
-// array's [n] (temp: rows * scan_temp_bytes(n)).
-void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, void* temp, hipStream_t s);
+// array's [n] and in totals[row] (temp: rows * scan_temp_bytes(n)).
+void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, int64_t* totals, void* temp,
+                            hipStream_t s);
 
 // ---- coarsening ------------------------------------------------------------
 // With gid (per current vertex) / gid0 (per original vertex) set, only the
@@ -384,9 +374,10 @@ void launch_coarse_insert(const int64_t* hpre, int64_t n, int64_t max_arcs, cons
                           fx_t* tval, hipStream_t s);
 void launch_slot_words(const int* tkey, int64_t nwords, int64_t* wcnt, hipStream_t s);
 void launch_coarse_count(const int64_t* toff, const int64_t* wpre, int64_t K, int64_t* cnt, hipStream_t s);
-void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, double* nw,
+// (ncol32: the same ids in 32 bits)
+void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, int* ncol32, double* nw,
                         const int64_t* cpos, const int* ckey, const double* cw, hipStream_t s);
 void launch_coarse_emit_hbm(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K, const int64_t* wpre,
-                            int64_t nwords, const int64_t* noff, int64_t* ncol, double* nw, hipStream_t s);
+                            int64_t nwords, const int64_t* noff, int64_t* ncol, int* ncol32, double* nw, hipStream_t s);
 
 }  // namespace nido

@@ -23,56 +23,127 @@ __global__ void fill_kernel(T* __restrict__ p, T val, int64_t n)
 // ---------------------------------------------------------------------------
 // Vertex weights (graph_cuda.cu:302-346), singleton (graph_cuda.cu:410-429)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock)
-vw_small_kernel(const int64_t* __restrict__ off, const double* __restrict__ w,
-                const int* __restrict__ small, int64_t n, fx_t* __restrict__ k, int* __restrict__ src)
+// Adds a lane's view of the weights to the whole: the largest fractional bits
+// and magnitude, and flags.  A wavefront that has nothing new leaves the
+// memory alone: atomics on one address take their turn, about 10 ns each, and
+// 8,192 wavefronts' made most of this pass (R-MAT scale 20, 60 M arcs: 194 us
+// with them, a tenth of that read time).
+__device__ __forceinline__ void join_grid(WeightGrid* G, int f, unsigned long long mx, unsigned flags)
 {
-    // kRowLanes lanes per row (at most kSmallRowArcs arcs), each taking
-    // every kRowLanes-th arc: neighbouring lanes read neighbouring arcs, and
-    // the group's first lane adds up their exact partial sums (any order
-    // gives the same sum).  The partials meet in LDS: summed with 128-bit
-    // lane shuffles of width kRowLanes instead, some k_v came out wrong on
-    // gfx950, a different few on every run.
-    __shared__ fx_t part[kBlock];
-    const int lane = threadIdx.x & (kRowLanes - 1);
-    const int64_t stride = (int64_t)gridDim.x * (kBlock / kRowLanes);
-    for (int64_t i = blockIdx.x * (int64_t)(kBlock / kRowLanes) + threadIdx.x / kRowLanes; i < n; i += stride) {
-        const int v = small[i];   // uniform within the group
-        const int64_t e1 = off[v + 1];
-        fx_t s = 0;
-        for (int64_t e = off[v] + lane; e < e1; e += kRowLanes) {
-            s += fx_from_double(w[e]);
-            src[e] = v;
-        }
-        part[threadIdx.x] = s;
-        wave_lds_sync();   // a group's lanes share one wavefront
-        if (lane == 0) {
-            fx_t t = 0;
 #pragma unroll
-            for (int j = 0; j < kRowLanes; ++j) t += part[threadIdx.x + j];
-            k[v] = t;
-        }
-        wave_lds_sync();   // read before the group's next row overwrites them
+    for (int msk = 32; msk > 0; msk >>= 1) {
+        const int of = __shfl_xor(f, msk, 64);
+        const unsigned long long om = __shfl_xor(mx, msk, 64);
+        f = of > f ? of : f;
+        mx = om > mx ? om : mx;
+        flags |= __shfl_xor(flags, msk, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        if (f > ld_i32_agent(&G->fneed)) atomicMax(&G->fneed, f);
+        if (mx > ld_u64_agent(&G->wmax)) atomicMax(&G->wmax, mx);
+        if (flags & ~(unsigned)ld_i32_agent(&G->flags)) atomicOr(&G->flags, (int)flags);
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
-vw_items_kernel(const double* __restrict__ w, const RowItem* __restrict__ items, int64_t n,
-                fx_t* __restrict__ k, int* __restrict__ src)
+// The fractional bits a weight needs (w = sig 2^(ex - 1075), lowest set bit
+// 2^(ex - 1075 + ctz(sig)); 2000 for a subnormal or non-finite weight), given
+// the bits b of |w|, not zero.
+__device__ __forceinline__ int bits_needed(unsigned long long b)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t wid = (blockIdx.x * (int64_t)kBlock + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * kBlock) >> 6;
-    for (int64_t i = wid; i < n; i += nw) {
-        const RowItem it = items[i];
-        fx_t s = 0;
-        for (int64_t e = it.e0 + lane; e < it.e1; e += 64) {
-            s += fx_from_double(w[e]);
-            src[e] = (int)it.v;
+    const int ex = (int)(b >> 52);
+    if (ex == 0 || ex == 0x7ff) return 2000;
+    return 1075 - ex - __builtin_ctzll((b & 0x000fffffffffffffull) | 0x0010000000000000ull);
+}
+
+// k (zeroed by the caller) and src[e] = the row of arc e, and the grid of the
+// weights, in one pass over the arcs: a workgroup takes tiles of kSumTile
+// consecutive arcs and a thread kSumRun consecutive ones of them; the rows of a
+// tile are found once (a 64-way search, then kSumRows offsets at a time in LDS,
+// empty rows skipped) and a thread walks them forward, summing a row's arcs in
+// registers and then in LDS.  A row inside the tile is stored, a row that
+// crosses its ends added with one atomic.  Exact integer sums: the split does
+// not change them.  No list of rows is needed (the host built two per phase,
+// or the device with two round trips), and the weights are read once for
+// everything.  Bound by the 12 B per arc and the walk.
+constexpr int kSumRun = 8, kSumTile = kBlock * kSumRun, kSumRows = 512;
+__global__ void __launch_bounds__(kBlock)
+row_sums_kernel(const int64_t* __restrict__ off, const double* __restrict__ w, int64_t nv, int64_t ne,
+                fx_t* __restrict__ k, int* __restrict__ src, WeightGrid* G)
+{
+    __shared__ int s_off[kSumRows + 1];
+    __shared__ unsigned long long lo[kSumRows], hi[kSumRows];
+    __shared__ int64_t s_row;
+    int f = INT_MIN;
+    unsigned long long mx = 0;
+    for (int64_t t0 = (int64_t)blockIdx.x * kSumTile; t0 < ne; t0 += (int64_t)gridDim.x * kSumTile) {
+        const int n = (int)(t0 + kSumTile < ne ? kSumTile : ne - t0);
+        if (threadIdx.x < 64) {
+            const int64_t r = wave_row_of(off, 0, nv, t0);
+            if (threadIdx.x == 0) s_row = r;
         }
-        s = wave_sum_fx(s);
-        if (lane == 0) acc_add(k + it.v, s);
+        const int x0 = threadIdx.x * kSumRun;
+        double wt[kSumRun];
+#pragma unroll
+        for (int j = 0; j < kSumRun; ++j) {
+            wt[j] = x0 + j < n ? w[t0 + x0 + j] : 0.0;
+            const unsigned long long b = nido_dbits(wt[j]) & 0x7fffffffffffffffull;
+            if (b == 0) continue;
+            const int need = bits_needed(b);
+            f = need > f ? need : f;
+            mx = b > mx ? b : mx;
+        }
+        __syncthreads();
+        for (;;) {                               // uniform: kSumRows rows at a time
+            const int64_t r0 = s_row;
+            for (int q = threadIdx.x; q <= kSumRows; q += kBlock) {
+                const int64_t at = (r0 + q < nv ? off[r0 + q] : ne) - t0;
+                s_off[q] = at < 0 ? 0 : at < n ? (int)at : n;
+            }
+            for (int q = threadIdx.x; q < kSumRows; q += kBlock) {
+                lo[q] = 0;
+                hi[q] = 0;
+            }
+            __syncthreads();
+            const int c0 = s_off[0], c1 = s_off[kSumRows];
+            int l = -1;                          // the row of the arc before
+            fx_t sum = 0;
+#pragma unroll
+            for (int j = 0; j < kSumRun; ++j) {
+                const int x = x0 + j;
+                if (x < c0 || x >= c1) continue;
+                if (l < 0) {
+                    l = 0;
+#pragma unroll
+                    for (int st = kSumRows / 2; st > 0; st >>= 1)
+                        if (s_off[l + st] <= x) l += st;
+                } else if (s_off[l + 1] <= x) {
+                    fx_atomic_add(&lo[l], &hi[l], sum);
+                    sum = 0;
+                    do ++l;
+                    while (s_off[l + 1] <= x);   // x < c1 = s_off[kSumRows]: ends
+                }
+                sum += fx_from_double(wt[j]);
+                src[t0 + x] = (int)(r0 + l);
+            }
+            if (l >= 0) fx_atomic_add(&lo[l], &hi[l], sum);
+            __syncthreads();
+            for (int q = threadIdx.x; q < kSumRows; q += kBlock) {
+                if (s_off[q] >= s_off[q + 1]) continue;   // no arcs in this tile
+                const int64_t r = r0 + q;
+                const fx_t x = fx_make(lo[q], (int64_t)hi[q]);
+                if (off[r] >= t0 && off[r + 1] <= t0 + n) k[r] = x;
+                else acc_add(k + r, x);
+            }
+            if (c1 >= n) break;                  // uniform
+            if (threadIdx.x < 64) {              // the next row with arcs in this tile
+                const int64_t r = wave_row_of(off, r0 + kSumRows, nv, t0 + c1);
+                if (threadIdx.x == 0) s_row = r;
+            }
+            __syncthreads();
+        }
+        __syncthreads();                         // s_row and the sums are reused by the next tile
     }
+    join_grid(G, f, mx, 0);
 }
 
 // kd = FP64(k); part[block] = this block's sum of k; *maxabs = max |kd| as
@@ -98,7 +169,7 @@ round_kernel(const fx_t* __restrict__ k, double* __restrict__ kd, int64_t n,
         const unsigned long long o = __shfl_xor(mx, msk, 64);
         mx = o > mx ? o : mx;
     }
-    if ((threadIdx.x & 63) == 0 && mx) atomicMax(maxabs, mx);
+    if ((threadIdx.x & 63) == 0 && mx > ld_u64_agent(maxabs)) atomicMax(maxabs, mx);
     s = block_sum_fx(s, red);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -136,14 +207,6 @@ singleton_kernel(int64_t* __restrict__ C, int64_t* __restrict__ Cn, int* __restr
 }
 
 __global__ void __launch_bounds__(kBlock)
-narrow_kernel(const int64_t* __restrict__ col, int* __restrict__ col32, int64_t n)
-{
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * kBlock)
-        col32[i] = (int)col[i];
-}
-
-__global__ void __launch_bounds__(kBlock)
 widen_kernel(const int* __restrict__ col32, int64_t* __restrict__ col, int64_t n)
 {
     for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n;
@@ -151,57 +214,16 @@ widen_kernel(const int* __restrict__ col32, int64_t* __restrict__ col, int64_t n
         col[i] = col32[i];
 }
 
-// Adds a lane's view of the weights to the whole: the largest fractional bits
-// and magnitude, and flags.  A wavefront that has nothing new leaves the
-// memory alone: atomics on one address take their turn, about 10 ns each, and
-// 8,192 wavefronts' made most of this pass (R-MAT scale 20, 60 M arcs: 194 us
-// with them, a tenth of that read time).
-__device__ __forceinline__ void join_grid(WeightGrid* G, int f, unsigned long long mx, unsigned flags)
-{
-#pragma unroll
-    for (int msk = 32; msk > 0; msk >>= 1) {
-        const int of = __shfl_xor(f, msk, 64);
-        const unsigned long long om = __shfl_xor(mx, msk, 64);
-        f = of > f ? of : f;
-        mx = om > mx ? om : mx;
-        flags |= __shfl_xor(flags, msk, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        if (f > ld_i32_agent(&G->fneed)) atomicMax(&G->fneed, f);
-        if (mx > ld_u64_agent(&G->wmax)) atomicMax(&G->wmax, mx);
-        if (flags & ~(unsigned)ld_i32_agent(&G->flags)) atomicOr(&G->flags, (int)flags);
-    }
-}
-
-// The fractional bits a weight needs (w = sig 2^(ex - 1075), lowest set bit
-// 2^(ex - 1075 + ctz(sig)); 2000 for a subnormal or non-finite weight), given
-// the bits b of |w|, not zero.
-__device__ __forceinline__ int bits_needed(unsigned long long b)
-{
-    const int ex = (int)(b >> 52);
-    if (ex == 0 || ex == 0x7ff) return 2000;
-    return 1075 - ex - __builtin_ctzll((b & 0x000fffffffffffffull) | 0x0010000000000000ull);
-}
-
 __global__ void grid_init_kernel(WeightGrid* G)
 {
     *G = WeightGrid{0, INT_MIN, 0};
 }
 
-// The grid every weight lies on (WeightGrid).
-__global__ void __launch_bounds__(kBlock)
-weight_grid_kernel(const double* __restrict__ w, int64_t ne, WeightGrid* G)
+__global__ void phase_init_kernel(PhaseOut* out)
 {
-    int f = INT_MIN;
-    unsigned long long mx = 0;
-    for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < ne; e += (int64_t)gridDim.x * kBlock) {
-        const unsigned long long b = nido_dbits(w[e]) & 0x7fffffffffffffffull;
-        if (b == 0) continue;
-        const int need = bits_needed(b);
-        f = need > f ? need : f;
-        mx = b > mx ? b : mx;
-    }
-    join_grid(G, f, mx, 0);
+    out->twom = 0;
+    out->maxk = 0;
+    out->grid = WeightGrid{0, INT_MIN, 0};
 }
 
 // The caller's arcs once they are on the device: ids narrowed into col32, an
@@ -402,11 +424,15 @@ __device__ __forceinline__ unsigned long long arc_hash(unsigned a, unsigned b, u
     return mix64(mix64((((unsigned long long)a << 32) | b) ^ key) ^ wb);
 }
 
+// Each workgroup leaves its four sums in part; sym_sum_kernel adds them up
+// (8,192 wavefronts adding to the same four words took 320 us whatever the
+// size of the graph, 546 us for 60 M arcs).
 __global__ void __launch_bounds__(kBlock)
 sym_hash_kernel(const int* __restrict__ src, const int* __restrict__ col, const double* __restrict__ w, int64_t ne,
-                unsigned long long* __restrict__ out)
+                unsigned long long* __restrict__ part)
 {
     constexpr unsigned long long k1 = 0x6a09e667f3bcc909ull, k2 = 0xbb67ae8584caa73bull;
+    __shared__ unsigned long long red[4][kBlock / 64];
     unsigned long long h[4] = {0, 0, 0, 0};
     for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < ne; e += (int64_t)gridDim.x * kBlock) {
         const unsigned a = (unsigned)src[e], b = (unsigned)col[e];
@@ -420,8 +446,27 @@ sym_hash_kernel(const int* __restrict__ src, const int* __restrict__ col, const 
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
         for (int msk = 32; msk > 0; msk >>= 1) h[i] += __shfl_xor(h[i], msk, 64);
-        if ((threadIdx.x & 63) == 0 && h[i] != 0) atomicAdd(out + i, h[i]);
+        if ((threadIdx.x & 63) == 0) red[i][threadIdx.x >> 6] = h[i];
     }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        unsigned long long t = 0;
+        for (int i = 0; i < kBlock / 64; ++i) t += red[threadIdx.x][i];
+        part[4 * (int64_t)blockIdx.x + threadIdx.x] = t;
+    }
+}
+
+// out[i] = the sum of part[4 j + i] over the n workgroups j (a wavefront per i).
+__global__ void __launch_bounds__(kBlock)
+sym_sum_kernel(const unsigned long long* __restrict__ part, int n, unsigned long long* __restrict__ out)
+{
+    static_assert(kBlock / 64 == 4, "a wavefront per sum");
+    const int i = threadIdx.x >> 6;
+    unsigned long long t = 0;
+    for (int j = threadIdx.x & 63; j < n; j += 64) t += part[4 * j + i];
+#pragma unroll
+    for (int msk = 32; msk > 0; msk >>= 1) t += __shfl_xor(t, msk, 64);
+    if ((threadIdx.x & 63) == 0) out[i] = t;
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -509,7 +554,8 @@ scan_tile_sums_kernel(const int64_t* __restrict__ in, int64_t n, int64_t* __rest
 
 __global__ void __launch_bounds__(kBlock)
 scan_tile_apply_kernel(const int64_t* in, int64_t* out, int64_t n,
-                       const int64_t* __restrict__ tile_off, int64_t* total, int64_t stride)
+                       const int64_t* __restrict__ tile_off, int64_t* total, int64_t stride,
+                       int64_t* __restrict__ totals)
 {
     __shared__ int64_t wt[kBlock / 64];
     in += blockIdx.y * stride;
@@ -533,7 +579,10 @@ scan_tile_apply_kernel(const int64_t* in, int64_t* out, int64_t n,
         if (i < n) out[i] = run;
         run += v[j];
     }
-    if (total && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) *total = run;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) {
+        if (total) *total = run;
+        if (totals) totals[blockIdx.y] = run;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1086,7 +1135,8 @@ constexpr int kEmitRun = 32;
 __global__ void __launch_bounds__(kBlock)
 coarse_emit_hbm_kernel(const int64_t* __restrict__ toff, const int* __restrict__ tkey,
                        const fx_t* __restrict__ tval, int64_t K, const int64_t* __restrict__ wpre, int64_t nwords,
-                       const int64_t* __restrict__ noff, int64_t* __restrict__ ncol, double* __restrict__ nw_out)
+                       const int64_t* __restrict__ noff, int64_t* __restrict__ ncol, int* __restrict__ ncol32,
+                       double* __restrict__ nw_out)
 {
     const int lane = threadIdx.x & 63;
     const int64_t nw = (int64_t)gridDim.x * (kBlock / 64);
@@ -1111,6 +1161,7 @@ coarse_emit_hbm_kernel(const int64_t* __restrict__ toff, const int* __restrict__
             if (c >= 0) {
                 const int64_t p = delta + wpre[x] + __popcll(m & ((1ull << lane) - 1));
                 ncol[p] = c;
+                ncol32[p] = c;
                 nw_out[p] = fx_to_double(tval[s]);
             }
         }
@@ -1120,7 +1171,8 @@ coarse_emit_hbm_kernel(const int64_t* __restrict__ toff, const int* __restrict__
 // The compact entries of the LDS-aggregated rows into the coarse CSR.
 __global__ void __launch_bounds__(kBlock)
 coarse_emit_kernel(const int64_t* __restrict__ toff, int64_t K, const int64_t* __restrict__ noff,
-                   int64_t* __restrict__ ncol, double* __restrict__ nw_out, const int64_t* __restrict__ cpos,
+                   int64_t* __restrict__ ncol, int* __restrict__ ncol32, double* __restrict__ nw_out,
+                   const int64_t* __restrict__ cpos,
                    const int* __restrict__ ckey, const double* __restrict__ cw)
 {
     const int lane = threadIdx.x & 63;
@@ -1131,6 +1183,7 @@ coarse_emit_kernel(const int64_t* __restrict__ toff, int64_t K, const int64_t* _
         const int64_t pos = noff[i], n = noff[i + 1] - pos, c0 = cpos[i];
         for (int64_t r = lane; r < n; r += 64) {
             ncol[pos + r] = ckey[c0 + r];
+            ncol32[pos + r] = ckey[c0 + r];
             nw_out[pos + r] = cw[c0 + r];
         }
     }
@@ -1229,12 +1282,6 @@ void launch_fill_i64(int64_t* p, int64_t val, int64_t n, hipStream_t s)
     fill_kernel<int64_t><<<grid_for(n, kBlock * 4), kBlock, 0, s>>>(p, val, n);
 }
 
-void launch_weight_grid(const double* w, int64_t ne, WeightGrid* G, hipStream_t s)
-{
-    grid_init_kernel<<<1, 1, 0, s>>>(G);
-    if (ne > 0) weight_grid_kernel<<<grid_for(ne, kBlock * 8, 2048), kBlock, 0, s>>>(w, ne, G);
-}
-
 void launch_take_arcs(const ArcPiece* pieces, int64_t n, int64_t ne, int64_t nv, const int64_t* col, const double* w,
                       int* col32, WeightGrid* G, hipStream_t s)
 {
@@ -1265,22 +1312,17 @@ void launch_fill_fx(fx_t* p, int64_t n, hipStream_t s)
     fill_kernel<fx_t><<<grid_for(n, kBlock * 4), kBlock, 0, s>>>(p, (fx_t)0, n);
 }
 
-void launch_vertex_weights(const int64_t* off, const double* w, const int* small, int64_t nsmall,
-                           const RowItem* items, int64_t nitems, fx_t* k, double* kd,
-                           int64_t nv, fx_t* acc, unsigned long long* maxabs, fx_t* part, int* src,
-                           hipStream_t s)
+void launch_vertex_weights(const int64_t* off, const double* w, int64_t ne, fx_t* k, double* kd, int64_t nv,
+                           PhaseOut* out, fx_t* part, int* src, hipStream_t s)
 {
-    launch_fill_i64(reinterpret_cast<int64_t*>(maxabs), 0, 1, s);
-    launch_fill_fx(acc, 1, s);
+    phase_init_kernel<<<1, 1, 0, s>>>(out);
     if (nv <= 0) return;
     launch_fill_fx(k, nv, s);
-    if (nsmall > 0)
-        vw_small_kernel<<<grid_for(nsmall * kRowLanes, kBlock), kBlock, 0, s>>>(off, w, small, nsmall, k, src);
-    if (nitems > 0)
-        vw_items_kernel<<<grid_for(nitems, kBlock / 64), kBlock, 0, s>>>(w, items, nitems, k, src);
+    if (ne > 0)
+        row_sums_kernel<<<grid_for(ne, kSumTile, 8192), kBlock, 0, s>>>(off, w, nv, ne, k, src, &out->grid);
     const unsigned g = grid_for(nv, kBlock, kPartBlocks);
-    round_kernel<<<g, kBlock, 0, s>>>(k, kd, nv, maxabs, part);
-    sum_partials_kernel<<<1, kBlock, 0, s>>>(part, (int)g, acc);
+    round_kernel<<<g, kBlock, 0, s>>>(k, kd, nv, &out->maxk, part);
+    sum_partials_kernel<<<1, kBlock, 0, s>>>(part, (int)g, &out->twom);
 }
 
 void launch_fx_round(const fx_t* x, double* out, int64_t n, hipStream_t s)
@@ -1295,11 +1337,6 @@ void launch_singleton(int64_t* C, int64_t* Cn, int* C32, fx_t* a, const fx_t* k,
     singleton_kernel<<<grid_for(nv, kBlock), kBlock, 0, s>>>(C, Cn, C32, a, k, nv);
 }
 
-void launch_narrow_ids(const int64_t* col, int* col32, int64_t n, hipStream_t s)
-{
-    if (n <= 0) return;
-    narrow_kernel<<<grid_for(n, kBlock), kBlock, 0, s>>>(col, col32, n);
-}
 
 void launch_widen_ids(const int* col32, int64_t* col, int64_t n, hipStream_t s)
 {
@@ -1334,10 +1371,13 @@ void launch_modularity_terms(const fx_t* a, int64_t nv, double twom_d, fx_t* acc
     mod_acc_finish_kernel<<<1, 64, 0, s>>>(acc, twom_d, q);
 }
 
-void launch_sym_hash(const int* src, const int* col, const double* w, int64_t ne, unsigned long long* out,
-                     hipStream_t s)
+void launch_sym_hash(const int* src, const int* col, const double* w, int64_t ne, unsigned long long* part,
+                     unsigned long long* out, hipStream_t s)
 {
-    if (ne > 0) sym_hash_kernel<<<grid_for(ne, kBlock, 2048), kBlock, 0, s>>>(src, col, w, ne, out);
+    static_assert(4 * sizeof(unsigned long long) == 2 * sizeof(fx_t), "kPartBlocks workgroups' sums fit the partials");
+    const unsigned g = grid_for(ne, kBlock, kPartBlocks);
+    sym_hash_kernel<<<g, kBlock, 0, s>>>(src, col, w, ne, part);
+    sym_sum_kernel<<<1, kBlock, 0, s>>>(part, (int)g, out);
 }
 
 void launch_mod_delta(int b, int64_t v0, int64_t v1, const int64_t* Cn, const int* C32, const int* col,
@@ -1369,19 +1409,19 @@ size_t scan_temp_bytes(int64_t n)
 }
 
 static void scan_rows(const int64_t* in, int64_t* out, int64_t n, int rows, int64_t stride, int64_t* total,
-                      void* temp, hipStream_t s)
+                      int64_t* totals, void* temp, hipStream_t s)
 {
     const int64_t tiles = (n + kScanTile - 1) / kScanTile;
     const dim3 grid((unsigned)tiles, (unsigned)rows);
     if (tiles == 1) {
-        scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, nullptr, total, stride);
+        scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, nullptr, total, stride, totals);
         return;
     }
     int64_t* sums = reinterpret_cast<int64_t*>(temp);
     void* rest = sums + tiles * rows;
     scan_tile_sums_kernel<<<grid, kBlock, 0, s>>>(in, n, sums, stride);
-    scan_rows(sums, sums, tiles, rows, tiles, nullptr, rest, s);
-    scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, sums, total, stride);
+    scan_rows(sums, sums, tiles, rows, tiles, nullptr, nullptr, rest, s);
+    scan_tile_apply_kernel<<<grid, kBlock, 0, s>>>(in, out, n, sums, total, stride, totals);
 }
 
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* total,
@@ -1391,12 +1431,13 @@ void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* 
         if (total) launch_fill_i64(total, 0, 1, s);
         return;
     }
-    scan_rows(in, out, n, 1, 0, total, temp, s);
+    scan_rows(in, out, n, 1, 0, total, nullptr, temp, s);
 }
 
-void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, void* temp, hipStream_t s)
+void launch_exclusive_scans(int64_t* x, int64_t n, int rows, int64_t stride, int64_t* totals, void* temp,
+                            hipStream_t s)
 {
-    if (n > 0) scan_rows(x, x, n, rows, stride, x + n, temp, s);
+    if (n > 0) scan_rows(x, x, n, rows, stride, x + n, totals, temp, s);
 }
 
 void launch_mark_communities(const int64_t* C, int64_t nv, int64_t* flag, hipStream_t s,
@@ -1505,19 +1546,20 @@ void launch_coarse_count(const int64_t* toff, const int64_t* wpre, int64_t K, in
     if (K > 0) coarse_count_kernel<<<grid_for(K, kBlock), kBlock, 0, s>>>(toff, wpre, K, cnt);
 }
 
-void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, double* nw,
+void launch_coarse_emit(const int64_t* toff, int64_t K, const int64_t* noff, int64_t* ncol, int* ncol32, double* nw,
                         const int64_t* cpos, const int* ckey, const double* cw, hipStream_t s)
 {
     if (K > 0)
-        coarse_emit_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(toff, K, noff, ncol, nw, cpos, ckey, cw);
+        coarse_emit_kernel<<<grid_for(K, kBlock / 64), kBlock, 0, s>>>(toff, K, noff, ncol, ncol32, nw, cpos, ckey,
+                                                                       cw);
 }
 
 void launch_coarse_emit_hbm(const int64_t* toff, const int* tkey, const fx_t* tval, int64_t K, const int64_t* wpre,
-                            int64_t nwords, const int64_t* noff, int64_t* ncol, double* nw, hipStream_t s)
+                            int64_t nwords, const int64_t* noff, int64_t* ncol, int* ncol32, double* nw, hipStream_t s)
 {
     if (nwords > 0)
         coarse_emit_hbm_kernel<<<grid_for(nwords, kEmitRun * (kBlock / 64)), kBlock, 0, s>>>(
-            toff, tkey, tval, K, wpre, nwords, noff, ncol, nw);
+            toff, tkey, tval, K, wpre, nwords, noff, ncol, ncol32, nw);
 }
 
 }  // namespace nido
