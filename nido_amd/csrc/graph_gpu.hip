@@ -190,8 +190,15 @@ struct BatchResult {
     std::vector<nido_phase_stats> phases;
 };
 
-constexpr int64_t kSegArcs = 65536;    // arcs per per-graph modularity item
-constexpr int64_t kSegVerts = 16384;   // vertices per per-graph modularity item
+// Arcs of a per-graph modularity item: a power of two that gives the sweep some
+// 4,096 items, within bounds; a quarter as many vertices.
+constexpr int64_t kSegArcsMin = 2048, kSegArcsMax = 16384, kSegItems = 4096;
+int64_t seg_arcs(int64_t ne)
+{
+    int64_t a = kSegArcsMin;
+    while (a < kSegArcsMax && a * kSegItems < ne) a *= 2;
+    return a;
+}
 
 double now_s()
 {
@@ -930,13 +937,14 @@ int setup_phase(nido_graph* g)
     if (G > 1) {
         // per-graph modularity items: arc and vertex chunks of each graph
         std::vector<SegItem> seg;
+        const int64_t sa = seg_arcs(g->ne), sv = sa / 4;
         for (int gg = 0; gg < G; ++gg) {
             const int64_t v0 = g->vb[(size_t)gg], v1 = g->vb[(size_t)gg + 1];
             const int64_t e0 = off[v0], e1 = off[v1];
-            const int64_t n = std::max((e1 - e0 + kSegArcs - 1) / kSegArcs, (v1 - v0 + kSegVerts - 1) / kSegVerts);
+            const int64_t n = std::max((e1 - e0 + sa - 1) / sa, (v1 - v0 + sv - 1) / sv);
             for (int64_t i = 0; i < n; ++i)
-                seg.push_back(SegItem{gg, std::min(e1, e0 + i * kSegArcs), std::min(e1, e0 + (i + 1) * kSegArcs),
-                                      std::min(v1, v0 + i * kSegVerts), std::min(v1, v0 + (i + 1) * kSegVerts)});
+                seg.push_back(SegItem{gg, std::min(e1, e0 + i * sa), std::min(e1, e0 + (i + 1) * sa),
+                                      std::min(v1, v0 + i * sv), std::min(v1, v0 + (i + 1) * sv)});
         }
         g->nseg = (int64_t)seg.size();
         NIDO_TRY(upload(g, &g->d_seg, &g->seg_cap, seg));
