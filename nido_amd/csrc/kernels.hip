@@ -57,31 +57,35 @@ __device__ __forceinline__ int bits_needed(unsigned long long b)
 
 // k (zeroed by the caller) and src[e] = the row of arc e, and the grid of the
 // weights, in one pass over the arcs: a workgroup takes tiles of kSumTile
-// consecutive arcs and a thread kSumRun consecutive ones of them; the rows of a
-// tile are found once (a 64-way search, then kSumRows offsets at a time in LDS,
-// empty rows skipped; coarse graphs of R-MAT have ten rows without arcs for one
-// with some, and with 512 at a time the search set the time, 92 us on 5 K rows
-// and 44 K arcs) and a thread walks them forward, summing a row's arcs in
-// registers and then in LDS.  A row inside the tile is stored, a row that
-// crosses its ends added with one atomic.  Exact integer sums: the split does
-// not change them.  No list of rows is needed (the host built two per phase,
-// or the device with two round trips), and the weights are read once for
-// everything.  Bound by the 12 B per arc and the walk.
-constexpr int kSumRun = 8, kSumTile = kBlock * kSumRun, kSumRows = 2048;
+// consecutive arcs and a thread kSumRun consecutive ones of them.  The first
+// and the last row of a tile are found by 64-way searches.  Where at most
+// kSumSpan rows lie between them, the workgroup takes kSumRows offsets at a
+// time into LDS and a thread walks them forward, summing a row's arcs in
+// registers and then in LDS; a row inside the tile is stored, a row that
+// crosses its ends added with one atomic.  Where more lie between them, most
+// have no arcs (coarse graphs of R-MAT: ten without for one with some): every
+// thread then searches for the rows of its own arcs and adds a row's sum to k.
+// Walking such tiles through LDS as well took one of them to 3.9 ms (first
+// coarse graph of R-MAT scale 20, 0.03 ms with the search).  Exact integer
+// sums: the split does not change them.  No list of rows is needed (the host
+// built two per phase, or the device with two round trips), and the weights
+// are read once for everything.  Bound by the 12 B per arc and the walk.
+constexpr int kSumRun = 8, kSumTile = kBlock * kSumRun, kSumRows = 2048, kSumSpan = 2 * kSumRows;
 __global__ void __launch_bounds__(kBlock)
 row_sums_kernel(const int64_t* __restrict__ off, const double* __restrict__ w, int64_t nv, int64_t ne,
                 fx_t* __restrict__ k, int* __restrict__ src, WeightGrid* G)
 {
     __shared__ int s_off[kSumRows + 1];
     __shared__ unsigned long long lo[kSumRows], hi[kSumRows];
-    __shared__ int64_t s_row;
+    __shared__ int64_t s_row[2];
     int f = INT_MIN;
     unsigned long long mx = 0;
     for (int64_t t0 = (int64_t)blockIdx.x * kSumTile; t0 < ne; t0 += (int64_t)gridDim.x * kSumTile) {
         const int n = (int)(t0 + kSumTile < ne ? kSumTile : ne - t0);
-        if (threadIdx.x < 64) {
-            const int64_t r = wave_row_of(off, 0, nv, t0);
-            if (threadIdx.x == 0) s_row = r;
+        if (threadIdx.x < 128) {                 // wavefront 0: the first row, 1: the last
+            const int last = threadIdx.x >> 6;
+            const int64_t r = wave_row_of(off, 0, nv, last ? t0 + n - 1 : t0);
+            if ((threadIdx.x & 63) == 0) s_row[last] = r;
         }
         const int x0 = threadIdx.x * kSumRun;
         double wt[kSumRun];
@@ -95,8 +99,28 @@ row_sums_kernel(const int64_t* __restrict__ off, const double* __restrict__ w, i
             mx = b > mx ? b : mx;
         }
         __syncthreads();
-        for (;;) {                               // uniform: kSumRows rows at a time
-            const int64_t r0 = s_row;
+        const int64_t rf = s_row[0], span = s_row[1] - rf + 1;
+        if (span > kSumSpan) {                   // uniform
+            if (x0 < n) {
+                int64_t x[kSumRun], row[kSumRun];
+#pragma unroll
+                for (int j = 0; j < kSumRun; ++j) x[j] = t0 + (x0 + j < n ? x0 + j : n - 1);
+                rows_of<kSumRun>(off, rf, span, x, row);
+                fx_t sum = 0;
+#pragma unroll
+                for (int j = 0; j < kSumRun; ++j) {
+                    if (x0 + j >= n) break;
+                    src[t0 + x0 + j] = (int)row[j];
+                    sum += fx_from_double(wt[j]);
+                    if (j + 1 < kSumRun && x0 + j + 1 < n && row[j + 1] == row[j]) continue;
+                    acc_add(k + row[j], sum);
+                    sum = 0;
+                }
+            }
+            __syncthreads();                     // s_row is reused by the next tile
+            continue;
+        }
+        for (int64_t r0 = rf; r0 < rf + span; r0 += kSumRows) {   // uniform: kSumRows rows at a time
             for (int q = threadIdx.x; q <= kSumRows; q += kBlock) {
                 const int64_t at = (r0 + q < nv ? off[r0 + q] : ne) - t0;
                 s_off[q] = at < 0 ? 0 : at < n ? (int)at : n;
@@ -136,14 +160,8 @@ row_sums_kernel(const int64_t* __restrict__ off, const double* __restrict__ w, i
                 if (off[r] >= t0 && off[r + 1] <= t0 + n) k[r] = x;
                 else acc_add(k + r, x);
             }
-            if (c1 >= n) break;                  // uniform
-            if (threadIdx.x < 64) {              // the next row with arcs in this tile
-                const int64_t r = wave_row_of(off, r0 + kSumRows, nv, t0 + c1);
-                if (threadIdx.x == 0) s_row = r;
-            }
-            __syncthreads();
+            __syncthreads();                     // s_off and the sums are reused
         }
-        __syncthreads();                         // s_row and the sums are reused by the next tile
     }
     join_grid(G, f, mx, 0);
 }

@@ -73,17 +73,19 @@ na_check_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ com
 // every weight into P.mass.  Arc-parallel: a workgroup takes tiles of
 // kNaTile consecutive arcs and a thread kNaRun consecutive ones of them, whose
 // loads and comm gathers are all in flight before the first is used; the rows
-// of the tile are found once per workgroup (a 64-way search, then kNaRows
-// offsets at a time in LDS) and a thread walks them forward.  The weights of a
-// thread's part of a row are summed in registers, then per community in an LDS
-// table, so a community takes one global atomic per tile.  Exact integer sums:
+// of the tile are found once per workgroup (64-way searches of the first and
+// the last, then kNaRows offsets at a time in LDS) and a thread walks them
+// forward.  The weights of a thread's part of a row are summed in registers,
+// then per community in an LDS table, so a community takes one global atomic
+// per tile.  A tile that spans more than kNaSpan rows, most of them empty, has
+// every thread search for its own arcs' rows instead.  Exact integer sums:
 // neither the split nor the order changes them.  Bound by the 16 B per arc and
 // the comm gathers; 2^20 vertices, 14.7 M arcs in planted blocks: 150 us,
 // against 511 us with a wavefront per row (a quarter of its lanes busy, a
 // 128-bit wavefront sum and two global atomics per row).  An id outside [0, nv)
 // is never used as an index: it sets the flag; with the flag set by
 // na_check_kernel nothing is read.
-constexpr int kNaRun = 8, kNaTile = kBlock * kNaRun, kNaRows = 512, kNaSlots = 2 * kNaRows;
+constexpr int kNaRun = 8, kNaTile = kBlock * kNaRun, kNaRows = 512, kNaSlots = 2 * kNaRows, kNaSpan = 8 * kNaRows;
 __global__ void __launch_bounds__(kBlock)
 na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col, const double* __restrict__ w,
                const int64_t* __restrict__ comm, int64_t nv, fx_t* __restrict__ a, Partials P)
@@ -92,7 +94,7 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
     __shared__ unsigned long long lo[kNaSlots], hi[kNaSlots];
     __shared__ int s_off[kNaRows + 1], s_comm[kNaRows], s_slot[kNaRows];
     __shared__ fx_t red[kBlock / 64];
-    __shared__ int64_t s_row;
+    __shared__ int64_t s_row[2];
     // Set by na_check_kernel.  A workgroup that sees it set by another one of
     // this launch (an arc id out of range) may leave as well: Q is NaN then.
     __shared__ int s_bad;
@@ -109,9 +111,10 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
             lo[s] = 0;
             hi[s] = 0;
         }
-        if (threadIdx.x < 64) {
-            const int64_t r = wave_row_of(off, 0, nv, t0);
-            if (threadIdx.x == 0) s_row = r;
+        if (threadIdx.x < 128) {                     // wavefront 0: the first row, 1: the last
+            const int last = threadIdx.x >> 6;
+            const int64_t r = wave_row_of(off, 0, nv, last ? t0 + n - 1 : t0);
+            if ((threadIdx.x & 63) == 0) s_row[last] = r;
         }
         const int x0 = threadIdx.x * kNaRun;
         int64_t u[kNaRun];
@@ -129,7 +132,31 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
             cu[j] = ok ? (int)comm[u[j]] : -1;
         }
         __syncthreads();
-        for (int64_t r0 = s_row;; r0 += kNaRows) {   // uniform: kNaRows rows at a time
+        const int64_t rf = s_row[0], span = s_row[1] - rf + 1;
+        if (span > kNaSpan) {                        // uniform
+            if (x0 < n) {
+                int64_t x[kNaRun], row[kNaRun];
+#pragma unroll
+                for (int j = 0; j < kNaRun; ++j) x[j] = t0 + (x0 + j < n ? x0 + j : n - 1);
+                rows_of<kNaRun>(off, rf, span, x, row);
+                fx_t k = 0;
+#pragma unroll
+                for (int j = 0; j < kNaRun; ++j) {
+                    if (x0 + j >= n) break;
+                    const int64_t c = comm[row[j]];
+                    const fx_t f = fx_from_double(wt[j]);
+                    k += f;
+                    M += f;
+                    if (cu[j] == c) I += f;
+                    if (j + 1 < kNaRun && x0 + j + 1 < n && row[j + 1] == row[j]) continue;
+                    acc_add(a + c, k);
+                    k = 0;
+                }
+            }
+            __syncthreads();                         // the table and s_row are reused
+            continue;
+        }
+        for (int64_t r0 = rf; r0 < rf + span; r0 += kNaRows) {   // uniform: kNaRows rows at a time
             for (int q = threadIdx.x; q <= kNaRows; q += kBlock) {
                 const int64_t at = (r0 + q < nv ? off[r0 + q] : A1) - t0;
                 s_off[q] = at < 0 ? 0 : at < n ? (int)at : n;
@@ -177,7 +204,6 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
                 hi[s] = 0;
             }
             __syncthreads();                         // s_off and the table are reused
-            if (c1 >= n) break;                      // uniform
         }
     }
     I = block_sum_fx(I, red);
