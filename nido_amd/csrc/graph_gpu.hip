@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/nido_amd.h"
+#include "device_mem.h"
 #include "errors.h"
 #include "host_bins.h"
 #include "host_check.h"
@@ -41,57 +42,19 @@ namespace {
     } while (0)
 
 
-// Device memory is stream-ordered: allocations and frees made while a
-// handle's AllocScope is active go through a library-owned memory pool on
-// that handle's stream (hipMallocFromPoolAsync / hipFreeAsync), so a free
-// never waits for the whole device -- handles running side by side on
-// their own streams (a serving loop) do not stall each other.  The pool
-// keeps freed memory for reuse.
-thread_local hipStream_t t_alloc_stream = nullptr;
+// The memory (device_mem.h) of the handle whose AllocScope is active in this
+// thread.
+thread_local DeviceMem* t_mem = nullptr;
 
 struct AllocScope {
-    hipStream_t prev;
-    explicit AllocScope(hipStream_t s) : prev(t_alloc_stream) { t_alloc_stream = s; }
-    ~AllocScope() { t_alloc_stream = prev; }
+    DeviceMem* prev;
+    explicit AllocScope(DeviceMem& m) : prev(t_mem) { t_mem = &m; }
+    ~AllocScope() { t_mem = prev; }
 };
-
-hipMemPool_t device_pool()
-{
-    static std::mutex mu;
-    static std::vector<hipMemPool_t> pools;
-    static std::vector<char> tried;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lock(mu);
-    if ((int)pools.size() <= dev) {
-        pools.resize((size_t)dev + 1, nullptr);
-        tried.resize((size_t)dev + 1, 0);
-    }
-    if (!tried[(size_t)dev]) {
-        tried[(size_t)dev] = 1;
-        hipMemPoolProps props{};
-        props.allocType = hipMemAllocationTypePinned;
-        props.handleTypes = hipMemHandleTypeNone;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        hipMemPool_t pool = nullptr;
-        if (hipMemPoolCreate(&pool, &props) == hipSuccess) {
-            uint64_t keep = UINT64_MAX;
-            (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-            pools[(size_t)dev] = pool;
-        } else {
-            (void)hipGetLastError();
-        }
-    }
-    return pools[(size_t)dev];
-}
 
 int raw_alloc(void** p, size_t bytes)
 {
-    *p = nullptr;
-    if (bytes == 0) bytes = 16;
-    hipMemPool_t pool = t_alloc_stream ? device_pool() : nullptr;
-    hipError_t e = pool ? hipMallocFromPoolAsync(p, bytes, pool, t_alloc_stream) : hipMalloc(p, bytes);
+    const hipError_t e = t_mem ? t_mem->get(p, bytes) : hipMalloc(p, std::max<size_t>(bytes, 16));
     if (e != hipSuccess) {
         *p = nullptr;
         (void)hipGetLastError();
@@ -104,7 +67,7 @@ int raw_alloc(void** p, size_t bytes)
 void raw_free(void* p)
 {
     if (!p) return;
-    if (t_alloc_stream && device_pool()) (void)hipFreeAsync(p, t_alloc_stream);
+    if (t_mem) t_mem->put(p);
     else (void)hipFree(p);
 }
 
@@ -296,6 +259,7 @@ struct nido_graph {
     bool own_stream = false;
     hipStream_t side = nullptr;    // long rows of a batch, beside the short rows on `stream`
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    DeviceMem mem;
     int device = 0;
     int nb = NIDO_DEFAULT_BATCHES;
     nido_tuning tuning{};
@@ -443,7 +407,8 @@ struct nido_graph {
     hipEvent_t ev_copied[2] = {nullptr, nullptr};   // half h of the window holds its next batch
     hipEvent_t ev_free[2] = {nullptr, nullptr};     // half h's last batch is done with it
     bool win_live = false;               // an iteration is streaming its batches through the halves
-    int* h_col32 = nullptr;              // the phase's CSR on the host (pinned) while windowed
+    PinnedBlock pin_col, pin_w;          // the phase's CSR on the host (pinned) while windowed:
+    int* h_col32 = nullptr;
     double* h_w = nullptr;
     int64_t h_cap = 0;
     std::vector<int64_t> units;          // window units: consecutive rows of one batch
@@ -1954,7 +1919,8 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
             return fail(set_error(NIDO_ERR_HIP, "hipStreamCreate failed"));
         g->own_stream = true;
     }
-    AllocScope scope(g->stream);
+    g->mem.open(g->stream);
+    AllocScope scope(g->mem);
     g->n0 = nv;
     g->nv = nv;
     g->ne = ne;
@@ -1967,9 +1933,12 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
     const int64_t cap = windowed0 ? window : ne;
     int rc;
     if (windowed0) {
-        if (hipHostMalloc(reinterpret_cast<void**>(&g->h_col32), sizeof(int) * (size_t)ne) != hipSuccess ||
-            hipHostMalloc(reinterpret_cast<void**>(&g->h_w), sizeof(double) * (size_t)ne) != hipSuccess)
+        g->pin_col = pinned_get(sizeof(int) * (size_t)ne);
+        g->pin_w = pinned_get(sizeof(double) * (size_t)ne);
+        if (!g->pin_col.p || !g->pin_w.p)
             return fail(set_error(NIDO_ERR_NOMEM, "pinned host allocation of %lld arcs failed", (long long)ne));
+        g->h_col32 = reinterpret_cast<int*>(g->pin_col.p);
+        g->h_w = reinterpret_cast<double*>(g->pin_w.p);
         g->h_cap = ne;
 #pragma omp parallel for schedule(static) if (ne >= (int64_t(1) << 22))
         for (int64_t e = 0; e < ne; ++e) {
@@ -2176,6 +2145,7 @@ int nido_graph_create(int64_t nv, int64_t ne, const int64_t* off, const int64_t*
         const int64_t arcs = off[nv] - off[0];
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
+            free_b += DeviceMem::cached();
             const double avail = 0.85 * (double)free_b - kDeviceBytesPerVertex * (double)nv;
             if (kDeviceBytesPerArc * (double)arcs > avail && avail > 0)
                 window = std::max<int64_t>((int64_t)(avail / kWindowBytesPerArc), 1);
@@ -2198,7 +2168,8 @@ int nido_graph_destroy(nido_graph* g)
 {
     if (!g) return NIDO_OK;
     if (g->stream) (void)hipStreamSynchronize(g->stream);
-    AllocScope scope(g->stream);
+    if (g->side) (void)hipStreamSynchronize(g->side);
+    AllocScope scope(g->mem);
     drop_iteration_graph(g);
     free_graph_arrays(g);
     dev_free(g->d_C); dev_free(g->d_Cn); dev_free(g->d_k); dev_free(g->d_a); dev_free(g->d_kd);
@@ -2217,9 +2188,10 @@ int nido_graph_destroy(nido_graph* g)
     dev_free(g->d_pg); dev_free(g->d_pc); dev_free(g->d_pself); dev_free(g->d_cnt);
     dev_free(g->d_tkey); dev_free(g->d_tval);
     raw_free(g->d_scan_tmp);
+    g->mem.release();
     pinned_put(g->pin);
-    if (g->h_col32) (void)hipHostFree(g->h_col32);
-    if (g->h_w) (void)hipHostFree(g->h_w);
+    pinned_put(g->pin_col);
+    pinned_put(g->pin_w);
     if (g->ev_fork) (void)hipEventDestroy(g->ev_fork);
     if (g->ev_join) (void)hipEventDestroy(g->ev_join);
     for (int h = 0; h < 2; ++h) {
@@ -2269,7 +2241,7 @@ int nido_graph_set_tuning(nido_graph* g, const nido_tuning* t)
         return set_error(NIDO_ERR_INVALID, "full_modularity must be 0, 1 or 2");
     if ((t->fixed_short | 1) != 1) return set_error(NIDO_ERR_INVALID, "fixed_short must be 0 or 1");
     if (!g) return set_error(NIDO_ERR_INVALID, "null handle");
-    AllocScope scope(g->stream);
+    AllocScope scope(g->mem);
     API_GUARD(g->tuning = *t; return setup_phase(g);)
 }
 
@@ -2330,7 +2302,7 @@ int nido_aggregation(nido_graph* g, int* done)
 {
     NIDO_TRY(single_graph(g));
     if (!done) return set_error(NIDO_ERR_INVALID, "null argument");
-    AllocScope scope(g->stream);
+    AllocScope scope(g->mem);
     API_GUARD(return do_aggregation(g, done);)
 }
 
@@ -2471,7 +2443,7 @@ int nido_louvain_run(nido_graph* g, int64_t max_loops, double tol, double tol_ph
                      int verbose, nido_run_stats* stats)
 {
     NIDO_TRY(single_graph(g));
-    AllocScope scope(g->stream);
+    AllocScope scope(g->mem);
     API_GUARD(return do_run(g, max_loops, tol, tol_phase, record, verbose, stats);)
 }
 
@@ -2494,7 +2466,7 @@ int nido_batch_create(int ngraphs, const int64_t* vptr, const int64_t* off, cons
 int nido_batch_run(nido_graph* g, int64_t max_loops, double tol, double tol_phase, nido_run_stats* stats)
 {
     if (!g) return set_error(NIDO_ERR_INVALID, "null graph");
-    AllocScope scope(g->stream);
+    AllocScope scope(g->mem);
     if (g->G == 1) {
         // one graph: the plain path, with its result kept in the batched form
         nido_run_stats S{};
@@ -2513,7 +2485,7 @@ int nido_autotune(nido_graph* g, int iterations, nido_tuning* chosen)
 {
     if (!g) return set_error(NIDO_ERR_INVALID, "null graph");
     if (iterations < 1) return set_error(NIDO_ERR_INVALID, "iterations must be >= 1");
-    AllocScope scope(g->stream);
+    AllocScope scope(g->mem);
     API_GUARD(return do_autotune(g, iterations, chosen);)
 }
 
