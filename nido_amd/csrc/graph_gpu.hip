@@ -884,7 +884,7 @@ int setup_phase(nido_graph* g)
     if (g->tuning.fixed_short && g->ne > 0 && g->twom != 0 && !g->windowed) {
         const int fneed = out.grid.fneed, F = std::max(fneed, 0);
         const double wq_max = std::ldexp(nido_bitsd(out.grid.wmax), F);   // exact: a power-of-two scaling
-        const uint64_t dmax = (uint64_t)std::max<int64_t>(g->tuning.big_min_deg, kThreadMaxDeg);
+        const uint64_t dmax = (uint64_t)std::max<int64_t>({g->tuning.big_min_deg, kThreadMaxDeg, kFixedArcs});
         if (fneed <= 62 && wq_max < 0x1p62 &&
             (unsigned __int128)(uint64_t)wq_max * dmax < ((unsigned __int128)1 << 63)) {
             if (g->ne > g->wq_cap) {

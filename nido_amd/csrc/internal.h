@@ -25,6 +25,9 @@ constexpr int NUM_SMALL_BINS = BIN_BIG;
 // faster with 8 lanes each (one arc per lane, LDS table) than with one lane
 // holding the whole row: R-MAT s22 end to end, +5% over a bound of 8.
 constexpr int kThreadMaxDeg = 2;
+// Fixed-point weights are taken where at least this many of them sum below
+// 2^63, and any short row (the key fill sums that many in a wavefront).
+constexpr int64_t kFixedArcs = 512;
 constexpr int64_t kBinMaxDeg[NUM_BINS] = {kThreadMaxDeg, 16, 32, 64, 128, 512, INT64_MAX};
 constexpr int64_t kBigPartArcs = 1024;    // expected distinct keys per partition, at most
 constexpr int kBigSlots = 2048;           // LDS table of a partition workgroup (40/48 KB: 4 or 3 per CU)

@@ -424,11 +424,33 @@ __device__ __forceinline__ void block_body(const LmArgs& A, const BinRow* __rest
 constexpr int kFillUnroll = (int)(kKeyChunkArcs / kBlock);
 constexpr int kFillScan = (kMaxParts + 1 + kBlock - 1) / kBlock;   // counters per thread in the scan
 
-template <bool Multi>
+// Once communities have formed, a few of them hold most of a hub's arcs, and
+// all arcs into one community fall into one partition: on a Chung-Lu graph of
+// 2.1 M vertices one of the 74 partitions of a row had 14,897 of its 64,511
+// arcs, the median one 130, and took 59 us of inserts in a launch whose other
+// workgroups were done after 15.  A wavefront therefore looks at up to
+// kHeavyTries communities of its first 64 arcs and sums those of its arcs (up
+// to 512) that lead into one which at least kHeavyMin of the 64 have; the sum
+// takes their place as one entry, or as two where it has more bits than an FP64
+// significand.  Iterations of that graph's first phase: 41.9 -> 30.6 ms; with 8
+// tries 31.2, from 6 of 64 arcs 33.0; R-MAT scale 20, whole run: 56.3 -> 54.5.
+// Rows of fewer than kHeavyParts partitions leave it out: none of theirs can
+// hold up a launch, and the sums' chain of a load and two LDS round trips cost
+// the small launches of R-MAT scale 17 2%.  With fixed-point weights only:
+// kFixedArcs of them sum below 2^63.
+constexpr int kHeavyTries = 12, kHeavyMin = 4, kHeavyParts = 16;
+static_assert(kFillUnroll * 64 <= kFixedArcs, "a wavefront's fixed-point sums could overflow");
+
+// LDS of the key fill: counters, then the summed communities' sums.
+constexpr int kFillCounters = ((kMaxParts + 1 + kBlock / 64) * 4 + 15) & ~15;
+constexpr int kFillLds = kFillCounters + kBlock / 64 * kHeavyTries * 8;
+
+template <bool Multi, bool Fixed>
 __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L, int bi, int nbk, char* lds)
 {
     int* cnt = reinterpret_cast<int*>(lds);      // kMaxParts + 1 counters
     int* wtot = cnt + kMaxParts + 1;
+    unsigned long long* hsum = reinterpret_cast<unsigned long long*>(lds + kFillCounters);
     for (int64_t i = bi; i < L.nchunks; i += nbk) {
         const KeyChunk ch = L.chunks[i];
         Mass m;
@@ -447,7 +469,48 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
         }
 #pragma unroll
         for (int j = 0; j < kFillUnroll; ++j) cc[j] = cc[j] >= 0 ? (cc[j] != ch.v ? A.C[cc[j]] : -1) : -2;
+        int xc = -2;                // this lane's summed community (-2: none)
+        int64_t xs = 0;             // its sum in units of 2^-F
+        if constexpr (Fixed) {
+            const int lane = threadIdx.x & 63;
+            unsigned long long* const hs = hsum + (threadIdx.x >> 6) * kHeavyTries;
+            unsigned long long left = P >= kHeavyParts ? __ballot(cc[0] >= 0) : 0;
+            int nh = 0;
+            for (int t = 0; t < kHeavyTries && left; ++t) {
+                const int c = __builtin_amdgcn_readlane(cc[0], __builtin_ctzll(left));
+                const unsigned long long same = __ballot(cc[0] == c);
+                left &= ~same;
+                if (__popcll(same) < kHeavyMin) continue;
+                if (lane == nh) {
+                    xc = c;
+                    hs[nh] = 0;
+                }
+#pragma unroll
+                for (int j = 0; j < kFillUnroll; ++j)
+                    if (cc[j] == c) cc[j] = -3 - nh;
+                ++nh;
+            }
+            if (nh) {               // uniform over the wavefront
+                wave_lds_sync();
+#pragma unroll
+                for (int j = 0; j < kFillUnroll; ++j)
+                    if (cc[j] <= -3) {
+                        atomicAdd(&hs[-3 - cc[j]], (unsigned long long)A.wq[ch.e0 + j * kBlock + threadIdx.x]);
+                        cc[j] = -2;
+                    }
+                wave_lds_sync();
+                if (lane < nh) xs = (int64_t)hs[lane];
+            }
+        }
+        // in two parts, each exact in FP64, where the sum itself may not be
+        const int64_t x1 = xs & ~((int64_t(1) << 11) - 1), x2 = xs - x1;
+        const bool two = x2 != 0 && (xs >= int64_t(1) << 53 || xs <= -(int64_t(1) << 53));
         auto part_of = [&](int c) { return c == -2 ? -1 : c < 0 ? P : part_of_key(c, P); };
+        int xr = 0;
+        if constexpr (Fixed) {
+            const int px = part_of(xc);
+            if (px >= 0) xr = atomicAdd(&cnt[px], two ? 2 : 1);
+        }
 #pragma unroll
         for (int j = 0; j < kFillUnroll; ++j) {
             const int pj = part_of(cc[j]);
@@ -484,14 +547,25 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
                 L.bw[pos] = A.w[ch.e0 + j * kBlock + threadIdx.x];
             }
         }
+        if constexpr (Fixed) {
+            const int px = part_of(xc);
+            if (px >= 0) {
+                const int64_t pos = ch.k0 + cnt[px] + xr;
+                L.bkey[pos] = xc;
+                L.bw[pos] = (double)(two ? x1 : xs) * A.wscale;
+                if (two) {
+                    L.bkey[pos + 1] = xc;
+                    L.bw[pos + 1] = (double)x2 * A.wscale;
+                }
+            }
+        }
         __syncthreads();          // cnt and wtot are reused by the next chunk
     }
 }
 
 constexpr int kSmallLds = 20480;   // (256/G)*S*20 for every short-row bin
 constexpr int kSmallLdsFixed = 12288;   // (256/G)*S*12: fixed-point sums need no high words
-static_assert((kMaxParts + 1 + kBlock / 64) * 4 <= kSmallLdsFixed, "key-fill counters exceed the LDS buffer");
-static_assert((kMaxParts + 1 + kBlock / 64) * 4 <= kSmallLds, "key-fill counters exceed the LDS buffer");
+static_assert(kFillLds <= kSmallLdsFixed && kFillLds <= kSmallLds, "the key fill exceeds the LDS buffer");
 
 // Seven waves per SIMD; eight for a handle of many graphs with fixed-point
 // sums (12 KB of tables instead of 20 KB, registers held to 64 with a few
@@ -521,7 +595,7 @@ lm_small_kernel(LmArgs A, SmallBins L)
     case BIN_G64: group_body<64, 256, Multi, Fixed>(A, NIDO_BIN_ARGS(BIN_G64), lds, sself); break;
     case BIN_B256: block_body<1024, Multi, Fixed>(A, NIDO_BIN_ARGS(BIN_B256), lds, R, sself); break;
     case NUM_SMALL_BINS:
-        keyfill_body<Multi>(A, L, b - L.blk0[NUM_SMALL_BINS], L.blk0[NUM_SMALL_BINS + 1] - L.blk0[NUM_SMALL_BINS],
+        keyfill_body<Multi, Fixed>(A, L, b - L.blk0[NUM_SMALL_BINS], L.blk0[NUM_SMALL_BINS + 1] - L.blk0[NUM_SMALL_BINS],
                             lds);
         break;
     default:
