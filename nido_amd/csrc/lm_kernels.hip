@@ -441,9 +441,13 @@ constexpr int kFillScan = (kMaxParts + 1 + kBlock - 1) / kBlock;   // counters p
 constexpr int kHeavyTries = 12, kHeavyMin = 4, kHeavyParts = 16;
 static_assert(kFillUnroll * 64 <= kFixedArcs, "a wavefront's fixed-point sums could overflow");
 
-// LDS of the key fill: counters, then the summed communities' sums.
+// LDS of the key fill: counters, the summed communities' sums, and the buckets
+// on their way out.
 constexpr int kFillCounters = ((kMaxParts + 1 + kBlock / 64) * 4 + 15) & ~15;
-constexpr int kFillLds = kFillCounters + kBlock / 64 * kHeavyTries * 8;
+constexpr int kFillSums = kBlock / 64 * kHeavyTries * 8;
+constexpr int kFillHalf = (int)kKeyChunkArcs / 2;
+constexpr int kFillLds = kFillCounters + kFillSums + (int)kKeyChunkArcs * 4;
+static_assert(kFillHalf * 8 == (int)kKeyChunkArcs * 4, "keys and half of the weights share the buffer");
 
 template <bool Multi, bool Fixed>
 __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L, int bi, int nbk, char* lds)
@@ -451,6 +455,8 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
     int* cnt = reinterpret_cast<int*>(lds);      // kMaxParts + 1 counters
     int* wtot = cnt + kMaxParts + 1;
     unsigned long long* hsum = reinterpret_cast<unsigned long long*>(lds + kFillCounters);
+    int* skey = reinterpret_cast<int*>(lds + kFillCounters + kFillSums);
+    double* sw = reinterpret_cast<double*>(skey);
     for (int64_t i = bi; i < L.nchunks; i += nbk) {
         const KeyChunk ch = L.chunks[i];
         Mass m;
@@ -538,33 +544,53 @@ __device__ __forceinline__ void keyfill_body(const LmArgs& A, const SmallBins& L
             pre += loc[q];
         }
         __syncthreads();
+        // The buckets leave through LDS, keys first, then the weights in two
+        // halves.  Stored straight from the lanes, a row's 2 x 2048 values went
+        // to nearly as many lines, a line a clock and CU: with the C gathers
+        // that is what bounds the fill (31 us a chunk with seven workgroups on
+        // a CU in the batches of R-MAT scale 22 that hold its hubs).  Iterations
+        // of its first phase 43.3 -> 42.3 ms; with
+        // the weights loaded half by half 42.6.
+        double wt[kFillUnroll];
+        const int total = cnt[P];
 #pragma unroll
         for (int j = 0; j < kFillUnroll; ++j) {
             const int pj = part_of(cc[j]);
-            if (pj >= 0 && pj < P) {
-                const int64_t pos = ch.k0 + cnt[pj] + rk[j];
-                L.bkey[pos] = cc[j];
-                L.bw[pos] = A.w[ch.e0 + j * kBlock + threadIdx.x];
-            }
+            const bool in = pj >= 0 && pj < P;
+            wt[j] = in ? A.w[ch.e0 + j * kBlock + threadIdx.x] : 0.0;
+            rk[j] = in ? rk[j] + cnt[pj] : -1;
+            if (in) skey[rk[j]] = cc[j];
         }
-        if constexpr (Fixed) {
-            const int px = part_of(xc);
-            if (px >= 0) {
-                const int64_t pos = ch.k0 + cnt[px] + xr;
-                L.bkey[pos] = xc;
-                L.bw[pos] = (double)(two ? x1 : xs) * A.wscale;
-                if (two) {
-                    L.bkey[pos + 1] = xc;
-                    L.bw[pos + 1] = (double)x2 * A.wscale;
-                }
+        const int px = part_of(xc);
+        const int xpos = px >= 0 ? cnt[px] + xr : -1;
+        if (Fixed && xpos >= 0) {
+            skey[xpos] = xc;
+            if (two) skey[xpos + 1] = xc;
+        }
+        __syncthreads();
+        for (int q = threadIdx.x; q < total; q += kBlock) L.bkey[ch.k0 + q] = skey[q];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int q0 = h * kFillHalf;
+            if (q0 >= total) break;                     // uniform
+            __syncthreads();                            // the buffer has been read
+#pragma unroll
+            for (int j = 0; j < kFillUnroll; ++j)
+                if (rk[j] >= q0 && rk[j] < q0 + kFillHalf) sw[rk[j] - q0] = wt[j];
+            if (Fixed && xpos >= 0) {
+                if (xpos >= q0 && xpos < q0 + kFillHalf) sw[xpos - q0] = (double)(two ? x1 : xs) * A.wscale;
+                if (two && xpos + 1 >= q0 && xpos + 1 < q0 + kFillHalf) sw[xpos + 1 - q0] = (double)x2 * A.wscale;
             }
+            __syncthreads();
+            const int n = total - q0 < kFillHalf ? total - q0 : kFillHalf;
+            for (int q = threadIdx.x; q < n; q += kBlock) L.bw[ch.k0 + q0 + q] = sw[q];
         }
         __syncthreads();          // cnt and wtot are reused by the next chunk
     }
 }
 
 constexpr int kSmallLds = 20480;   // (256/G)*S*20 for every short-row bin
-constexpr int kSmallLdsFixed = 12288;   // (256/G)*S*12: fixed-point sums need no high words
+constexpr int kSmallLdsFixed = 12800;   // (256/G)*S*12 = 12288: fixed-point sums need no high words; the key fill takes the rest
 static_assert(kFillLds <= kSmallLdsFixed && kFillLds <= kSmallLds, "the key fill exceeds the LDS buffer");
 
 // Seven waves per SIMD; eight for a handle of many graphs with fixed-point
