@@ -378,20 +378,20 @@ __device__ __forceinline__ int64_t wave_row_of(const int64_t* __restrict__ off, 
     return lo;
 }
 
-// row[j] = the last row l of [r0, r0 + span) with off[l] <= x[j], given
-// off[r0] <= x[j] and off nondecreasing: N searches side by side, so that a
-// thread waits for ceil(log2(span)) loads, not N times as many.
+// r0 + row[j] = the last row l of [r0, r0 + span) with off[l] <= min(x + j,
+// last), given off[r0] <= x and off nondecreasing: N searches side by side, so
+// that a thread waits for ceil(log2(span)) loads, not N times as many.
 template <int N>
-__device__ __forceinline__ void rows_of(const int64_t* __restrict__ off, int64_t r0, int64_t span, const int64_t* x,
-                                        int64_t* row)
+__device__ __forceinline__ void rows_of(const int64_t* __restrict__ off, int64_t r0, int span, int64_t x, int64_t last,
+                                        int* row)
 {
 #pragma unroll
-    for (int j = 0; j < N; ++j) row[j] = r0;
+    for (int j = 0; j < N; ++j) row[j] = 0;
     while (span > 1) {
-        const int64_t half = span / 2;
+        const int half = span / 2;
 #pragma unroll
         for (int j = 0; j < N; ++j)
-            if (off[row[j] + half] <= x[j]) row[j] += half;
+            if (off[r0 + row[j] + half] <= (x + j < last ? x + j : last)) row[j] += half;
         span -= half;
     }
 }

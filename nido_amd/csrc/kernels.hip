@@ -102,18 +102,16 @@ row_sums_kernel(const int64_t* __restrict__ off, const double* __restrict__ w, i
         const int64_t rf = s_row[0], span = s_row[1] - rf + 1;
         if (span > kSumSpan) {                   // uniform
             if (x0 < n) {
-                int64_t x[kSumRun], row[kSumRun];
-#pragma unroll
-                for (int j = 0; j < kSumRun; ++j) x[j] = t0 + (x0 + j < n ? x0 + j : n - 1);
-                rows_of<kSumRun>(off, rf, span, x, row);
+                int row[kSumRun];
+                rows_of<kSumRun>(off, rf, (int)span, t0 + x0, t0 + n - 1, row);
                 fx_t sum = 0;
 #pragma unroll
                 for (int j = 0; j < kSumRun; ++j) {
                     if (x0 + j >= n) break;
-                    src[t0 + x0 + j] = (int)row[j];
+                    src[t0 + x0 + j] = (int)(rf + row[j]);
                     sum += fx_from_double(wt[j]);
                     if (j + 1 < kSumRun && x0 + j + 1 < n && row[j + 1] == row[j]) continue;
-                    acc_add(k + row[j], sum);
+                    acc_add(k + rf + row[j], sum);
                     sum = 0;
                 }
             }

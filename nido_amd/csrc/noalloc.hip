@@ -79,14 +79,18 @@ na_check_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ com
 // then per community in an LDS table, so a community takes one global atomic
 // per tile.  A tile that spans more than kNaSpan rows, most of them empty, has
 // every thread search for its own arcs' rows instead.  Exact integer sums:
-// neither the split nor the order changes them.  Bound by the 16 B per arc and
-// the comm gathers; 2^20 vertices, 14.7 M arcs in planted blocks: 150 us,
-// against 511 us with a wavefront per row (a quarter of its lanes busy, a
-// 128-bit wavefront sum and two global atomics per row).  An id outside [0, nv)
+// neither the split nor the order changes them.  Bound by the comm gathers and
+// by the loads of a thread's run, whose lanes lie 64 bytes apart; four waves a
+// SIMD (128 registers, 48 bytes of scratch) hide them better than the three
+// that 162 registers allow, and better than five (96 registers, 112 bytes: 197
+// us).  A call on 2^20 vertices, 14.7 M arcs in planted blocks: 150 us, 180 with
+// three waves, 157 without the loads of 16 bytes; 544 us with a wavefront per
+// row (a quarter of its lanes busy, a 128-bit wavefront sum and two global
+// atomics per row).  An id outside [0, nv)
 // is never used as an index: it sets the flag; with the flag set by
 // na_check_kernel nothing is read.
 constexpr int kNaRun = 8, kNaTile = kBlock * kNaRun, kNaRows = 512, kNaSlots = 2 * kNaRows, kNaSpan = 8 * kNaRows;
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock, 4)
 na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col, const double* __restrict__ w,
                const int64_t* __restrict__ comm, int64_t nv, fx_t* __restrict__ a, Partials P)
 {
@@ -120,10 +124,17 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
         int64_t u[kNaRun];
         double wt[kNaRun];
         int cu[kNaRun];
+        if (n == kNaTile) {                          // uniform: loads of 16 bytes
 #pragma unroll
-        for (int j = 0; j < kNaRun; ++j) {
-            u[j] = x0 + j < n ? col[t0 + x0 + j] : 0;
-            wt[j] = x0 + j < n ? w[t0 + x0 + j] : 0.0;
+            for (int j = 0; j < kNaRun; ++j) u[j] = col[t0 + x0 + j];
+#pragma unroll
+            for (int j = 0; j < kNaRun; ++j) wt[j] = w[t0 + x0 + j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < kNaRun; ++j) {
+                u[j] = x0 + j < n ? col[t0 + x0 + j] : 0;
+                wt[j] = x0 + j < n ? w[t0 + x0 + j] : 0.0;
+            }
         }
 #pragma unroll
         for (int j = 0; j < kNaRun; ++j) {
@@ -135,16 +146,15 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
         const int64_t rf = s_row[0], span = s_row[1] - rf + 1;
         if (span > kNaSpan) {                        // uniform
             if (x0 < n) {
-                int64_t x[kNaRun], row[kNaRun];
-#pragma unroll
-                for (int j = 0; j < kNaRun; ++j) x[j] = t0 + (x0 + j < n ? x0 + j : n - 1);
-                rows_of<kNaRun>(off, rf, span, x, row);
+                int row[kNaRun];
+                rows_of<kNaRun>(off, rf, (int)span, t0 + x0, t0 + n - 1, row);
                 fx_t k = 0;
 #pragma unroll
                 for (int j = 0; j < kNaRun; ++j) {
                     if (x0 + j >= n) break;
-                    const int64_t c = comm[row[j]];
-                    const fx_t f = fx_from_double(wt[j]);
+                    const int64_t c = comm[rf + row[j]];
+                    asm volatile("" : "+v"(wt[j]));      // keeps the eight conversions apart
+                const fx_t f = fx_from_double(wt[j]);
                     k += f;
                     M += f;
                     if (cu[j] == c) I += f;
@@ -187,6 +197,7 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
                     do ++l;
                     while (s_off[l + 1] <= x);       // x < c1 = s_off[kNaRows]: ends
                 }
+                asm volatile("" : "+v"(wt[j]));      // keeps the eight conversions apart
                 const fx_t f = fx_from_double(wt[j]);
                 k += f;
                 M += f;
