@@ -1997,33 +1997,37 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
         for (int i = 0; i < G; ++i)
             for (int64_t e = gstart[(size_t)i]; e < gstart[(size_t)i + 1]; e += kPieceArcs)
                 pieces.push_back(ArcPiece{e, std::min(gstart[(size_t)i + 1], e + kPieceArcs), gv[i], gv[i + 1] - gv[i]});
-    if (on_device) {
+    // scratch is given back before a failure destroys the handle that owns it
+    auto take_arcs = [&]() -> int {
         ArenaScope tmp(g->ws);
         ArcPiece* d_pieces = nullptr;
-        if (G > 1 && ((rc = g->ws.get(&d_pieces, (int64_t)pieces.size())) ||
-                      (rc = send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size()))))
-            return fail(rc);
+        if (G > 1) {
+            NIDO_TRY(g->ws.get(&d_pieces, (int64_t)pieces.size()));
+            NIDO_TRY(send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size()));
+        }
         launch_take_arcs(d_pieces, G > 1 ? (int64_t)pieces.size() : (ne + kPieceArcs - 1) / kPieceArcs, ne, nv, g->d_col,
                          g->d_w, g->d_col32, &g->d_out->grid, s);
-        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "checking the uploaded arcs failed"));
+        if (hipGetLastError() != hipSuccess) return set_error(NIDO_ERR_HIP, "checking the uploaded arcs failed");
         WeightGrid grid{};
-        if ((rc = fetch(g, &grid, &g->d_out->grid, sizeof(grid)))) return fail(rc);
+        NIDO_TRY(fetch(g, &grid, &g->d_out->grid, sizeof(grid)));
         // (the bits of a NaN order above those of infinity)
         const bool exact = grid.flags != 0 || grid.wmax > nido_dbits(0x1p61) ||
                            nido_bitsd(grid.wmax) * (double)ne > 0x1p61;
-        if (exact && (rc = check_csr(nv, off, col, w, G, gv, &nonneg, nullptr))) return fail(rc);
-    }
-    g->nonneg = nonneg;
-    if (local16) {
-        // graph-local ids back to handle ids
+        return exact ? check_csr(nv, off, col, w, G, gv, &nonneg, nullptr) : NIDO_OK;
+    };
+    // graph-local ids back to handle ids
+    auto widen_local = [&]() -> int {
         ArenaScope tmp(g->ws);
         ArcPiece* d_pieces = nullptr;
-        if ((rc = g->ws.get(&d_pieces, (int64_t)pieces.size())) ||
-            (rc = send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size())))
-            return fail(rc);
+        NIDO_TRY(g->ws.get(&d_pieces, (int64_t)pieces.size()));
+        NIDO_TRY(send(g, d_pieces, pieces.data(), sizeof(ArcPiece) * pieces.size()));
         launch_widen_local(d_pieces, (int64_t)pieces.size(), reinterpret_cast<const uint16_t*>(g->d_col), g->d_col32, s);
-        if (hipGetLastError() != hipSuccess) return fail(set_error(NIDO_ERR_HIP, "widening the graph-local ids failed"));
-    }
+        if (hipGetLastError() != hipSuccess) return set_error(NIDO_ERR_HIP, "widening the graph-local ids failed");
+        return NIDO_OK;
+    };
+    if (on_device && (rc = take_arcs())) return fail(rc);
+    g->nonneg = nonneg;
+    if (local16 && (rc = widen_local())) return fail(rc);
     // ids crossed the host link as int32 or 16-bit local ids (all below
     // nv < 2^31 - 1, checked); the int64 copy overwrites the local ids
     if (fused) launch_widen_ids(g->d_col32, g->d_col, ne, s);
