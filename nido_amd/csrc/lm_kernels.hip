@@ -21,7 +21,7 @@
 //               workgroup (v, p) of launch 2 reads only its own buckets;
 //               with P <= 2 each workgroup reads the row and filters it.
 // Launch 1 = short-row bins + long-row key fill (20 KB LDS per workgroup,
-// 12 KB with fixed-point sums);
+// 12.5 KB with fixed-point sums);
 // launch 2 = long-row partitions (40 KB LDS with the default 2048-slot
 // table).  Row loops keep two to eight independent loads in flight per lane.
 #include <type_traits>
