@@ -341,8 +341,8 @@ void launch_widen_local(const ArcPiece* pieces, int64_t n, const uint16_t* local
 // out[i] = clus[i] - base[gid0[i]] for the n0 original vertices.
 void launch_local_ids(const int64_t* clus, int64_t n0, const int* gid0, const int64_t* base, int64_t* out,
                       hipStream_t s);
-// Coarse rows of at most kWaveRowArcs arcs are aggregated in LDS by one
-// wavefront, of at most kLdsRowArcs by one workgroup, longer ones in HBM
+// Coarse rows of at most kWaveRowArcs arcs and members are aggregated in LDS by
+// one wavefront, others of at most kLdsRowArcs arcs by one workgroup, longer ones in HBM
 // hash tables of whole kSlotWord-slot words.
 constexpr int64_t kWaveRowArcs = 64;
 constexpr int64_t kLdsRowArcs = 1024;

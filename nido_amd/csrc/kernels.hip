@@ -688,11 +688,21 @@ member_counts_kernel(const int64_t* __restrict__ C, const int64_t* __restrict__ 
     }
 }
 
+// Whether one wavefront aggregates a coarse row of a arcs and m members: each
+// lane takes one member, then one arc.  Members without arcs count: a vertex
+// that only has arcs towards it, as one-way inputs give, joins no community but
+// others join its own, so a row has up to a + 1 members.
+__device__ __forceinline__ bool wave_row(int64_t a, int64_t m)
+{
+    return a <= kWaveRowArcs && m <= kWaveRowArcs;
+}
+
 // Coarse row i with arcs[i] <= kLdsRowArcs is aggregated in LDS and needs
 // csz[i] = min(arcs, K) compact entries; a longer one gets an HBM hash table
 // of tsz[i] slots (a power of two >= twice its possible keys, whole words of
-// kSlotWord slots).  ml / mh: the members of LDS and of HBM rows.  The rows
-// longer than a wavefront aggregates are listed in mid[0, *nmid).
+// kSlotWord slots).  ml / mh: the members of LDS and of HBM rows.  The LDS
+// rows of more arcs or members than a wavefront has lanes are listed in mid[0,
+// *nmid).
 __global__ void __launch_bounds__(kBlock)
 coarse_sizes_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__ cnt, int64_t K,
                     int64_t* __restrict__ ml, int64_t* __restrict__ mh, int64_t* __restrict__ tsz,
@@ -714,7 +724,7 @@ coarse_sizes_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict_
             csz[i] = hbm ? 0 : need;
             ml[i] = hbm ? 0 : m;
             mh[i] = hbm ? m : 0;
-            listed = !hbm && a > kWaveRowArcs;
+            listed = !hbm && !wave_row(a, m);
         }
         const unsigned long long w = __ballot(listed);
         if (w) {   // uniform in the wavefront
@@ -771,11 +781,10 @@ member_scatter_kernel(const int* __restrict__ cid, const int64_t* __restrict__ o
     }
 }
 
-// Coarse rows of at most kWaveRowArcs arcs, one wavefront each: a row has at
-// most as many members as arcs (or one member without arcs), so each lane
-// holds one member, the lengths are scanned with shuffles, and each lane
-// then takes one arc and inserts its coarse target into the wavefront's
-// 128-slot LDS table.  No workgroup barrier: most coarse rows of a sparse
+// Coarse rows of at most kWaveRowArcs arcs and as many members (wave_row), one
+// wavefront each: each lane holds one member, the lengths are scanned with
+// shuffles, and each lane then takes one arc and inserts its coarse target into
+// the wavefront's 128-slot LDS table.  No workgroup barrier: most coarse rows of a sparse
 // graph are this short; bound by the round trips of a row (members, offsets,
 // arcs, ids), of which 8,192 wavefronts keep as many in flight.  R-MAT scale
 // 20's first coarse graph (316 K rows): 33 us, against 880 us with a
@@ -795,8 +804,8 @@ coarse_wave_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__
     unsigned long long *const lo = s_lo[wv], *const hi = s_hi[wv];
     const int64_t nw = (int64_t)gridDim.x * (kBlock / 64);
     for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + wv; i < K; i += nw) {   // uniform in the wavefront
-        const int64_t a = arcs[i];
-        if (a > kWaveRowArcs) continue;      // a longer LDS row or an HBM row
+        const int64_t a = arcs[i], m0 = ml[i], m = ml[i + 1] - m0;
+        if (!wave_row(a, m)) continue;       // a listed LDS row or an HBM row
         if (a == 0) {
             if (lane == 0) cnt[i] = 0;
             continue;
@@ -807,8 +816,7 @@ coarse_wave_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__
             lo[s] = 0;
             hi[s] = 0;
         }
-        const int64_t m0 = ml[i];
-        const int nm = (int)(ml[i + 1] - m0);   // <= a <= 64
+        const int nm = (int)m;               // <= 64
         int d = 0;
         int64_t e0 = 0;
         if (lane < nm) {
@@ -864,8 +872,8 @@ coarse_wave_kernel(const int64_t* __restrict__ arcs, const int64_t* __restrict__
     }
 }
 
-// The listed coarse rows (more than kWaveRowArcs, at most kLdsRowArcs arcs),
-// one workgroup each: the arcs of its members (their concatenation, 256 at a
+// The listed coarse rows (at most kLdsRowArcs arcs, more arcs or members than a
+// wavefront takes), one workgroup each: the arcs of its members (their concatenation, 256 at a
 // time, each thread locating its member by binary search over the scanned
 // lengths) go into an LDS table keyed by the coarse target, with exact Q64.64
 // sums; the arcs into the row itself are summed per wavefront first and
