@@ -128,10 +128,10 @@ hipError_t DeviceMem::get(void** p, size_t bytes)
             all.swap(c.blocks);
             c.bytes = 0;
         }
-        all.insert(all.end(), idle_.begin(), idle_.end());
+        for (const Block& b : all) runtime_free(b.p, pool, s_);
+        for (const Block& b : idle_) runtime_free(b.p, pool, s_);
         idle_.clear();
         idle_bytes_ = 0;
-        for (const Block& b : all) runtime_free(b.p, pool, s_);
         (void)hipStreamSynchronize(s_);
         if (pool) (void)hipMemPoolTrimTo(pool, 0);
         e = runtime_alloc(p, need, pool, s_);

@@ -10,9 +10,11 @@ namespace nido {
 
 // Device memory of one handle, in the order of its stream: a block it frees is
 // handed out again to the same handle at once (what follows on the stream comes
-// after what the block was used for).  release(), once the stream has been
-// waited for, gives the idle blocks to a cache of the device that all handles
+// after what the block was used for).  release(), whenever the handle has waited
+// for its stream, gives the idle blocks to a cache of the device that all handles
 // and threads take from; their uses are over, so no stream matters any more.
+// What live handles have freed is so within the bound of the cache, and within
+// reach of another one's failed allocation.
 // Below both is a memory pool of the runtime (hipMallocFromPoolAsync), whose
 // frees do not wait for the whole device.  It gives freed memory back to the
 // system as it sees fit, 0.3 to 7 ms at a time, and hands out a block again for

@@ -466,11 +466,19 @@ int need_side(nido_graph* g)
     return NIDO_OK;
 }
 
-// Waits for the handle's stream.
+// The handle's stream has been waited for: the pinned block is free, and what the
+// handle freed on the device is any handle's (what ran on the second stream, the
+// first one has waited for).
+void waited(nido_graph* g)
+{
+    g->pin_used = 0;
+    g->mem.release();
+}
+
 int wait_stream(nido_graph* g)
 {
     HIP_TRY(hipStreamSynchronize(g->stream));
-    g->pin_used = 0;
+    waited(g);
     return NIDO_OK;
 }
 
@@ -480,7 +488,7 @@ int send(nido_graph* g, void* dst, const void* src, size_t bytes)
     if (bytes == 0) return NIDO_OK;
     if (bytes > kPinBytes - kPinScalars) {
         HIP_TRY(staged_h2d(dst, src, bytes, g->stream));
-        g->pin_used = 0;                            // it waits for the stream
+        waited(g);
         return NIDO_OK;
     }
     if (g->pin_used + bytes > kPinBytes - kPinScalars) NIDO_TRY(wait_stream(g));
@@ -497,7 +505,7 @@ int fetch(nido_graph* g, void* dst, const void* src, size_t bytes)
     if (bytes == 0) return wait_stream(g);
     if (bytes > kPinBytes - kPinScalars) {
         HIP_TRY(staged_d2h(dst, src, bytes, g->stream));
-        g->pin_used = 0;
+        waited(g);
         return NIDO_OK;
     }
     char* p = g->pin.p;

@@ -9,10 +9,16 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <map>
+#include <mutex>
+
 namespace {
 void* g_hip = nullptr;
 int g_launch = 0;              // the g_launch-th launch from now fails (0: none)
 hipError_t g_last = hipSuccess;
+std::mutex g_mu;
+std::map<void*, size_t> g_blocks;   // what the pool handed out
+size_t g_used = 0, g_limit = 0;     // its sum; beyond g_limit (0: none) allocations fail
 
 template <typename F>
 F real(const char* name)
@@ -30,11 +36,33 @@ int shim_init(const char* path)
     return g_hip ? 0 : 1;
 }
 void shim_fail_launch(int k) { g_launch = k; }
+void shim_pool_limit(size_t bytes) { g_limit = bytes; }
+size_t shim_pool_used(void) { return g_used; }
 
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s)
 {
     if (g_launch > 0 && --g_launch == 0) return g_last = hipErrorLaunchFailure;
     return real<decltype(&hipLaunchKernel)>("hipLaunchKernel")(f, grid, block, args, lds, s);
+}
+
+hipError_t hipMallocFromPoolAsync(void** p, size_t n, hipMemPool_t pool, hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (g_limit && g_used + n > g_limit) return g_last = hipErrorOutOfMemory;
+    const hipError_t e = real<hipError_t (*)(void**, size_t, hipMemPool_t, hipStream_t)>("hipMallocFromPoolAsync")(p, n, pool, s);
+    if (e == hipSuccess) g_used += g_blocks[*p] = n;
+    return e;
+}
+
+hipError_t hipFreeAsync(void* p, hipStream_t s)
+{
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto it = g_blocks.find(p);
+    if (it != g_blocks.end()) {
+        g_used -= it->second;
+        g_blocks.erase(it);
+    }
+    return real<decltype(&hipFreeAsync)>("hipFreeAsync")(p, s);
 }
 
 hipError_t hipGetLastError(void)
