@@ -53,7 +53,7 @@ Cache& cache_of(int device)
         props.location.type = hipMemLocationTypeDevice;
         props.location.id = device;
         if (hipMemPoolCreate(&c.pool, &props) == hipSuccess) {
-            uint64_t keep = UINT64_MAX;
+            uint64_t keep = DeviceMem::kPoolKeep;
             (void)hipMemPoolSetAttribute(c.pool, hipMemPoolAttrReleaseThreshold, &keep);
         } else {
             (void)hipGetLastError();
@@ -199,7 +199,15 @@ size_t DeviceMem::cached()
     int device = -1;
     if (hipGetDevice(&device) != hipSuccess) return 0;
     std::lock_guard<std::mutex> lk(g_mu);
-    return g_cache.count(device) ? g_cache[device].bytes : 0;
+    const auto it = g_cache.find(device);
+    if (it == g_cache.end()) return 0;
+    size_t n = it->second.bytes;
+    uint64_t reserved = 0, used = 0;
+    if (it->second.pool &&
+        hipMemPoolGetAttribute(it->second.pool, hipMemPoolAttrReservedMemCurrent, &reserved) == hipSuccess &&
+        hipMemPoolGetAttribute(it->second.pool, hipMemPoolAttrUsedMemCurrent, &used) == hipSuccess && reserved > used)
+        n += (size_t)(reserved - used);
+    return n;
 }
 
 }  // namespace nido
