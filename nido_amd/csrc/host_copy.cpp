@@ -274,10 +274,13 @@ void pinned_put(PinnedBlock& b)
     {
         std::lock_guard<std::mutex> lk(g_pin_mu);
         if (g_pin_idle + b.bytes <= kPinKeep) {
-            g_pin->push_back(b);
-            g_pin_idle += b.bytes;
-            b = PinnedBlock{};
-            return;
+            try {
+                g_pin->push_back(b);
+                g_pin_idle += b.bytes;
+                b = PinnedBlock{};
+                return;
+            } catch (...) {   // no room for the list: it goes back
+            }
         }
     }
     (void)hipHostFree(b.p);

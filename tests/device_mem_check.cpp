@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <map>
+#include <new>
 #include <set>
 #include <string>
 #include <vector>
@@ -45,6 +46,24 @@ struct Dev {
     int host_allocs = 0, host_frees = 0;
     std::set<int> dead_streams;
 } D;
+static bool g_throw = false;              // operator new fails
+
+void* operator new(size_t n)
+{
+    void* p = g_throw ? nullptr : malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+
+// The runtime's own lists grow all the same.
+struct Grow {
+    bool was = g_throw;
+    Grow() { g_throw = false; }
+    ~Grow() { g_throw = was; }
+};
+
 // Frees that were waited for go back to the system above the pool's threshold.
 static void settle()
 {
@@ -60,6 +79,7 @@ static size_t held()
 }
 static hipError_t alloc(void** p, size_t n)
 {
+    Grow grow;
     const size_t reuse = std::min(D.pool_idle, n);
     if (held() - reuse + n > D.capacity) {
         ++D.oom;
@@ -75,6 +95,7 @@ static hipError_t alloc(void** p, size_t n)
 }
 static hipError_t release_to_pool(void* p, bool async)
 {
+    Grow grow;
     const auto it = D.live.find(p);
     if (it == D.live.end()) {
         ++D.bad_frees;
@@ -274,6 +295,38 @@ static void retry()
     CHECK(kept() == GiB / 2 && held() <= GiB / 2 + DeviceMem::kPoolKeep && D.bad_frees == 0);
 }
 
+// Lists that cannot grow lose no block and let no exception out.
+static void no_memory()
+{
+    DeviceMem a;
+    a.open(stream(1));
+    std::vector<void*> v;
+    for (int i = 0; i < 9; ++i) v.push_back(get(a, GiB / 8));
+    g_throw = true;
+    a.put(v[0]);
+    g_throw = false;
+    for (int i = 1; i < 9; ++i) a.put(v[(size_t)i]);
+    settle();
+    g_throw = true;
+    a.release();
+    g_throw = false;
+    settle();
+    CHECK(D.live.size() * (GiB / 8) == kept() && held() == kept());
+    g_throw = true;
+    void* p = nullptr;
+    const hipError_t e = a.get(&p, 5 * GiB);
+    g_throw = false;
+    CHECK(e == hipErrorOutOfMemory && p == nullptr);
+    settle();
+    CHECK(held() == kept() && D.bad_frees == 0);
+    nido::PinnedBlock b = nido::pinned_get(4 * MiB);
+    CHECK(b.p && b.bytes >= 4 * MiB);
+    g_throw = true;
+    nido::pinned_put(b);
+    g_throw = false;
+    CHECK(!b.p && D.host_frees + 1 >= D.host_allocs);
+}
+
 // Pinned blocks: reused from a quarter of their size up, 1 GiB idle at most.
 static void pinned()
 {
@@ -325,7 +378,7 @@ static void staged()
 int main(int argc, char** argv)
 {
     const std::map<std::string, void (*)()> all = {
-        {"bounded", bounded}, {"retry", retry}, {"pinned", pinned}, {"staged", staged}};
+        {"bounded", bounded}, {"retry", retry}, {"no_memory", no_memory}, {"pinned", pinned}, {"staged", staged}};
     const auto it = argc > 1 ? all.find(argv[1]) : all.end();
     if (it == all.end()) return 2;
     it->second();

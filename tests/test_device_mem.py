@@ -2,7 +2,7 @@
 buffers with their events) on the CPU: device_mem.cpp and host_copy.cpp built
 with g++ under sanitizers against a runtime whose device memory is addresses
 only, driven by device_mem_check.cpp: the stated bounds, the retry of a failed
-allocation."""
+allocation, lists that cannot grow."""
 import os
 import shutil
 import subprocess
@@ -24,7 +24,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["bounded", "retry", "pinned", "staged"])
+@pytest.mark.parametrize("scenario", ["bounded", "retry", "no_memory", "pinned", "staged"])
 def test_kept_memory(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=60, env=dict(os.environ, OMP_NUM_THREADS="2"))
     assert r.returncode == 0 and "ok" in r.stdout, (r.stdout[-3000:], r.stderr[-3000:])
