@@ -311,14 +311,14 @@ static void no_memory()
     a.release();
     g_throw = false;
     settle();
-    CHECK(D.live.size() * (GiB / 8) == kept() && held() == kept());
+    CHECK(D.live.size() * (GiB / 8) == kept() && held_here() == kept());
     g_throw = true;
     void* p = nullptr;
     const hipError_t e = a.get(&p, 5 * GiB);
     g_throw = false;
     CHECK(e == hipErrorOutOfMemory && p == nullptr);
     settle();
-    CHECK(held() == kept() && D.bad_frees == 0);
+    CHECK(held_here() == kept() && D.bad_frees == 0);
     nido::PinnedBlock b = nido::pinned_get(4 * MiB);
     CHECK(b.p && b.bytes >= 4 * MiB);
     g_throw = true;
