@@ -454,6 +454,13 @@ void batch_bounds(const std::vector<int64_t>& off, int64_t nv, int nb, std::vect
 constexpr size_t kPinBytes = size_t(4) << 20;   // of a handle's pinned block
 constexpr size_t kPinScalars = 4096;             // its first bytes: single results
 
+// Bytes of the pinned block for copies, after the single results: none in a block
+// that holds just those, and the copies are pageable ones then.
+size_t pin_room(const nido_graph* g)
+{
+    return std::min(g->pin.bytes, kPinBytes) - kPinScalars;
+}
+
 // The second stream and its events, made by the first iteration that uses them
 // (a replayed one, or one that streams its arcs): with the stream's end they
 // took 0.1 to 0.3 ms of every handle.
@@ -486,12 +493,12 @@ int wait_stream(nido_graph* g)
 int send(nido_graph* g, void* dst, const void* src, size_t bytes)
 {
     if (bytes == 0) return NIDO_OK;
-    if (bytes > kPinBytes - kPinScalars) {
+    if (bytes > pin_room(g)) {
         HIP_TRY(staged_h2d(dst, src, bytes, g->stream));
         waited(g);
         return NIDO_OK;
     }
-    if (g->pin_used + bytes > kPinBytes - kPinScalars) NIDO_TRY(wait_stream(g));
+    if (g->pin_used + bytes > pin_room(g)) NIDO_TRY(wait_stream(g));
     char* p = g->pin.p + kPinScalars + g->pin_used;
     std::memcpy(p, src, bytes);
     HIP_TRY(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, g->stream));
@@ -503,14 +510,14 @@ int send(nido_graph* g, void* dst, const void* src, size_t bytes)
 int fetch(nido_graph* g, void* dst, const void* src, size_t bytes)
 {
     if (bytes == 0) return wait_stream(g);
-    if (bytes > kPinBytes - kPinScalars) {
+    if (bytes > std::max(pin_room(g), kPinScalars)) {
         HIP_TRY(staged_d2h(dst, src, bytes, g->stream));
         waited(g);
         return NIDO_OK;
     }
     char* p = g->pin.p;
     if (bytes > kPinScalars) {
-        if (g->pin_used + bytes > kPinBytes - kPinScalars) NIDO_TRY(wait_stream(g));
+        if (g->pin_used + bytes > pin_room(g)) NIDO_TRY(wait_stream(g));
         p += kPinScalars + g->pin_used;
     }
     HIP_TRY(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, g->stream));
@@ -622,7 +629,7 @@ int device_bins(nido_graph* g, PhaseBins& pb, const unsigned char* keep)
     }
     // the long rows of every batch: into the pinned block and one wait, or
     // batch by batch when they do not fit it
-    if (sizeof(BinRow) * (size_t)nbig <= kPinBytes - kPinScalars && nbig > 0) {
+    if (sizeof(BinRow) * (size_t)nbig <= pin_room(g) && nbig > 0) {
         NIDO_TRY(wait_stream(g));
         BinRow* p = reinterpret_cast<BinRow*>(g->pin.p + kPinScalars);
         for (int b = 0; b < nb; ++b) {
@@ -1968,6 +1975,7 @@ int create_impl(int64_t nv, const int64_t* off, const int64_t* col, const double
         return fail(rc);
     if ((rc = raw_alloc(&g->d_scan_tmp, scan_temp_bytes(nv + 1)))) return fail(rc);
     g->pin = pinned_get(kPinBytes);
+    if (!g->pin.p) g->pin = pinned_get(kPinScalars);
     if (!g->pin.p) return fail(set_error(NIDO_ERR_NOMEM, "pinned allocation failed"));
     hipStream_t s = g->stream;
     launch_fill_fx(g->d_acc, 4, s);

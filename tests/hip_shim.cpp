@@ -19,6 +19,7 @@ hipError_t g_last = hipSuccess;
 std::mutex g_mu;
 std::map<void*, size_t> g_blocks;   // what the pool handed out
 size_t g_used = 0, g_limit = 0;     // its sum; beyond g_limit (0: none) allocations fail
+size_t g_pinned_max = SIZE_MAX;     // larger pinned allocations fail
 
 template <typename F>
 F real(const char* name)
@@ -38,6 +39,7 @@ int shim_init(const char* path)
 void shim_fail_launch(int k) { g_launch = k; }
 void shim_pool_limit(size_t bytes) { g_limit = bytes; }
 size_t shim_pool_used(void) { return g_used; }
+void shim_pinned_max(size_t bytes) { g_pinned_max = bytes; }
 
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s)
 {
@@ -63,6 +65,12 @@ hipError_t hipFreeAsync(void* p, hipStream_t s)
         g_blocks.erase(it);
     }
     return real<decltype(&hipFreeAsync)>("hipFreeAsync")(p, s);
+}
+
+hipError_t hipHostMalloc(void** p, size_t n, unsigned flags)
+{
+    if (n > g_pinned_max) return g_last = hipErrorOutOfMemory;
+    return real<hipError_t (*)(void**, size_t, unsigned)>("hipHostMalloc")(p, n, flags);
 }
 
 hipError_t hipGetLastError(void)
