@@ -19,10 +19,11 @@
 //
 // Calls on one GPU share its array: each call clears what it sums into
 // before using it (with a fill kernel, never hipMemsetAsync, so the launches
-// can be captured into a graph) and writes the flags of bad input that it
-// reads, so that no call depends on how the one before ended; two calls whose
-// launches overlap on one GPU -- on different streams without ordering between
-// them -- race on it.
+// can be captured into a graph; the flag of bad input, which that same
+// kernel may set, is cleared by the last kernel of the call, and by an extra one
+// where a launch of the call failed), and two calls whose launches overlap on
+// one GPU -- on different streams without ordering between them -- race on it.
+#include <atomic>
 #include <mutex>
 
 #include "../../include/nido_amd.h"
@@ -35,46 +36,31 @@ namespace {
 
 constexpr int64_t kNoAllocMaxVertices = NIDO_NOALLOC_MAX_VERTICES;
 // [0, max) community totals a_c, then three partial sums per workgroup
-// (internal weight, 2m, square terms), then a flag (a byte) per workgroup, set when
-// a row or community that it looked at lies outside the graph, and one per
-// wavefront for the arcs.  Workgroups leave partials instead of adding to one sum:
-// an atomic on one address takes its turn at the memory side, about 100 ns each
-// for the whole GPU, which was most of the time here.
+// (internal weight, 2m, square terms), then a flag set when an id lies outside
+// [0, nv).  Workgroups leave partials instead of adding to one sum: an atomic
+// on one address takes its turn at the memory side, about 100 ns each for the
+// whole GPU, which was most of the time here.
 constexpr int kNoAllocBlocks = 2048;
-constexpr int64_t kFlagFx = (1 + kBlock / 64) * kNoAllocBlocks / (int64_t)sizeof(fx_t);
-constexpr int64_t kScratchFx = kNoAllocMaxVertices + 3 * kNoAllocBlocks + kFlagFx;
+constexpr int64_t kScratchFx = kNoAllocMaxVertices + 3 * kNoAllocBlocks + 1;
 
 __device__ __align__(256) fx_t scratch[kScratchFx];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 fx_t* g_scratch_ptr[kMaxDevices] = {};
+// A failed call could not clear the flag either: the next one does so first.
+std::atomic<bool> g_flag_left[kMaxDevices];
 
 struct Partials {
     fx_t *inner, *mass, *term;   // kNoAllocBlocks each
-    unsigned char *bad_rows, *bad_arcs;   // kNoAllocBlocks and kBlock / 64 times as many
+    fx_t* bad;
 };
 
-// Whether one of n flags is set, found by each wavefront alone, 16 flags a lane
-// and load; what follows the n up to a multiple of 16 is zero.
-__device__ __forceinline__ bool na_flagged(const unsigned char* __restrict__ flags, int n)
-{
-    bool any = false;
-#pragma unroll
-    for (int r = 0; r < kNoAllocBlocks / 1024; ++r) {
-        const int i = r * 64 + (threadIdx.x & 63);
-        if (16 * i >= n) continue;
-        const uint4 x = reinterpret_cast<const uint4*>(flags)[i];
-        any |= (x.x | x.y | x.z | x.w) != 0;
-    }
-    return __ballot(any) != 0;
-}
-
-// Clears a[0, nv), and sets its workgroup's flag when a row is not part of the
-// arc arrays or a community is out of range.
+// Clears a[0, nv), and sets the flag when a row is not part of the arc
+// arrays or a community is out of range.
 __global__ void __launch_bounds__(kBlock)
 na_check_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ comm, int64_t nv, int64_t ne,
-                fx_t* __restrict__ a, unsigned char* __restrict__ bad_rows)
+                fx_t* __restrict__ a, fx_t* __restrict__ flag)
 {
     bool bad = false;
     for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < nv; i += (int64_t)gridDim.x * kBlock) {
@@ -82,12 +68,7 @@ na_check_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ com
         const int64_t e0 = off[i], e1 = off[i + 1], c = comm[i];
         bad |= e0 < 0 || e1 > ne || e0 > e1 || c < 0 || c >= nv;
     }
-    const int any = __syncthreads_or(bad);
-    if (threadIdx.x == 0) bad_rows[blockIdx.x] = any != 0;
-    if (blockIdx.x == 0 && threadIdx.x < 16 && (gridDim.x & 15)) {   // up to a multiple of 16
-        const unsigned i = (gridDim.x & ~15u) + threadIdx.x;
-        if (i >= gridDim.x) bad_rows[i] = 0;
-    }
+    if (bad) *flag = 1;   // every writer stores the same value
 }
 
 // k_v (self arcs included, graph_cuda.cu:302-346) into a[comm[v]], the weight
@@ -109,19 +90,24 @@ na_check_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ com
 // three waves, 157 without the loads of 16 bytes; 544 us with a wavefront per
 // row (a quarter of its lanes busy, a 128-bit wavefront sum and two global
 // atomics per row).  An id outside [0, nv)
-// is never used as an index: it sets the wavefront's flag; where one of
-// na_check_kernel's nc flags is set nothing is read.
+// is never used as an index: it sets the flag; with the flag set by
+// na_check_kernel nothing is read.
 constexpr int kNaRun = 8, kNaTile = kBlock * kNaRun, kNaRows = 512, kNaSlots = 2 * kNaRows, kNaSpan = 8 * kNaRows;
 __global__ void __launch_bounds__(kBlock, 4)
 na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col, const double* __restrict__ w,
-               const int64_t* __restrict__ comm, int64_t nv, fx_t* __restrict__ a, Partials P, int nc)
+               const int64_t* __restrict__ comm, int64_t nv, fx_t* __restrict__ a, Partials P)
 {
     __shared__ int key[kNaSlots];
     __shared__ unsigned long long lo[kNaSlots], hi[kNaSlots];
     __shared__ int s_off[kNaRows + 1], s_comm[kNaRows], s_slot[kNaRows];
     __shared__ fx_t red[kBlock / 64];
     __shared__ int64_t s_row[2];
-    if (na_flagged(P.bad_rows, nc)) return;          // uniform; Q is NaN then
+    // Set by na_check_kernel.  A workgroup that sees it set by another one of
+    // this launch (an arc id out of range) may leave as well: Q is NaN then.
+    __shared__ int s_bad;
+    if (threadIdx.x == 0) s_bad = ld_u64_agent(reinterpret_cast<const unsigned long long*>(P.bad)) != 0;
+    __syncthreads();
+    if (s_bad) return;
     const int64_t A0 = off[0], A1 = off[nv];
     fx_t I = 0, M = 0;
     bool bad = false;
@@ -171,7 +157,7 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
                     if (x0 + j >= n) break;
                     const int64_t c = comm[rf + row[j]];
                     asm volatile("" : "+v"(wt[j]));      // keeps the eight conversions apart
-                const fx_t f = fx_from_double(wt[j]);
+                    const fx_t f = fx_from_double(wt[j]);
                     k += f;
                     M += f;
                     if (cu[j] == c) I += f;
@@ -240,8 +226,7 @@ na_arcs_kernel(const int64_t* __restrict__ off, const int64_t* __restrict__ col,
         P.inner[blockIdx.x] = I;
         P.mass[blockIdx.x] = M;
     }
-    const unsigned long long m = __ballot(bad);
-    if ((threadIdx.x & 63) == 0) P.bad_arcs[blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)] = m != 0;
+    if (bad) *P.bad = 1;
 }
 
 // The sum of x[0, n) (valid in thread 0).
@@ -274,55 +259,42 @@ na_terms_kernel(const fx_t* __restrict__ a, int64_t nv, Partials P, int n)
     if (threadIdx.x == 0) P.term[blockIdx.x] = T;
 }
 
-// Q = RN(I) / 2m - RN(T); Q = 0 for a graph without weight, NaN when a flag
-// that the nc workgroups of na_check_kernel or the n of na_arcs_kernel left is set.
-// One workgroup: its time is the latency of its loads, so all are issued at once
-// (6.9 us at 2,048 partials; 10.0 sum by sum).
+// Q = RN(I) / 2m - RN(T); Q = 0 for a graph without weight, NaN when an id
+// was out of range.  Leaves the flag clear for the next call (flags written and
+// read within a call instead, by workgroup or wavefront, cost every call 1 to 3
+// us, 7% of a small one).
 __global__ void __launch_bounds__(kBlock)
-na_finish_kernel(Partials P, int nc, int n, int nt, double* __restrict__ q)
+na_finish_kernel(Partials P, int n, int nt, double* __restrict__ q)
 {
     __shared__ fx_t red[kBlock / 64];
-    constexpr int kPer = kNoAllocBlocks / kBlock;
-    fx_t xi[kPer], xm[kPer], xt[kPer];
-    unsigned arcs[kPer];             // a byte per wavefront of na_arcs_kernel: 4 n
-#pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-        const int i = r * kBlock + threadIdx.x;
-        xi[r] = i < n ? P.inner[i] : 0;
-        xm[r] = i < n ? P.mass[i] : 0;
-        xt[r] = i < nt ? P.term[i] : 0;
-        arcs[r] = i < n ? reinterpret_cast<const unsigned*>(P.bad_arcs)[i] : 0;
-    }
-    const bool rows = na_flagged(P.bad_rows, nc);
-    fx_t I = 0, m = 0, T = 0;
-    bool bad = false;
-#pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-        I += xi[r];
-        m += xm[r];
-        T += xt[r];
-        bad |= arcs[r] != 0;
-    }
-    I = block_sum_fx(I, red);
-    m = block_sum_fx(m, red);
-    T = block_sum_fx(T, red);
-    const int any = __syncthreads_or(bad) | (int)rows;
+    const fx_t I = na_sum(P.inner, n, red), m = na_sum(P.mass, n, red), T = na_sum(P.term, nt, red);
     if (threadIdx.x == 0) {
         const double twom_d = fx_to_double(m);
         double r = twom_d == 0.0 ? 0.0 : fx_to_double(I) / twom_d - fx_to_double(T);
-        if (any) r = __builtin_nan("");
+        if (*P.bad != 0) r = __builtin_nan("");
+        *P.bad = 0;
         *q = r;
     }
 }
 
+__global__ void na_clear_kernel(fx_t* bad) { *bad = 0; }
+
+// Whether the flag's clearing was launched.
+bool clear_flag(fx_t* bad, hipStream_t s)
+{
+    na_clear_kernel<<<1, 1, 0, s>>>(bad);
+    return hipGetLastError() == hipSuccess;
+}
+
 // The device address of `scratch` on the current device, resolved once per
 // device.
-int scratch_address(fx_t** out)
+int scratch_address(fx_t** out, int* device)
 {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return set_error(NIDO_ERR_HIP, "hipGetDevice: %s", hipGetErrorString(e));
     if (dev < 0 || dev >= kMaxDevices) return set_error(NIDO_ERR_INVALID, "device %d beyond %d", dev, kMaxDevices);
+    *device = dev;
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     if (!g_scratch_ptr[dev]) {
         void* p = nullptr;
@@ -349,27 +321,31 @@ extern "C" int nido_modularity_noalloc(int64_t nv, int64_t ne, const int64_t* of
     if (!q || (nv > 0 && (!offsets || !comm)) || (ne > 0 && (!cols || !weights)))
         return set_error(NIDO_ERR_INVALID, "null array");
     fx_t* base = nullptr;
-    int rc = scratch_address(&base);
+    int dev = 0;
+    int rc = scratch_address(&base, &dev);
     if (rc != NIDO_OK) return rc;
     fx_t* a = base;
     fx_t* part = base + kNoAllocMaxVertices;
-    unsigned char* flags = reinterpret_cast<unsigned char*>(part + 3 * kNoAllocBlocks);
-    const Partials P{part, part + kNoAllocBlocks, part + 2 * kNoAllocBlocks, flags, flags + kNoAllocBlocks};
+    const Partials P{part, part + kNoAllocBlocks, part + 2 * kNoAllocBlocks, part + 3 * kNoAllocBlocks};
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const unsigned nt = grid_for(nv, kBlock, 1024);
-    const unsigned nc = grid_for(nv, kBlock, kNoAllocBlocks);
-    unsigned n = 0;
-    na_check_kernel<<<nc, kBlock, 0, s>>>(offsets, comm, nv, ne, a, P.bad_rows);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess)   // what was not checked is not read
-        return set_error(NIDO_ERR_HIP, "nido_modularity_noalloc launch: %s", hipGetErrorString(e));
-    if (nv > 0 && ne > 0) {
-        n = grid_for(ne, kNaTile, kNoAllocBlocks);
-        na_arcs_kernel<<<n, kBlock, 0, s>>>(offsets, cols, weights, comm, nv, a, P, (int)nc);
+    if (g_flag_left[dev].load() && clear_flag(P.bad, s)) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusActive;   // captured: cleared at the replay only
+        if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) g_flag_left[dev] = false;
     }
-    na_terms_kernel<<<nt, kBlock, 0, s>>>(a, nv, P, (int)n);
-    na_finish_kernel<<<1, kBlock, 0, s>>>(P, (int)nc, (int)n, (int)nt, q);
-    e = hipGetLastError();
+    const unsigned nt = grid_for(nv, kBlock, 1024);
+    unsigned n = 0;
+    na_check_kernel<<<grid_for(nv, kBlock, 2048), kBlock, 0, s>>>(offsets, comm, nv, ne, a, P.bad);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) {   // what was not checked is not read
+        if (nv > 0 && ne > 0) {
+            n = grid_for(ne, kNaTile, kNoAllocBlocks);
+            na_arcs_kernel<<<n, kBlock, 0, s>>>(offsets, cols, weights, comm, nv, a, P);
+        }
+        na_terms_kernel<<<nt, kBlock, 0, s>>>(a, nv, P, (int)n);
+        na_finish_kernel<<<1, kBlock, 0, s>>>(P, (int)n, (int)nt, q);
+        e = hipGetLastError();
+        if (e != hipSuccess && !clear_flag(P.bad, s)) g_flag_left[dev] = true;
+    }
     if (e != hipSuccess) return set_error(NIDO_ERR_HIP, "nido_modularity_noalloc launch: %s", hipGetErrorString(e));
     return NIDO_OK;
 }

@@ -14,7 +14,7 @@
 
 namespace {
 void* g_hip = nullptr;
-int g_launch = 0;              // the g_launch-th launch from now fails (0: none)
+int g_launch = 0, g_launches = 0;   // g_launches launches from the g_launch-th on fail (0: none)
 hipError_t g_last = hipSuccess;
 std::mutex g_mu;
 std::map<void*, size_t> g_blocks;   // what the pool handed out
@@ -36,14 +36,21 @@ int shim_init(const char* path)
     g_hip = dlopen(path, RTLD_NOW | RTLD_NOLOAD);
     return g_hip ? 0 : 1;
 }
-void shim_fail_launch(int k) { g_launch = k; }
+void shim_fail_launch(int k, int n)
+{
+    g_launch = k;
+    g_launches = n;
+}
 void shim_pool_limit(size_t bytes) { g_limit = bytes; }
 size_t shim_pool_used(void) { return g_used; }
 void shim_pinned_max(size_t bytes) { g_pinned_max = bytes; }
 
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s)
 {
-    if (g_launch > 0 && --g_launch == 0) return g_last = hipErrorLaunchFailure;
+    if (g_launch > 0 && --g_launch == 0) {
+        if (--g_launches > 0) g_launch = 1;
+        return g_last = hipErrorLaunchFailure;
+    }
     return real<decltype(&hipLaunchKernel)>("hipLaunchKernel")(f, grid, block, args, lds, s);
 }
 

@@ -33,16 +33,19 @@ def q(cols, c):
 
 assert q(d_col, d_comm) == q1
 for cols, c in ((d_bad_col, d_comm), (d_col, d_bad_comm)):
-    for k in (1, 2, 3, 4):
-        shim.shim_fail_launch(k)
+    # the k-th launch of the call fails, and those after it up to n in all (more
+    # than the call has: the clean-up's too)
+    for k, n in ((1, 1), (2, 1), (3, 1), (4, 1), (2, 4), (4, 2)):
+        shim.shim_fail_launch(k, n)
         try:
             q(cols, c)
         except na.NidoError:
             pass
         else:
             raise SystemExit("the failed launch was not reported")
+        shim.shim_fail_launch(0, 0)
         assert hip.hipDeviceSynchronize() == 0
-        assert q(d_col, d_comm) == q1, (k, float(got[0]), q1)
+        assert q(d_col, d_comm) == q1, (k, n, float(got[0]), q1)
     assert np.isnan(q(cols, c))
 print("ok")
 """
