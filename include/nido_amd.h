@@ -74,7 +74,8 @@ typedef struct {
 typedef struct {
     int32_t thread_max_deg;   /* rows up to this length: one lane per vertex (0..2) */
     int32_t big_min_deg;      /* longer rows: hash-partitioned workgroups (0..512) */
-    int32_t big_part_arcs;    /* distinct communities expected per partition, at most (>= 1) */
+    int32_t big_part_arcs;    /* arcs per partition on average, at most (>= 1; fewer are taken where as many
+                                 communities could exceed big_key_limit) */
     int32_t big_key_limit;    /* LDS keys per partition before the exact HBM fallback (1..big_slots/2) */
     int32_t use_graph;        /* replay each phase's iterations from a hipGraph: 0 never, 1 for graphs of
                                  2^28+ arcs (default), 2 always; never while per-kernel events are on */
@@ -90,7 +91,7 @@ typedef struct {
                                  or 2, a windowed phase whose batches each fit the window takes the
                                  update from its first iteration on */
     int32_t fixed_short;      /* 1 (default): rows up to big_min_deg arcs sum in 64-bit fixed point when every
-                                 weight is a multiple of one power of two 2^-F and those rows' sums stay below
+                                 weight is a multiple of one power of two 2^-F and sums of 512 weights stay below
                                  2^63 in units of 2^-F (the same exact sums); 0: always Q64.64 (0/1) */
 } nido_tuning;
 

@@ -779,8 +779,8 @@ int build_lists(nido_graph* g, const unsigned char* keep)
     return NIDO_OK;
 }
 
-// Per-phase set-up: maximum order, batches, degree bins, the row slices of
-// the degree/modularity sweeps, k_v and 2m (GraphGPU ctor steps
+// Per-phase set-up: maximum order, batches, k_v and 2m, work lists, the
+// fixed-point weights and the items of per-graph modularity (GraphGPU ctor steps
 // graph_gpu.cpp:94-139 and aggregation steps graph_gpu.cpp:1487-1516).
 int setup_phase(nido_graph* g)
 {

@@ -29,7 +29,7 @@ constexpr int kThreadMaxDeg = 2;
 // 2^63, and any short row (the key fill sums that many in a wavefront).
 constexpr int64_t kFixedArcs = 512;
 constexpr int64_t kBinMaxDeg[NUM_BINS] = {kThreadMaxDeg, 16, 32, 64, 128, 512, INT64_MAX};
-constexpr int64_t kBigPartArcs = 1024;    // expected distinct keys per partition, at most
+constexpr int64_t kBigPartArcs = 1024;    // arcs of a partition on average, at most (876 with the limit below: partitions_of)
 constexpr int kBigSlots = 2048;           // LDS table of a partition workgroup (40/48 KB: 4 or 3 per CU)
 constexpr int kBigLimit = kBigSlots / 2;  // distinct keys before the exact HBM fallback
 
@@ -44,12 +44,15 @@ struct KeyChunk {
 constexpr int64_t kKeyChunkArcs = 2048;
 // Rows split into at most this many partitions skip the key fill: each
 // partition workgroup reads the whole row and keeps the arcs of its
-// partition (their items carry c0 = -1).  Measured on R-MAT s22: 2 is
-// +0.5% over 1, 4 is -4%.
+// partition (their items carry c0 = -1).  With partitions of up to 876 arcs,
+// iterations of a first phase in ms for 1 / 2 / 3 / 4: R-MAT scale 22 42.9 / 42.9
+// / 42.7 / 44.9, scale 17 2.68 / 2.71 / 2.71 / 3.15, Chung-Lu with 2.1 M vertices
+// 30.5 / 30.5 / 30.8 / 31.2.
 constexpr int kDirectParts = 2;
 constexpr int kMaxParts = 1024;           // partitions per row, at most
 
-// A slice of one row for the degree / modularity sweeps over long rows.
+// A run of one row's arcs, of the rows of moved vertices in the incremental
+// modularity.
 struct RowItem {
     int64_t v;
     int64_t e0, e1;
